@@ -115,6 +115,10 @@ struct sgeo_mesh {
   float* d_K32 = nullptr;   // derived operators (see refresh_operator)
   double* d_KP64 = nullptr;
   float* d_KP32 = nullptr;
+  // K was built from the corners and materials, so products can be formed
+  // from them; false for uploaded matrices
+  bool built = false;
+  double2* d_lame = nullptr;  // (lambda, mu) per material of the built K
   int k_ver = 0, k32_ver = -1, kp64_ver = -1, kp32_ver = -1;
   double* d_dinv = nullptr;
   // node map of the nodal result fields (sgeo_mesh_set_nodes)
@@ -377,7 +381,8 @@ extern "C" int sgeo_mesh_destroy(sgeo_mesh* m) {
   void* ptrs[] = {m->d_gdof, m->d_rowptr, m->d_slots, m->d_corners, m->d_mat,
                   m->d_K64,  m->d_K32,    m->d_KP64,  m->d_KP32,
                   m->d_dinv,  m->d_Y,       m->d_r,
-                  m->d_z,    m->d_p,      m->d_kp,    m->d_nrowptr, m->d_nslots};
+                  m->d_z,    m->d_p,      m->d_kp,    m->d_nrowptr, m->d_nslots,
+                  m->d_lame};
   for (void* p : ptrs)
     if (p) hipFree(p);
   delete m;
@@ -498,9 +503,15 @@ static int set_k_storage(sgeo_mesh* m, int kprec) {
   return 0;
 }
 
+// The packed FP64 operator of a built mesh is applied from the geometry
+// (k_mf64): its packed matrices are made only where a kernel reads them.
+static bool matrix_free(const sgeo_mesh* m) {
+  return m->built && m->kfmt == SGEO_KFMT_PACKED && m->kprec == SGEO_K_F64;
+}
+
 // Derived storage of the selected operator, rebuilt from the canonical FP64
 // full K whenever K changed (k_ver).
-static int refresh_operator(sgeo_mesh* m) {
+static int refresh_operator(sgeo_mesh* m, bool stored = false) {
   hipStream_t s = m->ctx->stream;
   const size_t nk = (size_t)m->nelmt * 6561;
   const size_t np = (size_t)m->nelmt * SGEO_KPACK;
@@ -511,6 +522,7 @@ static int refresh_operator(sgeo_mesh* m) {
       m->k32_ver = m->k_ver;
     }
   } else if (m->kfmt == SGEO_KFMT_PACKED && m->kprec == SGEO_K_F64) {
+    if (!stored && matrix_free(m)) return 0;
     if (!m->d_KP64) TRY(dalloc(&m->d_KP64, np, &m->bytes));
     if (m->kp64_ver != m->k_ver) {
       launch_pack_upper_f64(s, m->nelmt, m->d_K64, m->d_KP64);
@@ -566,6 +578,9 @@ extern "C" int sgeo_mesh_build_stiffness(sgeo_mesh* m, const double* gam,
   if (gam) HIPCHK(hipMemcpyAsync(d_gam, gam, m->nmat * 8, hipMemcpyHostToDevice, s));
   launch_stiffness(s, m->nelmt, m->d_corners, m->d_mat, d_ym, d_nu, m->d_K64,
                    d_kdiag, d_eld);
+  if (!m->d_lame) TRY(dalloc(&m->d_lame, m->nmat, &m->bytes));
+  launch_lame(s, m->nmat, d_ym, d_nu, m->d_lame);
+  m->built = true;
   // dprecon(egdof(k)) += km(k,k) in element order, then 1/d
   launch_assemble(s, n1, m->d_rowptr, m->d_slots, d_kdiag, m->d_dinv, c->d_sc, 0);
   launch_invert_diag(s, n1, m->d_dinv);
@@ -593,6 +608,7 @@ extern "C" int sgeo_mesh_upload_stiffness(sgeo_mesh* m, const double* k,
   hipStream_t s = c->stream;
   TRY(set_k_storage(m, kprec));
   const size_t nk = (size_t)m->nelmt * 6561;
+  m->built = false;
   HIPCHK(hipMemcpyAsync(m->d_K64, k, nk * 8, hipMemcpyHostToDevice, s));
   HIPCHK(hipMemcpyAsync(m->d_dinv, dprecon, ((size_t)m->neq + 1) * 8,
                         hipMemcpyHostToDevice, s));
@@ -614,7 +630,10 @@ extern "C" int sgeo_mesh_download_stiffness(sgeo_mesh* m, double* k) {
 static void ebe_elem(sgeo_mesh* m, const double* p, double* Y, int skip_mode) {
   hipStream_t s = m->ctx->stream;
   const PcgScalars* sc = m->ctx->d_sc;
-  if (m->kfmt == SGEO_KFMT_PACKED) {
+  if (matrix_free(m)) {
+    launch_mf64(s, m->nelmt, m->d_corners, m->d_gdof, m->d_mat, m->d_lame, p, Y, sc,
+                skip_mode);
+  } else if (m->kfmt == SGEO_KFMT_PACKED) {
     if (m->kprec == SGEO_K_F32)
       launch_ebe_packed_f32(s, m->nelmt, m->d_KP32, m->d_gdof, p, Y, sc, skip_mode);
     else
@@ -1488,7 +1507,7 @@ static int ensure_packed(sgeo_mesh* m, int kprec) {
   const int kp = m->kprec, kf = m->kfmt;
   m->kprec = kprec;
   m->kfmt = SGEO_KFMT_PACKED;
-  const int rc = refresh_operator(m);
+  const int rc = refresh_operator(m, true);
   m->kprec = kp;
   m->kfmt = kf;
   return rc;

@@ -61,6 +61,11 @@ void launch_ebe_packed_f64(hipStream_t s, int32_t nelmt, int n_cu, const double*
 void launch_ebe_packed_f32(hipStream_t s, int32_t nelmt, const float* KP,
                            const int32_t* gdof, const double* p, double* Y,
                            const PcgScalars* sc, int skip_mode);
+// product of a built mesh without stored matrices; lame: (lambda, mu) per material
+void launch_lame(hipStream_t s, int nmat, const double* ym, const double* nu, double2* lame);
+void launch_mf64(hipStream_t s, int32_t nelmt, const double* corners, const int32_t* gdof,
+                 const int32_t* mat_id, const double2* lame, const double* p, double* Y,
+                 const PcgScalars* sc, int skip_mode);
 void launch_pack_upper_f64(hipStream_t s, int32_t nelmt, const double* K,
                            double* KP);
 void launch_pack_upper_f32(hipStream_t s, int32_t nelmt, const double* K,
