@@ -50,8 +50,9 @@ struct sgeo_ctx {
   int device = 0;
   int n_cu = 0;  // compute units of the device
   hipStream_t stream = nullptr;
-  PcgScalars* d_sc = nullptr;
-  PcgScalars* h_sc = nullptr;  // pinned
+  PcgScalars* d_sc = nullptr;  // two: the fused iteration double-buffers them
+  PcgScalars* h_sc = nullptr;  // pinned, two
+  hipEvent_t ev_sc[2] = {nullptr, nullptr};  // their copies
   PlasticScalars* d_ps = nullptr;
   PlasticScalars* h_ps = nullptr;  // pinned
   double* d_part = nullptr;
@@ -231,15 +232,16 @@ extern "C" int sgeo_init(int device, sgeo_ctx** out) {
   HIPCHK(hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device));
   if (c->n_cu < 1) c->n_cu = 1;
   HIPCHK(hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking));
-  TRY(dalloc(&c->d_sc, 1));
+  TRY(dalloc(&c->d_sc, 2));
   TRY(dalloc(&c->d_ps, 1));
-  HIPCHK(hipHostMalloc((void**)&c->h_sc, sizeof(PcgScalars)));
+  HIPCHK(hipHostMalloc((void**)&c->h_sc, 2 * sizeof(PcgScalars)));
+  for (hipEvent_t& e : c->ev_sc) HIPCHK(hipEventCreateWithFlags(&e, hipEventDisableTiming));
   HIPCHK(hipHostMalloc((void**)&c->h_ps, sizeof(PlasticScalars)));
   HIPCHK(hipHostMalloc((void**)&c->h_flag, sizeof(int32_t)));
   // the device-current copy of the scratch array (every GPU has its own)
   HIPCHK(hipGetSymbolAddress((void**)&c->d_scratch, HIP_SYMBOL(scratch)));
   if (!c->d_scratch) return fail(SGEO_EHIP, "sgeo_init: no address for the scratch array");
-  HIPCHK(hipMemsetAsync(c->d_sc, 0, sizeof(PcgScalars), c->stream));
+  HIPCHK(hipMemsetAsync(c->d_sc, 0, 2 * sizeof(PcgScalars), c->stream));
   HIPCHK(hipMemsetAsync(c->d_ps, 0, sizeof(PlasticScalars), c->stream));
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -260,6 +262,8 @@ extern "C" int sgeo_finalize(sgeo_ctx* c) {
   if (c->h_ps) hipHostFree(c->h_ps);
   if (c->h_flag) hipHostFree(c->h_flag);
   for (hipEvent_t e : c->ev) hipEventDestroy(e);
+  for (hipEvent_t e : c->ev_sc)
+    if (e) hipEventDestroy(e);
   if (c->stream) hipStreamDestroy(c->stream);
   delete c;
   return 0;
@@ -368,7 +372,10 @@ extern "C" int sgeo_mesh_create(sgeo_ctx* c, int32_t nelmt, int32_t neq,
     HIPCHK(hipMemcpyAsync(m->d_mat, mat_id, (size_t)nelmt * 4,
                           hipMemcpyHostToDevice, s));
   }
-  TRY(ensure_part(c, 4 * (size_t)vec_reduce_blocks(n1) + 64));
+  // partials of the reductions, for any operator (at most one share of p.Kp
+  // per element)
+  TRY(ensure_part(c, std::max(4 * (size_t)vec_reduce_blocks(n1) + 64,
+                              std::max(pcg_tree_part(nelmt, n1), pcg_tree_part(0, n1)))));
   HIPCHK(hipStreamSynchronize(s));  // host vectors die at return
   *out = guard.release();
   return 0;
@@ -539,6 +546,17 @@ static int refresh_operator(sgeo_mesh* m, bool stored = false) {
   return 0;
 }
 
+// the packed matrices of a precision, whatever operator is selected
+static int ensure_packed(sgeo_mesh* m, int kprec) {
+  const int kp = m->kprec, kf = m->kfmt;
+  m->kprec = kprec;
+  m->kfmt = SGEO_KFMT_PACKED;
+  const int rc = refresh_operator(m, true);
+  m->kprec = kp;
+  m->kfmt = kf;
+  return rc;
+}
+
 extern "C" int sgeo_mesh_set_operator(sgeo_mesh* m, int kprec, int kfmt) {
   if (!m || m->kprec < 0) return fail(SGEO_EARG, "mesh has no stiffness");
   if ((kprec != SGEO_K_F64 && kprec != SGEO_K_F32) ||
@@ -627,23 +645,34 @@ extern "C" int sgeo_mesh_download_stiffness(sgeo_mesh* m, double* k) {
   return 0;
 }
 
-static void ebe_elem(sgeo_mesh* m, const double* p, double* Y, int skip_mode) {
+// Y = the element products of p; part (may be NULL): shares of p.Kp,
+// ebe_blocks(m) of them; sc: the scalars skip_mode reads; stored: multiply
+// the stored matrices
+static void ebe_elem(sgeo_mesh* m, const double* p, double* Y, int skip_mode,
+                     bool stored = false, double* part = nullptr,
+                     const PcgScalars* sc = nullptr) {
   hipStream_t s = m->ctx->stream;
-  const PcgScalars* sc = m->ctx->d_sc;
-  if (matrix_free(m)) {
-    launch_mf64(s, m->nelmt, m->d_corners, m->d_gdof, m->d_mat, m->d_lame, p, Y, sc,
+  if (!sc) sc = m->ctx->d_sc;
+  if (!stored && matrix_free(m)) {
+    launch_mf64(s, m->nelmt, m->d_corners, m->d_gdof, m->d_mat, m->d_lame, p, Y, part, sc,
                 skip_mode);
   } else if (m->kfmt == SGEO_KFMT_PACKED) {
     if (m->kprec == SGEO_K_F32)
-      launch_ebe_packed_f32(s, m->nelmt, m->d_KP32, m->d_gdof, p, Y, sc, skip_mode);
+      launch_ebe_packed_f32(s, m->nelmt, m->d_KP32, m->d_gdof, p, Y, part, sc, skip_mode);
     else
-      launch_ebe_packed_f64(s, m->nelmt, m->ctx->n_cu, m->d_KP64, m->d_gdof, p, Y, sc,
+      launch_ebe_packed_f64(s, m->nelmt, m->ctx->n_cu, m->d_KP64, m->d_gdof, p, Y, part, sc,
                             skip_mode);
   } else if (m->kprec == SGEO_K_F32) {
-    launch_ebe_elem_f32k(s, m->nelmt, m->d_K32, m->d_gdof, p, Y, sc, skip_mode);
+    launch_ebe_elem_f32k(s, m->nelmt, m->d_K32, m->d_gdof, p, Y, part, sc, skip_mode);
   } else {
-    launch_ebe_elem_f64(s, m->nelmt, m->d_K64, m->d_gdof, p, Y, sc, skip_mode);
+    launch_ebe_elem_f64(s, m->nelmt, m->d_K64, m->d_gdof, p, Y, part, sc, skip_mode);
   }
+}
+
+static int ebe_blocks(const sgeo_mesh* m) {
+  if (matrix_free(m)) return mf64_blocks(m->nelmt);
+  if (m->kfmt != SGEO_KFMT_PACKED) return ebe_elem_blocks(m->nelmt);
+  return m->kprec == SGEO_K_F32 ? m->nelmt : ebe_packed_blocks(m->nelmt, m->ctx->n_cu);
 }
 
 // --------------------------------------------------------------------------
@@ -817,9 +846,78 @@ extern "C" int sgeo_mesh_matvec(sgeo_mesh* m, const double* p, double* kp) {
 // Iterations are enqueued in chunks; each kernel of an iteration returns at
 // once when the device-side stop flag is set, so over-enqueued iterations
 // cost only their launches.  The host reads the flag once per chunk.
+//
+// A trial's solves (`trial`) multiply the stored matrices and form p.Kp from
+// the assembled vector; linear solves take the geometry where they can, and
+// the product's shares of p.Kp (sgeo_pcg.hip says why).  The share of every
+// block of a product needs room among the partials: systems with fewer
+// equations than that (nearly everything constrained, or a handful of
+// elements) assemble too.  The rule depends on the sizes and the operator
+// only, so the allocation-free entry point takes the same way.
+static bool pcg_shares(const sgeo_mesh* m, bool trial) {
+  const int64_t n1 = (int64_t)m->neq + 1;
+  return !trial && (int64_t)pcg_tree_part(ebe_blocks(m), n1) <= n1;
+}
+
+// Tree-ordered reductions.  The next chunk is enqueued before the last one's
+// flag is read, so the GPU does not wait for the host; a solve over-runs by
+// at most two chunks of launches that return at once.
+static int pcg_tree(sgeo_mesh* m, double* d_u, const double* d_f, double tol,
+                    int32_t maxiter, int32_t* cg_iter, int32_t* errcode, double* part,
+                    bool trial) {
+  sgeo_ctx* c = m->ctx;
+  hipStream_t s = c->stream;
+  const int64_t n1 = (int64_t)m->neq + 1;
+  const bool shares = pcg_shares(m, trial);
+  const PcgPart q = pcg_part(part, shares ? ebe_blocks(m) : 0, n1);
+  launch_pcg_begin(s, n1, d_u, part, c->d_sc, tol, maxiter);
+  ebe_elem(m, d_u, m->d_Y, 2, trial);
+  launch_assemble(s, n1, m->d_rowptr, m->d_slots, m->d_Y, m->d_kp, c->d_sc, 2);
+  launch_pcg_start(s, n1, d_f, m->d_kp, m->d_dinv, m->d_r, m->d_p, q, c->d_sc);
+  const int chunk = 16;
+  int32_t enq = 0, iter_prev = 0;
+  c->ev_used = 0;
+  for (int k = 0;; k++) {
+    const int n = std::min<int32_t>(chunk, maxiter - enq);
+    for (int it = 0; it < n; it++, enq++) {
+      TRY(prof_mark(c));
+      ebe_elem(m, m->d_p, m->d_Y, 1, trial, shares ? q.dot : nullptr, c->d_sc + (enq & 1));
+      TRY(prof_mark(c));
+      launch_pcg_iteration(s, n1, enq, m->d_rowptr, m->d_slots, m->d_Y,
+                           shares ? nullptr : m->d_kp, m->d_dinv, d_u, m->d_r, m->d_p, q,
+                           c->d_sc);
+    }
+    HIPCHK(hipGetLastError());
+    if (n > 0) {
+      HIPCHK(hipMemcpyAsync(c->h_sc + (k & 1), c->d_sc + (enq & 1), sizeof(PcgScalars),
+                            hipMemcpyDeviceToHost, s));
+      HIPCHK(hipEventRecord(c->ev_sc[k & 1], s));
+    }
+    // look at the chunk before (at this one when its launches are timed)
+    if (k == 0 && !c->prof) continue;
+    const int w = (c->prof ? k : k - 1) & 1;
+    HIPCHK(hipEventSynchronize(c->ev_sc[w]));
+    const PcgScalars sc = c->h_sc[w];
+    if (c->prof) {
+      // only the launches of iterations that ran (later ones return at once)
+      const int ran = sc.iter - iter_prev;
+      c->ev_used = std::min(c->ev_used, 2 * std::max(ran, 0));
+      TRY(prof_flush(c));
+      iter_prev = sc.iter;
+    }
+    if (sc.done) {
+      *cg_iter = sc.conv_iter;
+      *errcode = sc.done == 1 ? 0 : -1;
+      return 0;
+    }
+    if (n == 0)
+      return fail(SGEO_ESTATE, "PCG: %d iterations enqueued without a verdict", enq);
+  }
+}
+
 static int pcg_device(sgeo_mesh* m, double* d_u, const double* d_f, double tol,
                       int32_t maxiter, int32_t* cg_iter, int32_t* errcode,
-                      double* part = nullptr) {
+                      bool trial = false, double* part = nullptr) {
   sgeo_ctx* c = m->ctx;
   if (!part) part = c->d_part;
   hipStream_t s = c->stream;
@@ -830,12 +928,13 @@ static int pcg_device(sgeo_mesh* m, double* d_u, const double* d_f, double tol,
     *errcode = -1;
     return 0;
   }
+  if (c->reduction != SGEO_REDUCE_SEQUENTIAL)
+    return pcg_tree(m, d_u, d_f, tol, maxiter, cg_iter, errcode, part, trial);
+  // reference-order dot products
   launch_pcg_begin(s, n1, d_u, part, c->d_sc, tol, maxiter);
-  ebe_elem(m, d_u, m->d_Y, 2);
+  ebe_elem(m, d_u, m->d_Y, 2, trial);
   launch_assemble(s, n1, m->d_rowptr, m->d_slots, m->d_Y, m->d_kp, c->d_sc, 2);
-  const int seq = c->reduction == SGEO_REDUCE_SEQUENTIAL;
-  launch_pcg_init(s, n1, d_f, m->d_kp, m->d_dinv, m->d_r, m->d_z, m->d_p,
-                  part, c->d_sc, seq);
+  launch_pcg_init(s, n1, d_f, m->d_kp, m->d_dinv, m->d_r, m->d_z, m->d_p, c->d_sc);
   int32_t enq = 0, iter_prev = 0;
   int chunk = 8;
   c->ev_used = 0;
@@ -843,12 +942,12 @@ static int pcg_device(sgeo_mesh* m, double* d_u, const double* d_f, double tol,
     const int n = std::min<int32_t>(chunk, maxiter - enq);
     for (int it = 0; it < n; it++) {
       TRY(prof_mark(c));
-      ebe_elem(m, m->d_p, m->d_Y, 1);
+      ebe_elem(m, m->d_p, m->d_Y, 1, trial);
       TRY(prof_mark(c));
-      launch_pcg_assemble_dot(s, n1, m->d_rowptr, m->d_slots, m->d_Y, m->d_p,
-                              m->d_kp, part, c->d_sc, seq);
+      launch_pcg_assemble(s, n1, m->d_rowptr, m->d_slots, m->d_Y, m->d_p,
+                          m->d_kp, part, c->d_sc);
       launch_pcg_update(s, n1, m->d_p, m->d_kp, m->d_dinv, d_u, m->d_r,
-                        m->d_z, part, c->d_sc, seq);
+                        m->d_z, part, c->d_sc);
       launch_pcg_pupdate(s, n1, m->d_z, m->d_p, c->d_sc);
     }
     enq += n;
@@ -1048,7 +1147,10 @@ extern "C" int sgeo_pcg_solver_noalloc(sgeo_ctx* c, int32_t neq, int32_t nelmt,
   HIPCHK(hipStreamSynchronize(s));
   if (*c->h_flag)
     return fail(SGEO_EARG, "sgeo_pcg_solver_noalloc: gdof_elmt entry outside 0..%d", neq);
-  TRY(pcg_device(&m, d_u, d_f, cg_tol, cg_maxiter, cg_iter, errcode, part));
+  // the tree-reduced iteration stores no z: the product's shares and the
+  // other partials live there where it forms them
+  if (c->reduction != SGEO_REDUCE_SEQUENTIAL && pcg_shares(&m, false)) part = m.d_z;
+  TRY(pcg_device(&m, d_u, d_f, cg_tol, cg_maxiter, cg_iter, errcode, false, part));
   if (*errcode != 0) set_errtag(errtag, "ERROR: PCG solver doesn't converge!");
   else set_errtag(errtag, "");
   return 0;
@@ -1270,8 +1372,9 @@ extern "C" int sgeo_slope_plastic_iter(sgeo_slope* t, double cg_tol,
   hipStream_t s = c->stream;
   const int64_t n1 = (int64_t)m->neq + 1;
   int32_t it = 0, ec = -1;
+  if (matrix_free(m)) TRY(ensure_packed(m, SGEO_K_F64));  // a trial multiplies the matrices
   launch_load(s, n1, t->d_ext, t->d_body, t->d_load);
-  TRY(pcg_device(m, t->d_x, t->d_load, cg_tol, cg_maxiter, &it, &ec));
+  TRY(pcg_device(m, t->d_x, t->d_load, cg_tol, cg_maxiter, &it, &ec, true));
   if (cg_iter) *cg_iter = it;
   if (errcode) *errcode = ec;
   if (ec != 0) return 0;  // the caller stops (src/slope.F90:295)
@@ -1502,16 +1605,6 @@ struct sgeo_batch {
   std::vector<int32_t> nacc_valid;   // column's accumulators describe its state
   std::vector<int32_t> nacc_init;    // column's accumulators hold a started sum
 };
-
-static int ensure_packed(sgeo_mesh* m, int kprec) {
-  const int kp = m->kprec, kf = m->kfmt;
-  m->kprec = kprec;
-  m->kfmt = SGEO_KFMT_PACKED;
-  const int rc = refresh_operator(m, true);
-  m->kprec = kp;
-  m->kfmt = kf;
-  return rc;
-}
 
 // Packed FP32/FP64 operators and the FP32 inverse diagonal follow the mesh's
 // current stiffness (rebuilt when K changed since the last call).

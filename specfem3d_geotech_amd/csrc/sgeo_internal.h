@@ -50,22 +50,26 @@ void launch_stiffness(hipStream_t s, int32_t nelmt, const double* corners,
                       double* K, double* kdiag, double* eld);
 void launch_round_f32(hipStream_t s, int64_t n, const double* a, float* b);
 void launch_ebe_elem_f64(hipStream_t s, int32_t nelmt, const double* K,
-                         const int32_t* gdof, const double* p, double* Y,
+                         const int32_t* gdof, const double* p, double* Y, double* part,
                          const PcgScalars* sc, int skip_mode);
 void launch_ebe_elem_f32k(hipStream_t s, int32_t nelmt, const float* K,
-                          const int32_t* gdof, const double* p, double* Y,
+                          const int32_t* gdof, const double* p, double* Y, double* part,
                           const PcgScalars* sc, int skip_mode);
 void launch_ebe_packed_f64(hipStream_t s, int32_t nelmt, int n_cu, const double* KP,
-                           const int32_t* gdof, const double* p, double* Y,
+                           const int32_t* gdof, const double* p, double* Y, double* part,
                            const PcgScalars* sc, int skip_mode);
 void launch_ebe_packed_f32(hipStream_t s, int32_t nelmt, const float* KP,
-                           const int32_t* gdof, const double* p, double* Y,
+                           const int32_t* gdof, const double* p, double* Y, double* part,
                            const PcgScalars* sc, int skip_mode);
 // product of a built mesh without stored matrices; lame: (lambda, mu) per material
 void launch_lame(hipStream_t s, int nmat, const double* ym, const double* nu, double2* lame);
 void launch_mf64(hipStream_t s, int32_t nelmt, const double* corners, const int32_t* gdof,
                  const int32_t* mat_id, const double2* lame, const double* p, double* Y,
-                 const PcgScalars* sc, int skip_mode);
+                 double* part, const PcgScalars* sc, int skip_mode);
+// blocks of each product, the partials it writes when `part` is given
+int mf64_blocks(int32_t nelmt);
+int ebe_elem_blocks(int32_t nelmt);
+int ebe_packed_blocks(int32_t nelmt, int n_cu);
 void launch_pack_upper_f64(hipStream_t s, int32_t nelmt, const double* K,
                            double* KP);
 void launch_pack_upper_f32(hipStream_t s, int32_t nelmt, const double* K,
@@ -87,17 +91,30 @@ void launch_pcg_begin(hipStream_t s, int64_t n1, const double* u, double* part,
                       PcgScalars* sc, double tol, int32_t maxiter);
 void launch_pcg_init(hipStream_t s, int64_t n1, const double* f,
                      const double* kp, const double* dinv, double* r, double* z,
-                     double* p, double* part, PcgScalars* sc, int seq);
-void launch_pcg_assemble_dot(hipStream_t s, int64_t n1, const int32_t* rowptr,
+                     double* p, PcgScalars* sc);
+void launch_pcg_assemble(hipStream_t s, int64_t n1, const int32_t* rowptr,
                              const int32_t* slots, const double* Y,
                              const double* p, double* kp, double* part,
-                             PcgScalars* sc, int seq);
+                             PcgScalars* sc);
 void launch_pcg_update(hipStream_t s, int64_t n1, const double* p,
                        const double* kp, const double* dinv, double* u,
-                       double* r, double* z, double* part, PcgScalars* sc,
-                       int seq);
+                       double* r, double* z, double* part, PcgScalars* sc);
 void launch_pcg_pupdate(hipStream_t s, int64_t n1, const double* z, double* p,
                         const PcgScalars* sc);
+// partials of a tree-reduced solve (sgeo_pcg.hip): where each kind lives
+struct PcgPart {
+  int block, n_dot, n_vec;
+  double *dot, *u, *rz, *p[2], *c_dot, *c_vec;
+};
+size_t pcg_tree_part(int n_dot, int64_t n1);
+PcgPart pcg_part(double* part, int n_dot, int64_t n1);
+void launch_pcg_start(hipStream_t s, int64_t n1, const double* f, const double* kp,
+                      const double* dinv, double* r, double* p, const PcgPart& q,
+                      PcgScalars* sc);
+void launch_pcg_iteration(hipStream_t s, int64_t n1, int it, const int32_t* rowptr,
+                          const int32_t* slots, const double* Y, double* kp,
+                          const double* dinv, double* u, double* r, double* p,
+                          const PcgPart& q, PcgScalars* sc);
 void launch_load(hipStream_t s, int64_t n1, const double* ext,
                  const double* body, double* load);
 void launch_uerr(hipStream_t s, int64_t n1, double* x, double* oldx,

@@ -120,7 +120,7 @@ __global__ __launch_bounds__(256) void k_mf64(
     int32_t nelmt, int32_t nblk, const double* __restrict__ corners,
     const int32_t* __restrict__ gdof, const int32_t* __restrict__ mat_id,
     const double2* __restrict__ lame, const double* __restrict__ p, double* __restrict__ Y,
-    const PcgScalars* __restrict__ sc, int skip_mode) {
+    double* __restrict__ part, const PcgScalars* __restrict__ sc, int skip_mode) {
   if (skip_mode == 1 && sc->done) return;
   if (skip_mode == 2 && !sc->u_nonzero) return;
   const int32_t per = gridDim.x / MF_XCD;  // the grid is a multiple of MF_XCD
@@ -167,6 +167,7 @@ __global__ __launch_bounds__(256) void k_mf64(
       for (int c = 0; c < 3; c++) s_R[el][3 * b + c][i] = R[b][c];
   }
   __syncthreads();
+  double d = 0.0;  // the node's share of p.Kp
   if (on) {
     const DRow<double> dx = d_col<double>(ix), dy = d_col<double>(iy), dz = d_col<double>(iz);
     const int nx = i - ix, ny = i - 3 * iy, nz = i - 9 * iz;
@@ -176,6 +177,7 @@ __global__ __launch_bounds__(256) void k_mf64(
       double y = fma(dx.c, rx[2], fma(dx.b, rx[1], dx.a * rx[0]));
       y = fma(dy.c, ry[6], fma(dy.b, ry[3], fma(dy.a, ry[0], y)));
       y = fma(dz.c, rz[18], fma(dz.b, rz[9], fma(dz.a, rz[0], y)));
+      d = fma(s_u[el * 81 + 3 * i + c], y, d);
       s_u[el * 81 + 3 * i + c] = y;  // read back only after the barrier
     }
   }
@@ -184,6 +186,10 @@ __global__ __launch_bounds__(256) void k_mf64(
   for (int k = 0; k < 3; k++) {
     const int q = t + 256 * k;
     if (q < ne * 81) Y[e0 * 81 + q] = s_u[q];
+  }
+  if (part) {  // the block's, by block index within the element order
+    d = block_sum<4>(d, s_xc);
+    if (t == 0) part[blk] = d;
   }
 }
 
@@ -200,14 +206,16 @@ void launch_lame(hipStream_t s, int nmat, const double* ym, const double* nu, do
   hipLaunchKernelGGL(k_lame, dim3((nmat + 63) / 64), dim3(64), 0, s, nmat, ym, nu, lame);
 }
 
+int mf64_blocks(int32_t nelmt) { return (nelmt + MF_EPB - 1) / MF_EPB; }
+
 void launch_mf64(hipStream_t s, int32_t nelmt, const double* corners, const int32_t* gdof,
                  const int32_t* mat_id, const double2* lame, const double* p, double* Y,
-                 const PcgScalars* sc, int skip_mode) {
+                 double* part, const PcgScalars* sc, int skip_mode) {
   if (nelmt <= 0) return;
-  const int32_t nblk = (nelmt + MF_EPB - 1) / MF_EPB;
+  const int32_t nblk = mf64_blocks(nelmt);
   const unsigned grid = (unsigned)((nblk + MF_XCD - 1) / MF_XCD * MF_XCD);
   hipLaunchKernelGGL(k_mf64, dim3(grid), dim3(256), 0, s, nelmt, nblk, corners, gdof, mat_id,
-                     lame, p, Y, sc, skip_mode);
+                     lame, p, Y, part, sc, skip_mode);
 }
 
 }  // namespace sgeo

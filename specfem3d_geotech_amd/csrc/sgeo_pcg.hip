@@ -14,6 +14,7 @@
 // operation as the reference does.
 #pragma clang fp contract(off)
 
+#include <algorithm>
 #include <type_traits>
 
 #include "sgeo_device.h"
@@ -30,6 +31,14 @@ static inline unsigned grid_stride_blocks(int64_t n) {
   return (unsigned)(b < 65536 ? (b > 0 ? b : 1) : 65536);
 }
 
+// the block's sum of v (NW waves) into its partial
+template <int NW>
+__device__ __forceinline__ void put_share(double v, double* __restrict__ part) {
+  __shared__ double red[NW];
+  v = block_sum<NW>(v, red);
+  if (threadIdx.x == 0) part[blockIdx.x] = v;
+}
+
 // --------------------------------------------------------------------------
 // EBE product, element part: Y[e] = K_e p_e
 // --------------------------------------------------------------------------
@@ -40,10 +49,11 @@ static inline unsigned grid_stride_blocks(int64_t n) {
 // into LDS once; row r sums c = 0..80 in order, as matmul(km, p(egdof))
 // (src/solver.f90:57).
 // skip_mode: 0 none, 1 return when sc->done, 2 return when !sc->u_nonzero.
+// part (may be NULL): the block's share of p.Kp = sum_e p_e . Y_e.
 template <typename KT>
 __global__ __launch_bounds__(256) void k_ebe_elem(
     int32_t nelmt, const KT* __restrict__ K, const int32_t* __restrict__ gdof,
-    const double* __restrict__ p, double* __restrict__ Y,
+    const double* __restrict__ p, double* __restrict__ Y, double* __restrict__ part,
     const PcgScalars* __restrict__ sc, int skip_mode) {
   if (skip_mode == 1 && sc->done) return;
   if (skip_mode == 2 && !sc->u_nonzero) return;
@@ -54,13 +64,17 @@ __global__ __launch_bounds__(256) void k_ebe_elem(
   const bool valid = (t < 243) && (e < nelmt);
   if (valid) pe[el][r] = p[gdof[e * 81 + r]];
   __syncthreads();
-  if (!valid) return;
-  const KT* ke = K + e * 6561 + r;
-  const double* pl = pe[el];
-  double a = 0.0;
+  double d = 0.0;
+  if (valid) {
+    const KT* ke = K + e * 6561 + r;
+    const double* pl = pe[el];
+    double a = 0.0;
 #pragma unroll 27
-  for (int c = 0; c < 81; c++) a = a + (double)ke[c * 81] * pl[c];
-  Y[e * 81 + r] = a;
+    for (int c = 0; c < 81; c++) a = a + (double)ke[c * 81] * pl[c];
+    Y[e * 81 + r] = a;
+    d = a * pl[r];
+  }
+  if (part) put_share<4>(d, part);
 }
 
 // --------------------------------------------------------------------------
@@ -77,7 +91,7 @@ __global__ __launch_bounds__(256) void k_ebe_elem(
 template <typename KT>
 __global__ __launch_bounds__(128) void k_ebe_packed(
     int32_t nelmt, const KT* __restrict__ KP, const int32_t* __restrict__ gdof,
-    const double* __restrict__ p, double* __restrict__ Y,
+    const double* __restrict__ p, double* __restrict__ Y, double* __restrict__ part,
     const PcgScalars* __restrict__ sc, int skip_mode) {
   if (skip_mode == 1 && sc->done) return;
   if (skip_mode == 2 && !sc->u_nonzero) return;
@@ -96,16 +110,20 @@ __global__ __launch_bounds__(128) void k_ebe_packed(
   for (int q = t; q < NV; q += 128) dst[q] = __builtin_nontemporal_load(src + q);
   if (t < 81) pe[t] = p[gdof[e * 81 + t]];
   __syncthreads();
-  if (t >= 81) return;
-  const int r = t;
-  const int rbase = r * (r + 1) / 2;
-  double a = 0.0;
+  double d = 0.0;
+  if (t < 81) {
+    const int r = t;
+    const int rbase = r * (r + 1) / 2;
+    double a = 0.0;
 #pragma unroll 9
-  for (int c = 0; c < 81; c++) {
-    const int idx = (r <= c) ? (c * (c + 1) / 2 + r) : (rbase + c);
-    a = a + (double)u[idx] * pe[c];
+    for (int c = 0; c < 81; c++) {
+      const int idx = (r <= c) ? (c * (c + 1) / 2 + r) : (rbase + c);
+      a = a + (double)u[idx] * pe[c];
+    }
+    Y[e * 81 + r] = a;
+    d = a * pe[r];
   }
-  Y[e * 81 + r] = a;
+  if (part) put_share<2>(d, part);
 }
 
 // Persistent, pipelined form of k_ebe_packed<double>: a few 128-thread
@@ -117,7 +135,7 @@ __global__ __launch_bounds__(128) void k_ebe_packed(
 // bits.
 __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
     int32_t nelmt, const double* __restrict__ KP, const int32_t* __restrict__ gdof,
-    const double* __restrict__ p, double* __restrict__ Y,
+    const double* __restrict__ p, double* __restrict__ Y, double* __restrict__ part,
     const PcgScalars* __restrict__ sc, int skip_mode) {
   if (skip_mode == 1 && sc->done) return;
   if (skip_mode == 2 && !sc->u_nonzero) return;
@@ -144,6 +162,7 @@ __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
   const int r = t;
   const int rbase = r * (r + 1) / 2;
   int cur = 0;
+  double share = 0.0;
   for (; e < nelmt; e += stride) {
     v2d* dst = reinterpret_cast<v2d*>(u);
 #pragma unroll
@@ -174,12 +193,14 @@ __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
         a = a + u[idx] * pl[c];
       }
       Y[e * 81 + r] = a;
+      share = share + a * pl[r];
       pe[cur ^ 1][t] = pn;
     }
     gn = gnn;
     __syncthreads();  // u and pe[cur] free, pe[cur ^ 1] visible
     cur ^= 1;
   }
+  if (part) put_share<2>(share, part);
 }
 
 // blocks per CU of the persistent FP64 product (LDS 28 KB per block)
@@ -282,52 +303,41 @@ __global__ __launch_bounds__(SGEO_VEC_THREADS) void k_pcg_begin(
   if (threadIdx.x == 0) part[blockIdx.x] = m;
 }
 
-// r = f - kp (kp = K u if u != 0, else 0); z = dinv*r; p = z; partial r.z
+// The kernels of the reference-order mode, whose dot products k_pcg_seqdot
+// forms.
+// r = f - kp (kp = K u if u != 0, else 0); z = dinv*r; p = z
 __global__ __launch_bounds__(SGEO_VEC_THREADS) void k_pcg_init(
     int64_t n1, const double* __restrict__ f, const double* __restrict__ kp,
     const double* __restrict__ dinv, double* __restrict__ r,
-    double* __restrict__ z, double* __restrict__ p, double* __restrict__ part,
-    const PcgScalars* __restrict__ sc) {
-  __shared__ double red[SGEO_VEC_THREADS / 64];
+    double* __restrict__ z, double* __restrict__ p, const PcgScalars* __restrict__ sc) {
   const bool unz = sc->u_nonzero != 0;
-  double s = 0.0;
   VEC_LOOP(g) {
     const double rg = f[g] - (unz ? kp[g] : 0.0);
     const double zg = dinv[g] * rg;
     r[g] = rg;
     z[g] = zg;
     p[g] = zg;
-    s = s + rg * zg;
   }
-  s = block_sum<SGEO_VEC_THREADS / 64>(s, red);
-  if (threadIdx.x == 0) part[blockIdx.x] = s;
 }
 
-// kp = assemble(Y); partial p.kp and max|p|
-__global__ __launch_bounds__(SGEO_VEC_THREADS) void k_pcg_assemble_dot(
+// kp = assemble(Y); partial max|p|
+__global__ __launch_bounds__(SGEO_VEC_THREADS) void k_pcg_assemble_max(
     int64_t n1, const int32_t* __restrict__ rowptr,
     const int32_t* __restrict__ slots, const double* __restrict__ Y,
     const double* __restrict__ p, double* __restrict__ kp,
     double* __restrict__ part, const PcgScalars* __restrict__ sc) {
   if (sc->done) return;
   __shared__ double red[SGEO_VEC_THREADS / 64];
-  double s = 0.0, m = 0.0;
+  double m = 0.0;
   VEC_LOOP(g) {
-    const double v = (g == 0) ? 0.0 : gather_row(rowptr, slots, Y, g);
-    kp[g] = v;
-    const double pg = p[g];
-    s = s + pg * v;
-    m = fmax(m, fabs(pg));
+    kp[g] = (g == 0) ? 0.0 : gather_row(rowptr, slots, Y, g);
+    m = fmax(m, fabs(p[g]));
   }
-  const double bs = block_sum<SGEO_VEC_THREADS / 64>(s, red);
   const double bm = block_max<SGEO_VEC_THREADS / 64>(m, red);
-  if (threadIdx.x == 0) {
-    part[blockIdx.x] = bs;
-    part[gridDim.x + blockIdx.x] = bm;
-  }
+  if (threadIdx.x == 0) part[blockIdx.x] = bm;
 }
 
-// u += alpha p; partial max|u|; r -= alpha kp; z = dinv r; partial r.z
+// u += alpha p; partial max|u|; r -= alpha kp; z = dinv r
 __global__ __launch_bounds__(SGEO_VEC_THREADS) void k_pcg_update(
     int64_t n1, const double* __restrict__ p, const double* __restrict__ kp,
     const double* __restrict__ dinv, double* __restrict__ u,
@@ -336,23 +346,17 @@ __global__ __launch_bounds__(SGEO_VEC_THREADS) void k_pcg_update(
   if (sc->done) return;
   __shared__ double red[SGEO_VEC_THREADS / 64];
   const double alpha = sc->alpha;
-  double m = 0.0, s = 0.0;
+  double m = 0.0;
   VEC_LOOP(g) {
     const double ug = u[g] + alpha * p[g];
     u[g] = ug;
     m = fmax(m, fabs(ug));
     const double rg = r[g] - alpha * kp[g];
-    const double zg = dinv[g] * rg;
     r[g] = rg;
-    z[g] = zg;
-    s = s + rg * zg;
+    z[g] = dinv[g] * rg;
   }
   const double bm = block_max<SGEO_VEC_THREADS / 64>(m, red);
-  const double bs = block_sum<SGEO_VEC_THREADS / 64>(s, red);
-  if (threadIdx.x == 0) {
-    part[blockIdx.x] = bm;
-    part[gridDim.x + blockIdx.x] = bs;
-  }
+  if (threadIdx.x == 0) part[blockIdx.x] = bm;
 }
 
 // p = z + beta p
@@ -370,37 +374,26 @@ __global__ __launch_bounds__(SGEO_VEC_THREADS) void k_pcg_pupdate(
 // finalize: one block combines the nb partials in index order
 // --------------------------------------------------------------------------
 enum FinWhat {
-  FIN_BEGIN = 0,   // part[0..nb): max|u|           -> u_nonzero, reset
-  FIN_RZ = 1,      // part[0..nb): r.z              -> rz
-  FIN_ALPHA = 2,   // p.kp, max|p|                  -> alpha
-  FIN_MAXP = 3,    // max|p| only (p.kp in reference order)
-  FIN_UPDATE = 4,  // max|u|, r.z                   -> stop test, beta
-  FIN_UPDATE_NOBETA = 5,  // stop test only (r.z in reference order)
+  FIN_BEGIN = 0,   // max|u|  -> u_nonzero, reset
+  FIN_RZ = 1,      // r.z     -> rz
+  FIN_MAXP = 2,    // max|p|  (reference-order mode)
+  FIN_UPDATE = 3,  // max|u|  -> stop test (reference-order mode)
 };
 
 __global__ __launch_bounds__(256) void k_pcg_finalize(
     int nb, const double* __restrict__ part, PcgScalars* __restrict__ sc,
     int what, double tol, int32_t maxiter) {
   __shared__ double red[4];
-  if (what >= FIN_ALPHA && sc->done) return;
-  double v0 = 0.0, v1 = 0.0;
-  for (int b = threadIdx.x; b < nb; b += 256) {
-    const double a = part[b];
-    if (what == FIN_BEGIN) v0 = fmax(v0, a);
-    else if (what == FIN_UPDATE || what == FIN_UPDATE_NOBETA) v0 = fmax(v0, a);
-    else if (what != FIN_MAXP) v0 = v0 + a;
-    if (what == FIN_ALPHA || what == FIN_MAXP) v1 = fmax(v1, part[nb + b]);
-    if (what == FIN_UPDATE) v1 = v1 + part[nb + b];
-  }
-  const bool v0max = (what == FIN_BEGIN || what == FIN_UPDATE ||
-                      what == FIN_UPDATE_NOBETA);
-  v0 = v0max ? block_max<4>(v0, red) : block_sum<4>(v0, red);
-  const bool v1max = (what == FIN_ALPHA || what == FIN_MAXP);
-  v1 = v1max ? block_max<4>(v1, red) : block_sum<4>(v1, red);
+  if (what >= FIN_MAXP && sc->done) return;
+  double v = 0.0;
+#pragma unroll 4
+  for (int b = threadIdx.x; b < nb; b += 256)
+    v = what == FIN_RZ ? v + part[b] : fmax(v, part[b]);
+  v = what == FIN_RZ ? block_sum<4>(v, red) : block_max<4>(v, red);
   if (threadIdx.x != 0) return;
   switch (what) {
     case FIN_BEGIN:
-      sc->u_nonzero = v0 > 0.0 ? 1 : 0;
+      sc->u_nonzero = v > 0.0 ? 1 : 0;
       sc->iter = 0;
       sc->done = 0;
       sc->conv_iter = 0;
@@ -408,35 +401,278 @@ __global__ __launch_bounds__(256) void k_pcg_finalize(
       sc->maxiter = maxiter;
       break;
     case FIN_RZ:
-      sc->rz = v0;
-      break;
-    case FIN_ALPHA:
-      sc->pkp = v0;
-      sc->maxp = v1;
-      sc->alpha = sc->rz / v0;
+      sc->rz = v;
       break;
     case FIN_MAXP:
-      sc->maxp = v1;
+      sc->maxp = v;
       break;
-    case FIN_UPDATE:
-    case FIN_UPDATE_NOBETA: {
+    case FIN_UPDATE: {
       const int it = sc->iter + 1;
       sc->iter = it;
-      sc->maxu = v0;
+      sc->maxu = v;
       // src/solver.f90:65: stop after the u update, before the r update
-      if (fabs(sc->alpha) * sc->maxp / v0 <= sc->tol) {
+      if (fabs(sc->alpha) * sc->maxp / v <= sc->tol) {
         sc->done = 1;
         sc->conv_iter = it;
       } else if (it >= sc->maxiter) {
         sc->done = 2;
         sc->conv_iter = sc->maxiter + 1;  // DO-loop variable after exhaustion
-      } else if (what == FIN_UPDATE) {
-        sc->beta = v1 / sc->rz;
-        sc->rz = v1;
       }
       break;
     }
   }
+}
+
+// --------------------------------------------------------------------------
+// The iteration with tree-ordered reductions.  Linear solves run three
+// kernels:
+//   the element product, with its blocks' shares of p.Kp (p.Kp = sum_e
+//     p_e . Y_e, so alpha needs no assembled vector),
+//   k_pcg_step<true>: kp summed on the fly, u += alpha p, r -= alpha kp,
+//     partials of max|u| and r.z (z = dinv r is formed, not stored),
+//   k_pcg_dir: the stop test, p = z + beta p, partials of max|p|.
+// A trial's solves form p.Kp from the assembled vector (k_pcg_asm, then
+// k_pcg_step<false>): their x enters the yield function, which at the
+// corners of the Mohr-Coulomb pyramid turns the last bits of x into
+// relative changes of 1e-7 (asin near 1), so they keep the summation order
+// they have always had.
+// Every block combines the partials that the kernel before it left, all in
+// the same order, so that no one-block kernel stands between them; above
+// PCG_DIRECT partials k_pcg_collapse does it once, in that order, since each
+// block reading thousands would cost more than the extra launch.  The
+// scalars are double-buffered: the kernels of iteration `it` read
+// sc[it & 1] while k_pcg_dir's first block writes sc[(it + 1) & 1].
+// A block holds one equation per thread: the three dependent loads of a
+// gathered row set the time of small systems.  Blocks of 1,024 keep a
+// trial's partials (four values per lane, 256 equations apart, then the
+// lanes) and their number low; linear solves of up to 2^18 equations take
+// blocks of 256, four times as many compute units at work.
+// Measured, us per iteration without the product: 28,969 equations 29
+// before (five kernels, four rows per thread one after another), 12.7 with
+// blocks of 1,024, 10.6 with 256; 3,489,480 equations 141 before, 116 now.
+// --------------------------------------------------------------------------
+#define PCG_DIRECT 1024
+#define PCG_BLOCK 1024
+static_assert(PCG_BLOCK == SGEO_VEC_THREADS * SGEO_VEC_ITEMS, "partials of 1,024 equations");
+
+// sum (or max) of v[0..n) over the block in k_pcg_finalize's order; every
+// thread gets it
+template <bool MAX>
+__device__ __forceinline__ double combine(const double* __restrict__ v, int n, double* lds) {
+  if (n == 1) return v[0];
+  const int t = threadIdx.x;
+  if (t < 256) {
+    double a = 0.0;
+#pragma unroll 4
+    for (int b = t; b < n; b += 256) a = MAX ? fmax(a, v[b]) : a + v[b];
+    a = MAX ? wave_max(a) : wave_sum(a);
+    if ((t & 63) == 0) lds[t >> 6] = a;
+  }
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int i = 0; i < 4; i++) s = MAX ? fmax(s, lds[i]) : s + lds[i];
+  __syncthreads();
+  return s;
+}
+
+// partials in[k][0..n) -> out[k], kinds k < 3 (a NULL kind is left out); bit
+// k of `maxes`: a maximum.  One block.
+struct Kinds {
+  const double* in[3];
+  int maxes;
+};
+__global__ __launch_bounds__(256) void k_pcg_collapse(int n, Kinds kinds,
+                                                      double* __restrict__ out,
+                                                      const PcgScalars* __restrict__ sc) {
+  if (sc->done) return;
+  __shared__ double lds[4];
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    if (!kinds.in[k]) continue;
+    const double a = (kinds.maxes >> k) & 1 ? combine<true>(kinds.in[k], n, lds)
+                                            : combine<false>(kinds.in[k], n, lds);
+    if (threadIdx.x == 0) out[k] = a;
+  }
+}
+
+// a block's partial of one kind from its BS values; lds holds them
+template <int BS, bool MAX>
+__device__ __forceinline__ void block_partial(double v, double* lds, double* red,
+                                              double* __restrict__ part) {
+  const int t = threadIdx.x;
+  if (BS > 256) {
+    lds[t] = v;
+    __syncthreads();
+  }
+  if (t < 256) {
+    double a = BS > 256 ? 0.0 : v;
+#pragma unroll
+    for (int k = 0; k < BS / 256 && BS > 256; k++) a = MAX ? fmax(a, lds[t + 256 * k]) : a + lds[t + 256 * k];
+    a = MAX ? wave_max(a) : wave_sum(a);
+    if ((t & 63) == 0) red[t >> 6] = a;
+  }
+  __syncthreads();
+  if (t == 0) {
+    double s = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) s = MAX ? fmax(s, red[i]) : s + red[i];
+    part[blockIdx.x] = s;
+  }
+}
+
+// r = f - kp (kp = K u if u != 0, else 0); p = z = dinv r; r.z and max|p|
+template <int BS>
+__global__ __launch_bounds__(BS) void k_pcg_start(
+    int64_t n1, const double* __restrict__ f, const double* __restrict__ kp,
+    const double* __restrict__ dinv, double* __restrict__ r, double* __restrict__ p,
+    double* __restrict__ part_rz, double* __restrict__ part_p,
+    const PcgScalars* __restrict__ sc) {
+  __shared__ double lds[BS > 256 ? BS : 1], red[4];
+  const int64_t g = (int64_t)blockIdx.x * BS + threadIdx.x;
+  double s = 0.0, m = 0.0;
+  if (g < n1) {
+    const double rg = f[g] - (sc->u_nonzero ? kp[g] : 0.0);
+    const double zg = dinv[g] * rg;
+    r[g] = rg;
+    p[g] = zg;
+    s = rg * zg;
+    m = fabs(zg);
+  }
+  block_partial<BS, false>(s, lds, red, part_rz);
+  block_partial<BS, true>(m, lds, red, part_p);
+}
+
+// the row's element contributions (at most 8 on hexahedral meshes) loaded
+// together, then summed in slot order
+__device__ __forceinline__ double gather_row8(const int32_t* __restrict__ rowptr,
+                                              const int32_t* __restrict__ slots,
+                                              const double* __restrict__ Y, int64_t g) {
+  const int32_t q0 = rowptr[g], q1 = rowptr[g + 1];
+  double v[8];
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = q0 + i < q1 ? Y[slots[q0 + i]] : 0.0;
+  double kp = 0.0;
+#pragma unroll
+  for (int i = 0; i < 8; i++)
+    if (q0 + i < q1) kp = kp + v[i];
+  for (int32_t q = q0 + 8; q < q1; q++) kp = kp + Y[slots[q]];
+  return kp;
+}
+
+// kp and the partial of p.kp
+template <int BS>
+__global__ __launch_bounds__(BS) void k_pcg_asm(
+    int64_t n1, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ slots,
+    const double* __restrict__ Y, const double* __restrict__ p, double* __restrict__ kp,
+    double* __restrict__ part, const PcgScalars* __restrict__ sc) {
+  if (sc->done) return;
+  __shared__ double lds[BS > 256 ? BS : 1], red[4];
+  const int64_t g = (int64_t)blockIdx.x * BS + threadIdx.x;
+  double s = 0.0;
+  if (g < n1) {
+    const double v = g == 0 ? 0.0 : gather_row8(rowptr, slots, Y, g);
+    kp[g] = v;
+    s = p[g] * v;
+  }
+  block_partial<BS, false>(s, lds, red, part);
+}
+
+// n_dot partials of p.Kp in `dot`; FUSED: kp is summed from Y here
+template <int BS, bool FUSED>
+__global__ __launch_bounds__(BS) void k_pcg_step(
+    int64_t n1, const int32_t* __restrict__ rowptr, const int32_t* __restrict__ slots,
+    const double* __restrict__ Y, const double* __restrict__ kp,
+    const double* __restrict__ p, const double* __restrict__ dinv, double* __restrict__ u,
+    double* __restrict__ r, const double* __restrict__ dot, int n_dot,
+    double* __restrict__ part_u, double* __restrict__ part_rz, PcgScalars* __restrict__ sc) {
+  if (sc->done) return;
+  __shared__ double lds[BS > 256 ? BS : 1], red[4];
+  const int64_t g = (int64_t)blockIdx.x * BS + threadIdx.x;
+  const bool in = g < n1;
+  double v = 0.0, ug = 0.0, pg = 0.0, rg = 0.0, dg = 0.0;
+  if (in) {  // in flight while the partials are combined
+    ug = u[g];
+    pg = p[g];
+    rg = r[g];
+    dg = dinv[g];
+    if (!FUSED) v = kp[g];
+    else if (g > 0) v = gather_row8(rowptr, slots, Y, g);
+  }
+  const double pkp = combine<false>(dot, n_dot, red);
+  const double alpha = sc->rz / pkp;
+  double m = 0.0, s = 0.0;
+  if (in) {
+    ug = ug + alpha * pg;
+    u[g] = ug;
+    m = fabs(ug);
+    rg = rg - alpha * v;
+    r[g] = rg;
+    s = rg * (dg * rg);
+  }
+  block_partial<BS, true>(m, lds, red, part_u);
+  block_partial<BS, false>(s, lds, red, part_rz);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {  // read by later kernels only
+    sc->pkp = pkp;
+    sc->alpha = alpha;
+  }
+}
+
+// n_part partials of max|u|, r.z and this iteration's max|p|
+template <int BS>
+__global__ __launch_bounds__(BS) void k_pcg_dir(
+    int64_t n1, const double* __restrict__ r, const double* __restrict__ dinv,
+    double* __restrict__ p, const double* __restrict__ part_u,
+    const double* __restrict__ part_rz, const double* __restrict__ part_p, int n_part,
+    double* __restrict__ part_pn, const PcgScalars* __restrict__ sc,
+    PcgScalars* __restrict__ scn) {
+  const bool writer = blockIdx.x == 0 && threadIdx.x == 0;
+  if (sc->done) {
+    if (writer) *scn = *sc;
+    return;
+  }
+  __shared__ double lds[BS > 256 ? BS : 1], red[4];
+  const int64_t g = (int64_t)blockIdx.x * BS + threadIdx.x;
+  const bool in = g < n1;
+  double rg = 0.0, dg = 0.0, pg = 0.0;
+  if (in) {
+    rg = r[g];
+    dg = dinv[g];
+    pg = p[g];
+  }
+  const double maxu = combine<true>(part_u, n_part, red);
+  const double rz = combine<false>(part_rz, n_part, red);
+  const double maxp = combine<true>(part_p, n_part, red);
+  const int it = sc->iter + 1;
+  // src/solver.f90:65: the relative update of u
+  const bool conv = fabs(sc->alpha) * maxp / maxu <= sc->tol;
+  const bool fail = !conv && it >= sc->maxiter;
+  const double beta = rz / sc->rz;
+  if (writer) {
+    PcgScalars n = *sc;
+    n.iter = it;
+    n.maxu = maxu;
+    n.maxp = maxp;
+    if (conv) {
+      n.done = 1;
+      n.conv_iter = it;
+    } else if (fail) {
+      n.done = 2;
+      n.conv_iter = sc->maxiter + 1;  // DO-loop variable after exhaustion
+    } else {
+      n.beta = beta;
+      n.rz = rz;
+    }
+    *scn = n;
+  }
+  if (conv || fail) return;
+  double m = 0.0;
+  if (in) {
+    pg = dg * rg + beta * pg;
+    p[g] = pg;
+    m = fabs(pg);
+  }
+  block_partial<BS, true>(m, lds, red, part_pn);
 }
 
 // --------------------------------------------------------------------------
@@ -682,37 +918,40 @@ void launch_csr_build(hipStream_t s, int64_t ns, int32_t neq, const int32_t* gdo
 // launch wrappers
 // --------------------------------------------------------------------------
 void launch_ebe_elem_f64(hipStream_t s, int32_t nelmt, const double* K,
-                         const int32_t* gdof, const double* p, double* Y,
+                         const int32_t* gdof, const double* p, double* Y, double* part,
                          const PcgScalars* sc, int skip_mode) {
   if (nelmt <= 0) return;
   hipLaunchKernelGGL(k_ebe_elem<double>, dim3(nblk(nelmt, 3)), dim3(256), 0, s,
-                     nelmt, K, gdof, p, Y, sc, skip_mode);
+                     nelmt, K, gdof, p, Y, part, sc, skip_mode);
 }
 
 void launch_ebe_elem_f32k(hipStream_t s, int32_t nelmt, const float* K,
-                          const int32_t* gdof, const double* p, double* Y,
+                          const int32_t* gdof, const double* p, double* Y, double* part,
                           const PcgScalars* sc, int skip_mode) {
   if (nelmt <= 0) return;
   hipLaunchKernelGGL(k_ebe_elem<float>, dim3(nblk(nelmt, 3)), dim3(256), 0, s,
-                     nelmt, K, gdof, p, Y, sc, skip_mode);
+                     nelmt, K, gdof, p, Y, part, sc, skip_mode);
 }
 
 void launch_ebe_packed_f64(hipStream_t s, int32_t nelmt, int n_cu, const double* KP,
-                           const int32_t* gdof, const double* p, double* Y,
+                           const int32_t* gdof, const double* p, double* Y, double* part,
                            const PcgScalars* sc, int skip_mode) {
   if (nelmt <= 0) return;
-  int64_t g = (int64_t)n_cu * EBE_PIPE_BLOCKS_PER_CU;
-  if (g > nelmt) g = nelmt;
-  hipLaunchKernelGGL(k_ebe_packed_pipe, dim3((unsigned)g), dim3(128), 0, s, nelmt, KP,
-                     gdof, p, Y, sc, skip_mode);
+  hipLaunchKernelGGL(k_ebe_packed_pipe, dim3((unsigned)ebe_packed_blocks(nelmt, n_cu)), dim3(128), 0, s, nelmt, KP,
+                     gdof, p, Y, part, sc, skip_mode);
 }
 
 void launch_ebe_packed_f32(hipStream_t s, int32_t nelmt, const float* KP,
-                           const int32_t* gdof, const double* p, double* Y,
+                           const int32_t* gdof, const double* p, double* Y, double* part,
                            const PcgScalars* sc, int skip_mode) {
   if (nelmt <= 0) return;
   hipLaunchKernelGGL(k_ebe_packed<float>, dim3(nelmt), dim3(128), 0, s, nelmt,
-                     KP, gdof, p, Y, sc, skip_mode);
+                     KP, gdof, p, Y, part, sc, skip_mode);
+}
+
+int ebe_elem_blocks(int32_t nelmt) { return (int)nblk(nelmt, 3); }
+int ebe_packed_blocks(int32_t nelmt, int n_cu) {
+  return std::min<int64_t>((int64_t)n_cu * EBE_PIPE_BLOCKS_PER_CU, nelmt);
 }
 
 void launch_pack_upper_f64(hipStream_t s, int32_t nelmt, const double* K,
@@ -759,49 +998,118 @@ void launch_pcg_begin(hipStream_t s, int64_t n1, const double* u, double* part,
                      (int)FIN_BEGIN, tol, maxiter);
 }
 
+// reference-order dot products (k_pcg_seqdot)
 void launch_pcg_init(hipStream_t s, int64_t n1, const double* f,
                      const double* kp, const double* dinv, double* r, double* z,
-                     double* p, double* part, PcgScalars* sc, int seq) {
+                     double* p, PcgScalars* sc) {
   const unsigned nb = vec_reduce_blocks(n1);
   hipLaunchKernelGGL(k_pcg_init, dim3(nb), dim3(SGEO_VEC_THREADS), 0, s, n1, f,
-                     kp, dinv, r, z, p, part, sc);
-  if (seq)
-    hipLaunchKernelGGL(k_pcg_seqdot, dim3(1), dim3(256), 0, s, n1, r, z, sc, 0);
-  else
-    hipLaunchKernelGGL(k_pcg_finalize, dim3(1), dim3(256), 0, s, (int)nb, part,
-                       sc, (int)FIN_RZ, 0.0, 0);
+                     kp, dinv, r, z, p, sc);
+  hipLaunchKernelGGL(k_pcg_seqdot, dim3(1), dim3(256), 0, s, n1, r, z, sc, 0);
 }
 
-void launch_pcg_assemble_dot(hipStream_t s, int64_t n1, const int32_t* rowptr,
+void launch_pcg_assemble(hipStream_t s, int64_t n1, const int32_t* rowptr,
                              const int32_t* slots, const double* Y,
                              const double* p, double* kp, double* part,
-                             PcgScalars* sc, int seq) {
+                             PcgScalars* sc) {
   const unsigned nb = vec_reduce_blocks(n1);
-  hipLaunchKernelGGL(k_pcg_assemble_dot, dim3(nb), dim3(SGEO_VEC_THREADS), 0, s,
+  hipLaunchKernelGGL(k_pcg_assemble_max, dim3(nb), dim3(SGEO_VEC_THREADS), 0, s,
                      n1, rowptr, slots, Y, p, kp, part, sc);
   hipLaunchKernelGGL(k_pcg_finalize, dim3(1), dim3(256), 0, s, (int)nb, part, sc,
-                     (int)(seq ? FIN_MAXP : FIN_ALPHA), 0.0, 0);
-  if (seq)
-    hipLaunchKernelGGL(k_pcg_seqdot, dim3(1), dim3(256), 0, s, n1, p, kp, sc, 1);
+                     (int)FIN_MAXP, 0.0, 0);
+  hipLaunchKernelGGL(k_pcg_seqdot, dim3(1), dim3(256), 0, s, n1, p, kp, sc, 1);
 }
 
 void launch_pcg_update(hipStream_t s, int64_t n1, const double* p,
                        const double* kp, const double* dinv, double* u,
-                       double* r, double* z, double* part, PcgScalars* sc,
-                       int seq) {
+                       double* r, double* z, double* part, PcgScalars* sc) {
   const unsigned nb = vec_reduce_blocks(n1);
   hipLaunchKernelGGL(k_pcg_update, dim3(nb), dim3(SGEO_VEC_THREADS), 0, s, n1, p,
                      kp, dinv, u, r, z, part, sc);
   hipLaunchKernelGGL(k_pcg_finalize, dim3(1), dim3(256), 0, s, (int)nb, part, sc,
-                     (int)(seq ? FIN_UPDATE_NOBETA : FIN_UPDATE), 0.0, 0);
-  if (seq)
-    hipLaunchKernelGGL(k_pcg_seqdot, dim3(1), dim3(256), 0, s, n1, r, z, sc, 2);
+                     (int)FIN_UPDATE, 0.0, 0);
+  hipLaunchKernelGGL(k_pcg_seqdot, dim3(1), dim3(256), 0, s, n1, r, z, sc, 2);
 }
 
 void launch_pcg_pupdate(hipStream_t s, int64_t n1, const double* z, double* p,
                         const PcgScalars* sc) {
   hipLaunchKernelGGL(k_pcg_pupdate, dim3(grid_stride_blocks(n1)),
                      dim3(SGEO_VEC_THREADS), 0, s, n1, z, p, sc);
+}
+
+// equations per block (n_dot 0: a trial's solve, or one without shares)
+static inline int pcg_block(int n_dot, int64_t n1) {
+  return n_dot > 0 && n1 <= (1 << 18) ? 256 : PCG_BLOCK;
+}
+
+// doubles of a solve's partials: p.Kp (n_dot shares, or one per block of
+// equations), max|u| and r.z, two generations of max|p|, collapsed forms
+size_t pcg_tree_part(int n_dot, int64_t n1) {
+  const int nv = (int)nblk(n1, pcg_block(n_dot, n1));
+  return (size_t)std::max(n_dot, nv) + 4 * (size_t)nv + 4;
+}
+
+PcgPart pcg_part(double* part, int n_dot, int64_t n1) {
+  PcgPart q;
+  q.block = pcg_block(n_dot, n1);
+  q.n_vec = (int)nblk(n1, q.block);
+  q.n_dot = n_dot > 0 ? n_dot : q.n_vec;  // 0: from the assembled vector
+  q.dot = part;
+  q.u = q.dot + std::max(q.n_dot, q.n_vec);
+  q.rz = q.u + q.n_vec;
+  q.p[0] = q.rz + q.n_vec;
+  q.p[1] = q.p[0] + q.n_vec;
+  q.c_dot = q.p[1] + q.n_vec;
+  q.c_vec = q.c_dot + 1;
+  return q;
+}
+
+void launch_pcg_start(hipStream_t s, int64_t n1, const double* f, const double* kp,
+                      const double* dinv, double* r, double* p, const PcgPart& q,
+                      PcgScalars* sc) {
+  const auto k = q.block == 256 ? k_pcg_start<256> : k_pcg_start<PCG_BLOCK>;
+  hipLaunchKernelGGL(k, dim3(q.n_vec), dim3(q.block), 0, s, n1, f, kp, dinv, r, p, q.rz,
+                     q.p[0], (const PcgScalars*)sc);
+  hipLaunchKernelGGL(k_pcg_finalize, dim3(1), dim3(256), 0, s, q.n_vec, (const double*)q.rz,
+                     sc, (int)FIN_RZ, 0.0, 0);
+}
+
+// what follows the product in iteration `it` (0-based; sc: two buffers);
+// kp: NULL when the product left its shares of p.Kp
+void launch_pcg_iteration(hipStream_t s, int64_t n1, int it, const int32_t* rowptr,
+                          const int32_t* slots, const double* Y, double* kp,
+                          const double* dinv, double* u, double* r, double* p,
+                          const PcgPart& q, PcgScalars* sc) {
+  PcgScalars *cur = sc + (it & 1), *nxt = sc + (~it & 1);
+  const PcgScalars* cc = cur;
+  const double *dot = q.dot, *pu = q.u, *prz = q.rz, *pp = q.p[it & 1];
+  const dim3 grid(q.n_vec), block(q.block);
+  int nd = q.n_dot, np = q.n_vec;
+  if (kp)
+    hipLaunchKernelGGL(k_pcg_asm<PCG_BLOCK>, grid, block, 0, s, n1, rowptr, slots, Y,
+                       (const double*)p, kp, q.dot, cc);
+  if (nd > PCG_DIRECT) {
+    hipLaunchKernelGGL(k_pcg_collapse, dim3(1), dim3(256), 0, s, nd,
+                       Kinds{{dot, nullptr, nullptr}, 0}, q.c_dot, cc);
+    dot = q.c_dot;
+    nd = 1;
+  }
+  const auto step = kp               ? k_pcg_step<PCG_BLOCK, false>
+                    : q.block == 256 ? k_pcg_step<256, true>
+                                     : k_pcg_step<PCG_BLOCK, true>;
+  hipLaunchKernelGGL(step, grid, block, 0, s, n1, rowptr, slots, Y, (const double*)kp,
+                     (const double*)p, dinv, u, r, dot, nd, q.u, q.rz, cur);
+  if (np > PCG_DIRECT) {
+    hipLaunchKernelGGL(k_pcg_collapse, dim3(1), dim3(256), 0, s, np, Kinds{{pu, prz, pp}, 5},
+                       q.c_vec, cc);
+    pu = q.c_vec;
+    prz = pu + 1;
+    pp = pu + 2;
+    np = 1;
+  }
+  const auto dir = q.block == 256 ? k_pcg_dir<256> : k_pcg_dir<PCG_BLOCK>;
+  hipLaunchKernelGGL(dir, grid, block, 0, s, n1, (const double*)r, dinv, p, pu, prz, pp, np,
+                     q.p[~it & 1], cc, nxt);
 }
 
 void launch_load(hipStream_t s, int64_t n1, const double* ext,

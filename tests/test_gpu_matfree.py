@@ -51,3 +51,39 @@ def test_packed_product_from_geometry(ctx, grid):
         assert rel_l2(dm.matvec(p), 2.0 * full) < 1e-14
     finally:
         dm.close()
+
+
+# 2^18 equations is where the blocks of the vector kernels change; the small
+# grids have fewer equations than the product has shares of p.Kp
+@pytest.mark.parametrize("grid,full", [((1, 1, 1), True), ((2, 1, 1), True), ((4, 2, 3), True),
+                                       ((37, 7, 19), False), ((40, 10, 27), False),
+                                       ((41, 10, 27), True)])
+def test_solve_against_separate_reference_order(ctx, grid, full):
+    """The tree-reduced solve equals the reference-order one at a tight
+    tolerance: both stop at relative updates of 1e-13, so they differ by a
+    few hundred such updates at most."""
+    from specfem3d_geotech_amd.solver import REDUCE_SEQUENTIAL, REDUCE_TREE
+    mesh = _mesh(*grid)
+    spec = hex2spec(mesh)
+    gam, ym, nu, *_ = mesh.material_arrays()
+    dm = DeviceMesh(ctx, spec, len(gam))
+    try:
+        ext, _ = dm.build_stiffness(gam, ym, nu)
+        dm.set_operator(K_F64, KFMT_FULL if full else KFMT_PACKED)
+        cap = 20000 if spec.neq < 5000 else 40
+        u, it, ec = dm.solve(ext, cg_tol=1e-13, cg_maxiter=cap)
+        ctx.set_reduction(REDUCE_SEQUENTIAL)
+        v, jt, fc = dm.solve(ext, cg_tol=1e-13, cg_maxiter=cap)
+        # a warm start goes through the first residual's product
+        w, _, _ = dm.solve(ext, u0=v, cg_tol=1e-13, cg_maxiter=cap)
+        ctx.set_reduction(REDUCE_TREE)
+        x, _, _ = dm.solve(ext, u0=v, cg_tol=1e-13, cg_maxiter=cap)
+        assert ec == fc and abs(it - jt) <= 0.02 * jt
+        assert rel_l2(u, v) < 1e-10
+        assert rel_l2(x, w) < 1e-10
+        # at most two iterations
+        assert dm.solve(ext, cg_tol=1e-13, cg_maxiter=1)[1:] == (2, -1)
+        assert dm.solve(ext, cg_tol=1e-13, cg_maxiter=17)[1] <= 18
+    finally:
+        ctx.set_reduction(REDUCE_TREE)
+        dm.close()
