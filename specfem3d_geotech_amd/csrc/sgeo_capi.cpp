@@ -120,6 +120,8 @@ struct sgeo_mesh {
   // from them; false for uploaded matrices
   bool built = false;
   double2* d_lame = nullptr;  // (lambda, mu) per material of the built K
+  float4* d_geo = nullptr;    // the batched product's geometry, of version geo_ver
+  int geo_ver = -1;
   int k_ver = 0, k32_ver = -1, kp64_ver = -1, kp32_ver = -1;
   double* d_dinv = nullptr;
   // node map of the nodal result fields (sgeo_mesh_set_nodes)
@@ -389,7 +391,7 @@ extern "C" int sgeo_mesh_destroy(sgeo_mesh* m) {
                   m->d_K64,  m->d_K32,    m->d_KP64,  m->d_KP32,
                   m->d_dinv,  m->d_Y,       m->d_r,
                   m->d_z,    m->d_p,      m->d_kp,    m->d_nrowptr, m->d_nslots,
-                  m->d_lame};
+                  m->d_lame, m->d_geo};
   for (void* p : ptrs)
     if (p) hipFree(p);
   delete m;
@@ -1573,6 +1575,7 @@ struct sgeo_batch {
   int32_t memo_cg = 0;
   int64_t stat_inner = 0, stat_outer = 0, stat_steps = 0;
   int k_ver = -1;  // mesh stiffness version the FP32 diagonal was made from
+  bool built = false;  // the product the captured steps hold (sgeo_mesh::built)
   size_t bytes = 0;
   // HIP graphs of 8, 16 and 32 steps (every launch argument is fixed for
   // the engine's lifetime: the steps read their state from the device)
@@ -1608,9 +1611,22 @@ struct sgeo_batch {
 
 // Packed FP32/FP64 operators and the FP32 inverse diagonal follow the mesh's
 // current stiffness (rebuilt when K changed since the last call).
+static void batch_drop_graphs(sgeo_batch* b);
+
 static int batch_sync_operator(sgeo_batch* b) {
   sgeo_mesh* m = b->mesh;
-  TRY(ensure_packed(m, SGEO_K_F32));
+  if (b->built != m->built) batch_drop_graphs(b);  // they launch the other product
+  b->built = m->built;
+  if (m->built) {  // the FP32 product runs from the geometry
+    if (!m->d_geo) TRY(dalloc(&m->d_geo, (size_t)m->nelmt * 81, &m->bytes));
+    if (m->geo_ver != m->k_ver) {
+      launch_point_geometry(m->ctx->stream, m->nelmt, m->d_corners, m->d_mat, m->d_lame,
+                            m->d_geo);
+      m->geo_ver = m->k_ver;
+    }
+  } else {
+    TRY(ensure_packed(m, SGEO_K_F32));
+  }
   TRY(ensure_packed(m, SGEO_K_F64));
   if (b->k_ver != m->k_ver) {
     launch_to_f32(m->ctx->stream, b->n1, m->d_dinv, b->d_dinv32);
@@ -1826,7 +1842,21 @@ extern "C" int sgeo_batch_set_geometry(sgeo_batch* b, int32_t blocks_per_cu,
   return 0;
 }
 
-// Launch-geometry autotuner of the MFMA product: times `reps` launches of
+// Y = K P of the iterating columns, and the elements' p.Kp shares: from the
+// geometry on built meshes, else on the stored packed FP32 matrices
+static void batch_product(sgeo_batch* b, BmvGeom g) {
+  sgeo_mesh* m = b->mesh;
+  const int want = BCOL_BIT(BCOL_INNER);
+  if (m->built)
+    launch_bmf(m->ctx->stream, m->nelmt, b->B, g, m->d_geo, m->d_gdof,
+               b->d_eorder, b->d_p, b->n1 * b->B, b->d_Y32, b->d_edot, b->d_cst, b->d_bc, want);
+  else
+    launch_bmv_mfma_f32(m->ctx->stream, m->nelmt, b->B, m->ctx->n_cu, g, m->d_KP32, m->d_gdof,
+                        b->d_eorder, b->d_p, b->n1 * b->B, b->d_Y32, b->d_edot, b->d_cst,
+                        b->d_bc, want);
+}
+
+// Launch-geometry autotuner of the product: times `reps` launches of
 // every candidate (blocks per CU 1..3, XCD-aware split on/off) on the
 // engine's own mesh and the columns iterating now, and keeps the fastest.
 // The product only rewrites the element products of iterating columns from
@@ -1855,9 +1885,7 @@ extern "C" int sgeo_batch_autotune(sgeo_batch* b, int32_t reps, int32_t* blocks_
       g.blocks_per_cu = bpc;
       g.xcd_split = xs;
       auto launch = [&]() {
-        launch_bmv_mfma_f32(s, m->nelmt, b->B, c->n_cu, g, m->d_KP32, m->d_gdof,
-                            b->d_eorder, b->d_p, b->n1 * b->B, b->d_Y32, b->d_edot,
-                            b->d_cst, b->d_bc, BCOL_BIT(BCOL_INNER));
+        batch_product(b, g);
       };
       launch();  // warm-up
       HIPCHK(hipEventRecord(e0, s));
@@ -2141,9 +2169,7 @@ static void batch_step_launches(sgeo_batch* b, bool prof, bool resid, bool xw) {
   launch_bpupdate(s, n1, B, b->d_r, b->d_dinv32, b->d_p, b->d_part, b->d_cst, b->d_bc);
   if (prof) prof_mark(c);
   // Y = K P and the elements' p.Kp shares; alpha = r.z / p.Kp
-  launch_bmv_mfma_f32(s, m->nelmt, B, c->n_cu, b->geom, m->d_KP32, m->d_gdof, b->d_eorder,
-                      b->d_p, n1 * B, b->d_Y32, b->d_edot, b->d_cst, b->d_bc,
-                      BCOL_BIT(BCOL_INNER));
+  batch_product(b, b->geom);
   if (prof) prof_mark(c);
   launch_bfinalize(s, m->nelmt, B, b->d_edot, b->d_cst, b->d_bc, BFIN_ALPHA);
   // kp assembled from Y; r and r.z; on the x-writing steps x and max|x|;

@@ -87,3 +87,57 @@ def test_solve_against_separate_reference_order(ctx, grid, full):
     finally:
         ctx.set_reduction(REDUCE_TREE)
         dm.close()
+
+
+def _engine_x(ctx, mesh, spec, ncol, steps, upload=False, cols=1):
+    """x of column 0 after exactly `steps` CG steps of `cols` columns of the
+    elastic solve."""
+    from specfem3d_geotech_amd.batch import DEFAULT_INNER_TOL, BatchEngine, device_mesh
+    from specfem3d_geotech_amd.plastic import dt_viscoplas
+    _, ym, nu, phi, coh, psi = mesh.material_arrays()
+    dm, ext = device_mesh(ctx, mesh, spec)
+    try:
+        if upload:
+            _, dinv = dm.build_stiffness(mesh.material_arrays()[0], ym, nu)
+            dm.upload_stiffness(dm.download_stiffness(), dinv)
+        eng = BatchEngine(dm, ext, ncol)
+        try:
+            for j in range(cols):
+                eng.begin(j, ym, nu, phi, coh, psi, dt_viscoplas(nu, phi, ym))
+            if steps:
+                eng.advance(1e-14, 5000, DEFAULT_INNER_TOL, 5e-4, 300, max_steps=steps)
+            else:
+                eng.plastic_iter(np.zeros(ncol, np.int32), 1e-12, 20000, DEFAULT_INNER_TOL, 5e-4)
+            return eng.download(0)[0]
+        finally:
+            eng.close()
+    finally:
+        dm.close()
+
+
+def test_batched_product_same_bits_for_every_column_count(ctx):
+    """A column's bits do not depend on the engine's column count: 1 to 64
+    columns on 65,600 elements (a lane per element and column) and on 1,025
+    (64 columns by lanes, fewer by points), with idle columns beside it."""
+    for grid, steps in (((41, 40, 40), 16), ((41, 5, 5), 24)):
+        mesh = _mesh(*grid)
+        spec = hex2spec(mesh) if mesh.nelmt < 5000 else __import__(
+            "specfem3d_geotech_amd.spec", fromlist=["x"]).hex2spec_device(ctx, mesh)
+        ref = None
+        for ncol in (1, 2, 4, 8, 16, 32, 64):
+            x = _engine_x(ctx, mesh, spec, ncol, steps, cols=min(ncol, 3))
+            assert np.abs(x).max() > 0
+            ref = x if ref is None else ref
+            assert np.array_equal(x, ref), ncol
+
+
+@pytest.mark.parametrize("grid", [(1, 1, 1), (3, 1, 1), (3, 3, 1), (8, 4, 6)])
+def test_batched_solve_from_geometry_and_from_uploaded_matrices(ctx, grid):
+    """The engine's converged solve is the same on a built mesh and on one
+    whose (identical) matrices were uploaded: both end at relative updates
+    of 1e-12 from FP64 residuals, so they agree to 1e-10."""
+    mesh = _mesh(*grid)
+    spec = hex2spec(mesh)
+    a = _engine_x(ctx, mesh, spec, 4, 0)
+    b = _engine_x(ctx, mesh, spec, 4, 0, upload=True)
+    assert rel_l2(a, b) < 1e-10
