@@ -434,339 +434,6 @@ __global__ __launch_bounds__(256) void k_bmv64(int32_t nelmt, int B,
   }
 }
 
-// --------------------------------------------------------------------------
-// batched vector kernels.  Equations are split into fixed chunks of ck
-// equations (ck depends on the equation count only, see batch_chunk);
-// thread t owns column j = t % B and chunk blockIdx*(256/B) + t/B, and walks
-// its chunk in order, so every per-(chunk, column) partial is a sequential
-// sum whose value does not depend on B.  The finalize then combines the
-// chunk partials in a fixed order.
-// Partials: part[(kind*nch + chunk)*B + j].
-// --------------------------------------------------------------------------
-struct ChunkIdx {
-  int j;
-  int64_t chunk, g0, g1;
-  bool valid;
-};
-
-__device__ __forceinline__ ChunkIdx chunk_of(int64_t n1, int B, int ck) {
-  ChunkIdx c;
-  const int t = threadIdx.x;
-  c.j = t % B;
-  c.chunk = (int64_t)blockIdx.x * (blockDim.x / B) + t / B;
-  c.g0 = c.chunk * ck;
-  c.g1 = c.g0 + ck < n1 ? c.g0 + ck : n1;
-  c.valid = c.g0 < n1;
-  return c;
-}
-
-__device__ __forceinline__ int64_t nchunks(int64_t n1, int ck) {
-  return (n1 + ck - 1) / ck;
-}
-
-// Small systems (`grouped`: fewer than 16,384 chunks) combine the partials
-// of four consecutive chunks inside the block, in chunk order, and write
-// one value per group, part[(kind * ng4 + chunk / 4) * B + j] with
-// ng4 = ceil(nch / 4), which the final stage reads directly: one launch per
-// reduction.  The groups depend on the chunk index only (a block holds
-// 256 / B chunks, a multiple of 4), so a column's sums still do not depend
-// on B.  Every thread of the block takes part (there are barriers inside);
-// `put` says whether the thread's column writes.  Large systems write one
-// partial per chunk, part[(kind * nch + chunk) * B + j].
-template <bool GROUPED, int N>
-__device__ __forceinline__ void put_partials(double* __restrict__ part, double* lds,
-                                             int64_t nch, int B, const ChunkIdx& c,
-                                             const int (&kind)[N], const double (&v)[N],
-                                             const bool (&is_max)[N],
-                                             const bool (&put)[N]) {
-  if constexpr (!GROUPED) {
-#pragma unroll
-    for (int n = 0; n < N; n++)
-      if (put[n]) part[(kind[n] * nch + c.chunk) * B + c.j] = v[n];
-    return;
-  }
-  // lds holds N x 256 values; one barrier, the kernel's last use of lds
-  const int t = threadIdx.x;
-#pragma unroll
-  for (int n = 0; n < N; n++) lds[n * 256 + t] = v[n];
-  __syncthreads();
-  if (((t / B) & 3) != 0) return;
-  const int64_t ng4 = (nch + 3) / 4;
-#pragma unroll
-  for (int n = 0; n < N; n++) {
-    if (!put[n]) continue;
-    double a = v[n];
-    for (int k = 1; k < 4 && c.chunk + k < nch; k++) {
-      const double w = lds[n * 256 + t + k * B];
-      a = is_max[n] ? fmax(a, w) : a + w;
-    }
-    part[(kind[n] * ng4 + c.chunk / 4) * B + c.j] = a;
-  }
-}
-
-// p_i = D r + beta p_{i-1} for INNER columns with a pending beta (i the
-// iteration about to run; p_i in buffer i & pmask of the n1 x B buffers),
-// and the chunk partial of max|p_i| for the iteration's stop test
-template <bool GROUPED>
-__global__ __launch_bounds__(256) void k_bpupdate(int64_t n1, int B, int ck,
-                                                  const float* __restrict__ r,
-                                                  const float* __restrict__ dinv,
-                                                  float* __restrict__ p,
-                                                  double* __restrict__ part,
-                                                  const int32_t* __restrict__ cst,
-                                                  const BCol* __restrict__ bc) {
-  __shared__ double lds[GROUPED ? 256 : 1];
-  const ChunkIdx c = chunk_of(n1, B, ck);
-  const bool act = c.valid && cst[c.j] == BCOL_INNER && bc[c.j].pending;
-  double mp = 0.0;
-  if (act) {
-    const float beta = (float)bc[c.j].beta;
-    const int i = bc[c.j].it + 1;
-    const int64_t nv = n1 * B;
-    const int pm = bc[c.j].pmask;
-    const float* __restrict__ pold = p + ((i - 1) & pm) * nv;
-    float* __restrict__ pnew = p + (i & pm) * nv;
-    for (int64_t g = c.g0; g < c.g1; g++) {
-      const int64_t q = g * B + c.j;
-      const float pg = dinv[g] * r[q] + beta * pold[q];
-      pnew[q] = pg;
-      mp = fmax(mp, fabs((double)pg));
-    }
-  }
-  // max|p_i| (INNER kind 2)
-  put_partials<GROUPED, 1>(part, lds, nchunks(n1, ck), B, c, {2}, {mp}, {true}, {act});
-}
-
-// The deferred x updates of a column whose solve ended between two x
-// writes (DONE or FAIL with npend > 0): x += alpha_k p_k for the npend
-// iterations k after the last write, in order; k_bxlag_clear then clears
-// npend once every chunk is done.
-__global__ __launch_bounds__(256) void k_bmaterialize(int64_t n1, int B, int ck,
-                                                      double* __restrict__ x,
-                                                      const float* __restrict__ p,
-                                                      const int32_t* __restrict__ cst,
-                                                      const BCol* __restrict__ bc) {
-  const ChunkIdx c = chunk_of(n1, B, ck);
-  if (!c.valid) return;
-  const int st = cst[c.j];
-  const BCol& bj = bc[c.j];
-  const int np = bj.npend;  // at most 7
-  if ((st != BCOL_DONE && st != BCOL_FAIL) || np == 0) return;
-  const int64_t nv = n1 * B;
-  double al[8];
-  const float* pk[8];
-#pragma unroll
-  for (int k = 0; k < 8; k++) {
-    const int it = bj.it - np + 1 + (k < np ? k : 0);
-    al[k] = bj.alpha_hist[it & 7];
-    pk[k] = p + (it & bj.pmask) * nv;
-  }
-  for (int64_t g = c.g0; g < c.g1; g++) {
-    const int64_t q = g * B + c.j;
-    double xg = 0.0;
-    if (g != 0) {
-      xg = x[q];
-#pragma unroll
-      for (int k = 0; k < 8; k++)
-        if (k < np) xg = xg + al[k] * (double)pk[k][q];
-    }
-    x[q] = xg;
-  }
-}
-
-__global__ void k_bxlag_clear(int B, const int32_t* __restrict__ cst,
-                              BCol* __restrict__ bc) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= B) return;
-  if (cst[j] == BCOL_DONE || cst[j] == BCOL_FAIL) bc[j].npend = 0;
-}
-
-// The update of an iteration, with kp assembled on the fly:
-//   kp[g][j] = sum over the slots of Y (element order, FP32),
-//   r -= alpha kp, z = D r,
-// and the r.z partial (FP64) for INNER columns.  x is written by k_bxfold
-// on the steps that write it; the max|p| partial of the iteration comes from
-// where p was formed (k_bpupdate, or k_bresid for p_1), so the update reads
-// neither x nor p.  The (at most 8 on hexahedral meshes) element
-// contributions of an equation are loaded together, then summed in slot
-// order; UPD_EQ equations per trip keep that many gathers in flight.
-// WAVE_CHUNK: B = 64, so a wave's 64 lanes are the 64 columns of one chunk;
-// the chunk's row pointers and slots are first staged in the wave's LDS rows
-// (stage_indices), so each gather waits on the Y load only, not on a chain
-// of row-pointer and slot loads before it.
-#ifndef UPD_EQ
-#define UPD_EQ 4
-#endif
-#define UPD_SL 512  // staged slots per wave (64 equations, 8 slots each)
-// WAVE_CHUNK: the wave's chunk's row pointers rowptr[ga .. g1] (ga = max(g0,
-// 1): equation 0, the sink, has no update) and its slots, one coalesced load
-// each, into the wave's LDS rows rp[65], sl[UPD_SL], so the update's gathers
-// wait on one memory level instead of three.  All 64 lanes call it; false
-// when the slots do not fit (the update then reads the indices from memory).
-__device__ __forceinline__ bool stage_indices(const ChunkIdx& c,
-                                              const int32_t* __restrict__ rowptr,
-                                              const int32_t* __restrict__ slots,
-                                              int32_t* rp, int32_t* sl) {
-  const int ln = threadIdx.x & 63;
-  const int64_t ga = c.g0 > 0 ? c.g0 : 1;
-  const int nr = (int)(c.g1 - ga) + 1;  // <= 65
-  if (ln < nr) rp[ln] = rowptr[ga + ln];
-  if (ln == 0 && nr > 64) rp[64] = rowptr[ga + 64];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  const int32_t sb = rp[0], nsl = rp[nr - 1] - sb;
-  if (nsl > UPD_SL) return false;
-  for (int k = ln; k < nsl; k += 64) sl[k] = slots[sb + k];
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  return true;
-}
-
-// the body of k_bupdate for one active (chunk, column); rp / sl: the staged
-// indices (null: read them from memory)
-template <bool WAVE_CHUNK, bool STAGED>
-__device__ __forceinline__ void update_chunk(
-    int64_t n1, int B, int ck, const ChunkIdx& c, const int32_t* __restrict__ rowptr,
-    const int32_t* __restrict__ slots, const float* __restrict__ Y,
-    const float* __restrict__ dinv, float* __restrict__ r, const BCol* __restrict__ bc,
-    double& s, const int32_t* rp, const int32_t* sl) {
-  const float alpha32 = (float)bc[c.j].alpha;
-  const int64_t ga = c.g0 > 0 ? c.g0 : 1;
-  const int32_t sb = STAGED ? rp[0] : 0;
-  auto gather = [&](int64_t g, float* v, int32_t& q0, int32_t& q1) {
-    if constexpr (STAGED) {
-      q0 = g > 0 ? rp[g - ga] : 0;
-      q1 = g > 0 ? rp[g - ga + 1] : 0;
-#pragma unroll
-      for (int k = 0; k < 8; k++)
-        v[k] = (q0 + k < q1) ? Y[(int64_t)sl[q0 + k - sb] * B + c.j] : 0.0f;
-      return;
-    }
-    q0 = g > 0 ? rowptr[g] : 0;
-    q1 = g > 0 ? rowptr[g + 1] : 0;
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-      v[k] = (q0 + k < q1) ? Y[(int64_t)slots[q0 + k] * B + c.j] : 0.0f;
-  };
-  auto finish = [&](int64_t g, const float* v, int32_t q0, int32_t q1) {
-    float kp = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 8; k++)
-      if (q0 + k < q1) kp = kp + v[k];
-    for (int32_t q = q0 + 8; q < q1; q++)
-      kp = kp + Y[(int64_t)(STAGED ? sl[q - sb] : slots[q]) * B + c.j];
-    const int64_t q = g * B + c.j;
-    const float rg = r[q] - alpha32 * kp;
-    r[q] = rg;
-    const float zg = dinv[g] * rg;
-    s = s + (double)rg * (double)zg;
-  };
-  int64_t g = c.g0;
-  for (; g + UPD_EQ <= c.g1; g += UPD_EQ) {
-    float v[UPD_EQ][8];
-    int32_t q0[UPD_EQ], q1[UPD_EQ];
-#pragma unroll
-    for (int k = 0; k < UPD_EQ; k++) gather(g + k, v[k], q0[k], q1[k]);
-#pragma unroll
-    for (int k = 0; k < UPD_EQ; k++) finish(g + k, v[k], q0[k], q1[k]);
-  }
-  for (; g < c.g1; g++) {
-    float va[8];
-    int32_t a0, a1;
-    gather(g, va, a0, a1);
-    finish(g, va, a0, a1);
-  }
-}
-
-// one thread per (chunk, column); the r.z partial (kind 1)
-template <bool WAVE_CHUNK, bool GROUPED>
-__global__ __launch_bounds__(256) void k_bupdate(
-    int64_t n1, int B, int ck, const int32_t* __restrict__ rowptr,
-    const int32_t* __restrict__ slots, const float* __restrict__ Y,
-    const float* __restrict__ dinv, float* __restrict__ r, double* __restrict__ part,
-    const int32_t* __restrict__ cst, const BCol* __restrict__ bc) {
-  __shared__ double lds[GROUPED ? 256 : 1];
-  __shared__ int32_t idx[WAVE_CHUNK ? 4 * (65 + UPD_SL) : 1];
-  ChunkIdx c = chunk_of(n1, B, ck);
-  if (WAVE_CHUNK) {
-    const int ch = __builtin_amdgcn_readfirstlane((int)c.chunk);
-    c.chunk = ch;
-    c.g0 = (int64_t)ch * ck;
-    c.g1 = c.g0 + ck < n1 ? c.g0 + ck : n1;
-    c.valid = c.g0 < n1;
-  }
-  const bool act = c.valid && cst[c.j] == BCOL_INNER;
-  const int64_t nch = nchunks(n1, ck);
-  const int32_t* rp = nullptr;
-  const int32_t* sl = nullptr;
-  if constexpr (WAVE_CHUNK) {
-    int32_t* wr = idx + (threadIdx.x >> 6) * (65 + UPD_SL);
-    // c.valid is uniform over the wave (one chunk per wave); skip when no
-    // lane's column iterates
-    if (c.valid && __any(act) && stage_indices(c, rowptr, slots, wr, wr + 65)) {
-      rp = wr;
-      sl = wr + 65;
-    }
-  }
-  double s = 0.0;
-  if (act) {
-    if (rp)
-      update_chunk<WAVE_CHUNK, true>(n1, B, ck, c, rowptr, slots, Y, dinv, r, bc, s, rp, sl);
-    else
-      update_chunk<WAVE_CHUNK, false>(n1, B, ck, c, rowptr, slots, Y, dinv, r, bc, s, rp, sl);
-  }
-  put_partials<GROUPED, 1>(part, lds, nch, B, c, {1}, {s}, {false}, {act});
-}
-
-// The x write of an iteration i with i % xlen == 0 (INNER columns), after
-// the update of i: the npend deferred updates before i and i's own, in
-// order, x += alpha_k p_k for k = i - np + 1 .. i (np = npend + 1 <= 8),
-// and the max|x| partial (kind 0; x(0) = 0) for i's stop test.
-template <bool GROUPED>
-__global__ __launch_bounds__(256) void k_bxfold(int64_t n1, int B, int ck,
-                                                double* __restrict__ x,
-                                                const float* __restrict__ p,
-                                                double* __restrict__ part,
-                                                const int32_t* __restrict__ cst,
-                                                const BCol* __restrict__ bc) {
-  __shared__ double lds[GROUPED ? 256 : 1];
-  const ChunkIdx c = chunk_of(n1, B, ck);
-  bool act = c.valid && cst[c.j] == BCOL_INNER;
-  double mx = 0.0;
-  if (act) {
-    const BCol& bj = bc[c.j];
-    const int i = bj.it + 1;
-    // a column off the x-writing phase writes nothing here; the INNER
-    // finalize reports it
-    act = (i & (bj.xlen - 1)) == 0;
-    const int np = bj.npend + 1;
-    const int64_t nv = n1 * B;
-    double al[8];
-    uint32_t pk[8];  // buffer offsets, pmask n1 B < 2^32
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      const int it = i - np + 1 + (k < np ? k : 0);
-      al[k] = bj.alpha_hist[it & 7];
-      pk[k] = (uint32_t)(it & bj.pmask) * (uint32_t)nv;
-    }
-    for (int64_t g = act ? c.g0 : c.g1; g < c.g1; g++) {
-      const int64_t q = g * B + c.j;
-      double xg = 0.0;
-      if (g != 0) {
-        xg = x[q];
-#pragma unroll
-        for (int k = 0; k < 8; k++)
-          if (k < np) xg = xg + al[k] * (double)p[pk[k] + q];
-      }
-      x[q] = xg;
-      mx = fmax(mx, fabs(xg));
-    }
-  }
-  put_partials<GROUPED, 1>(part, lds, nchunks(n1, ck), B, c, {0}, {mx}, {true}, {act});
-}
-
 // At a residual step: INNER columns due for a replacement become REPLACE
 // (their last iteration left r_{k+1}, rz_prev = r_k.z_k and a pending beta,
 // which the FP64 residual's finalize recomputes), and the columns that need
@@ -797,230 +464,6 @@ __global__ __launch_bounds__(64) void k_bpromote(int B, int32_t* __restrict__ cs
   if (j == 0) rlist[64] = __popcll(m);
 }
 
-// FP64 residual for START / REPLACE columns: r64 = load - sum Y64 (element
-// order, FP64; Y64 holds the residual list's columns at their list places);
-// r = (float) r64; START: p_1 = D r; partials r.(D r) and (START) max|x_0|,
-// and for START the first iteration's max|p_1|
-template <bool GROUPED>
-__global__ __launch_bounds__(256) void k_bresid(
-    int64_t n1, int B, int ck, const int32_t* __restrict__ rowptr,
-    const int32_t* __restrict__ slots, const double* __restrict__ Y64,
-    const double* __restrict__ load, const float* __restrict__ dinv,
-    const double* __restrict__ x, float* __restrict__ r, float* __restrict__ p,
-    double* __restrict__ part, const int32_t* __restrict__ cst,
-    const int32_t* __restrict__ rslot) {
-  __shared__ double lds[GROUPED ? 3 * 256 : 1];
-  const ChunkIdx c = chunk_of(n1, B, ck);
-  const int st = c.valid ? cst[c.j] : BCOL_OFF;
-  const bool act = st == BCOL_START || st == BCOL_REPLACE;
-  const int qs = act ? rslot[c.j] : 0;
-  const int64_t nv = n1 * B;
-  double s = 0.0, mx = 0.0, mp = 0.0;
-  for (int64_t g = act ? c.g0 : c.g1; g < c.g1; g++) {
-    const int64_t q = g * B + c.j;
-    double kx = 0.0;
-    if (g > 0)
-      for (int32_t w = rowptr[g]; w < rowptr[g + 1]; w++)
-        kx = kx + Y64[(int64_t)slots[w] * B + qs];
-    const double r64 = (g == 0) ? 0.0 : load[q] - kx;
-    const float rg = (float)r64;
-    const float zg = dinv[g] * rg;
-    r[q] = rg;
-    if (st == BCOL_START) {  // p_1 = D r (buffer 1); max|x_0|, max|p_1|
-      p[nv + q] = zg;
-      mx = fmax(mx, fabs(x[q]));
-      mp = fmax(mp, fabs((double)zg));
-    }
-    s = s + (double)rg * (double)zg;
-  }
-  const int64_t nch = nchunks(n1, ck);
-  // kind 2 (max|p_1|, START columns) is the INNER reduction's third kind
-  put_partials<GROUPED, 3>(part, lds, nch, B, c, {0, 1, 2}, {s, mx, mp},
-                           {false, true, true}, {act, act, act && st == BCOL_START});
-}
-
-// Reductions of the chunk partials, in a fixed order independent of B.  On
-// large systems stage 1 (k_bgroup, thread per (group, column), column
-// fastest: coalesced) combines groups of G consecutive chunks per column
-// (batch_group: 64, or 16 for ALPHA below 16,384 elements) and stage 2
-// (k_bfinalize, one block per column) combines the groups and advances the
-// column's state machine.  Small systems skip
-// stage 1: their vector kernels already wrote one partial per four chunks
-// (put_partials), and the ALPHA reduction of up to BFIN_DIRECT_ELEMENTS
-// elements reads the per-element shares directly.
-//   RESID: chunks of equations; r.z of the FP64 residual, max|x| (START).
-//   ALPHA: the elements' p.Kp shares from the MFMA product (a "chunk" is an
-//          element).
-//   INNER: chunks of equations; max|x|, r.z, max|p|.
-#define BGROUP_MIN 16
-#define BFIN_KINDS 3
-
-__device__ __forceinline__ int fin_states(int what) {
-  return what == BFIN_RESID ? (BCOL_BIT(BCOL_START) | BCOL_BIT(BCOL_REPLACE))
-                            : BCOL_BIT(BCOL_INNER);
-}
-
-__device__ __forceinline__ int fin_kinds(int what) {
-  return what == BFIN_INNER ? 3 : what == BFIN_RESID ? 2 : 1;
-}
-
-// kind k of `what` combines by max (else by sum)
-__device__ __forceinline__ bool fin_max(int what, int k) {
-  return (what == BFIN_INNER && k != 1) || (what == BFIN_RESID && k == 1);
-}
-
-__global__ __launch_bounds__(256) void k_bgroup(int64_t nch, int B, int G,
-                                                const double* __restrict__ part,
-                                                double* __restrict__ part2,
-                                                const int32_t* __restrict__ cst,
-                                                int what) {
-  const int64_t ng = (nch + G - 1) / G;
-  const int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  if (q >= ng * B) return;
-  const int j = (int)(q % B);
-  const int64_t g = q / B;
-  if (!wanted(cst, j, fin_states(what))) return;
-  const int nk = fin_kinds(what);
-  const int64_t b0 = g * G, b1 = b0 + G < nch ? b0 + G : nch;
-  for (int k = 0; k < nk; k++) {
-    const bool mx = fin_max(what, k);
-    const double* src = part + k * nch * B;
-    double v = 0.0;
-    int64_t b = b0;
-    // sixteen partials loaded together, then combined in chunk order
-    for (; b + 16 <= b1; b += 16) {
-      double a[16];
-#pragma unroll
-      for (int i = 0; i < 16; i++) a[i] = src[(b + i) * B + j];
-#pragma unroll
-      for (int i = 0; i < 16; i++) v = mx ? fmax(v, a[i]) : v + a[i];
-    }
-    for (; b < b1; b++) {
-      const double a = src[b * B + j];
-      v = mx ? fmax(v, a) : v + a;
-    }
-    part2[(k * ng + g) * B + j] = v;
-  }
-}
-
-// `ng` values per column and kind in gp[(kind * ng + b) * B + j]: the
-// group partials of the two-stage form, or the partials written directly
-// by the kernels (grouped small systems; the element shares of ALPHA on
-// small meshes)
-__global__ __launch_bounds__(256) void k_bfinalize(int64_t ng, int B,
-                                                   const double* __restrict__ gp,
-                                                   int32_t* __restrict__ cst,
-                                                   BCol* __restrict__ bc,
-                                                   int what, int xw) {
-  __shared__ double red[BFIN_KINDS * 4];
-  const int j = blockIdx.x;
-  const int st = cst[j];
-  if (!wanted(cst, j, fin_states(what))) return;  // uniform per block
-  const int nk = fin_kinds(what);
-  // every kind in one pass (their loads overlap); per kind, each thread's
-  // values in group order, then a wave tree, then the four waves in order
-  double a[BFIN_KINDS] = {0.0, 0.0, 0.0};
-  for (int64_t b = threadIdx.x; b < ng; b += 256) {
-#pragma unroll
-    for (int k = 0; k < BFIN_KINDS; k++) {
-      if (k < nk) {
-        const double y = gp[(k * ng + b) * B + j];
-        a[k] = fin_max(what, k) ? fmax(a[k], y) : a[k] + y;
-      }
-    }
-  }
-  const int w = threadIdx.x >> 6;
-#pragma unroll
-  for (int k = 0; k < BFIN_KINDS; k++) {
-    if (k < nk) {
-      const double t = fin_max(what, k) ? wave_max(a[k]) : wave_sum(a[k]);
-      if ((threadIdx.x & 63) == 0) red[k * 4 + w] = t;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x != 0) return;
-  double v[BFIN_KINDS] = {0.0, 0.0, 0.0};
-  for (int k = 0; k < nk; k++) {
-    const bool mx = fin_max(what, k);
-#pragma unroll
-    for (int i = 0; i < 4; i++) v[k] = mx ? fmax(v[k], red[k * 4 + i]) : v[k] + red[k * 4 + i];
-  }
-  BCol& c = bc[j];
-  switch (what) {
-    case BFIN_RESID:  // v0 = r.z of the FP64 residual, v1 = max|x| (START)
-      c.nrep += 1;
-      if (st == BCOL_START) {
-        c.rz = v[0];
-        c.rz0 = v[0];
-        c.it = 0;
-        c.pending = 0;
-        c.maxx = v[1];
-        c.xsum = 0.0;
-        c.npend = 0;
-        cst[j] = (v[0] == 0.0) ? BCOL_DONE : BCOL_INNER;  // r = 0: x is exact
-      } else {  // replaces r_{k+1}: beta = r.z (true) / r_k.z_k
-        c.beta = v[0] / c.rz_prev;
-        c.rz = v[0];
-        c.rz0 = v[0];
-        c.pending = 1;
-        cst[j] = BCOL_INNER;
-      }
-      break;
-    case BFIN_ALPHA:  // v0 = p.Kp
-      c.alpha = c.rz / v[0];
-      c.alpha_hist[(c.it + 1) & 7] = c.alpha;
-      c.pending = 0;
-      break;
-    case BFIN_INNER: {  // v0 = max|x| (x written), v1 = r.z, v2 = max|p|
-      c.it += 1;
-      c.maxp = v[2];
-      const double a = fabs(c.alpha) * v[2];
-      const bool xit = (c.it & (c.xlen - 1)) == 0;
-      if (xit != (xw != 0)) {
-        // the step's update and the column disagree on whether x was
-        // written (the engine's step phase and the column's iteration
-        // count went apart): the column ends, and the host reports it
-        c.xerr = 1;
-        cst[j] = BCOL_FAIL;
-        break;
-      }
-      bool stop;
-      if (xit) {
-        // relative update test of src/solver.f90:65 (after the x update)
-        stop = a / v[0] <= c.tol;
-        c.maxx = v[0];
-        c.xsum = 0.0;
-        c.npend = 0;
-      } else {
-        // x_it = x_w + sum of alpha_k p_k over the iterations after the last
-        // write w is not written yet, but max|x_it| >= max|x_w| - xsum with
-        // xsum the sum of |alpha_k| max|p_k|: a <= tol (max|x_w| - xsum)
-        // passes the same test for certain.  Only inside the window of
-        // relative width ~tol xsum / max|x| (~xlen tol^2 near convergence)
-        // where the bound cannot decide does the solve iterate once more
-        // than the test would.
-        c.xsum += a;
-        stop = a <= c.tol * (c.maxx - c.xsum);
-        c.npend += 1;
-      }
-      if (stop) {
-        cst[j] = BCOL_DONE;
-      } else if (c.it >= c.maxiter) {
-        cst[j] = BCOL_FAIL;
-      } else {
-        c.rz_prev = c.rz;
-        // due for an FP64 residual: replaced at the next residual step, by
-        // when the column may have iterated on
-        if (v[1] <= c.inner_tol * c.rz0) c.want_rep = 1;
-        c.beta = v[1] / c.rz;
-        c.rz = v[1];
-        c.pending = 1;
-      }
-      break;
-    }
-  }
-}
-
 // load[g][j] = ext[g] + body[g][j] (load(0)=0) for active columns
 __global__ void k_bload(int64_t n1, int B, const double* __restrict__ ext,
                         const double* __restrict__ body, double* __restrict__ load,
@@ -1032,53 +475,6 @@ __global__ void k_bload(int64_t n1, int B, const double* __restrict__ ext,
     const int j = (int)(q - g * B);
     if (!active[j]) continue;
     load[q] = (g == 0) ? 0.0 : ext[g] + body[q];
-  }
-}
-
-// uerr per column: x(0)=0, partial max|x-oldx| and max|x|, oldx = x
-__global__ __launch_bounds__(256) void k_buerr(int64_t n1, int B, int ck,
-                                               double* __restrict__ x,
-                                               double* __restrict__ oldx,
-                                               double* __restrict__ part,
-                                               const int32_t* __restrict__ active) {
-  const ChunkIdx c = chunk_of(n1, B, ck);
-  if (!c.valid || !active[c.j]) return;
-  double md = 0.0, mx = 0.0;
-  for (int64_t g = c.g0; g < c.g1; g++) {
-    const int64_t q = g * B + c.j;
-    double xg = x[q];
-    if (g == 0) { xg = 0.0; x[q] = 0.0; }
-    md = fmax(md, fabs(xg - oldx[q]));
-    mx = fmax(mx, fabs(xg));
-    oldx[q] = xg;
-  }
-  const int64_t nch = nchunks(n1, ck);
-  part[(0 * nch + c.chunk) * B + c.j] = md;
-  part[(1 * nch + c.chunk) * B + c.j] = mx;
-}
-
-__global__ __launch_bounds__(256) void k_buerr_finalize(
-    int64_t nch, int B, const double* __restrict__ part,
-    PlasticScalars* __restrict__ ps, const int32_t* __restrict__ active,
-    double nl_tol) {
-  __shared__ double red[4];
-  const int j = blockIdx.x;
-  if (!active[j]) return;
-  double vd = 0.0, vx = 0.0;
-#pragma unroll 4
-  for (int64_t b = threadIdx.x; b < nch; b += 256) {
-    vd = fmax(vd, part[(0 * nch + b) * B + j]);
-    vx = fmax(vx, part[(1 * nch + b) * B + j]);
-  }
-  vd = block_max<4>(vd, red);
-  vx = block_max<4>(vx, red);
-  if (threadIdx.x == 0) {
-    const double uerr = vd / vx;
-    ps[j].uerr = uerr;
-    ps[j].xmax = vx;
-    ps[j].nl_isconv = uerr <= nl_tol ? 1 : 0;
-    ps[j].fmax_bits = 0ull;  // fmax = zero (src/slope.F90:286)
-    ps[j].n_plastic = 0;
   }
 }
 
@@ -1133,44 +529,6 @@ static inline unsigned grid_stride(int64_t n) {
   return (unsigned)(b < 65536 ? (b > 0 ? b : 1) : 65536);
 }
 
-// Chunk length of the vector kernels: a function of the equation count
-// only (never of B), so a column's partial sums stay independent of the
-// batch.  Large systems use 64 equations per thread; small ones shorter
-// chunks, so that the launch still has enough waves to hide the latency of
-// each thread's walk.
-static int batch_chunk(int64_t n1) {
-  int ck = 64;
-  while (ck > 4 && n1 / ck < 16384) ck /= 2;
-  return ck;
-}
-
-static inline int64_t nchunks_host(int64_t n1) {
-  const int ck = batch_chunk(n1);
-  return (n1 + ck - 1) / ck;
-}
-
-// stage-1 group size of the reductions (a function of the chunk count only)
-static inline int batch_group(int64_t nch) { return nch < 16384 ? 16 : 64; }
-// small systems: the vector kernels combine groups of four chunks themselves
-static inline bool batch_grouped(int64_t nch) { return batch_group(nch) == BGROUP_MIN; }
-
-int64_t batch_partials(int64_t n1) {
-  const int64_t nch = nchunks_host(n1);
-  // chunk + group partials of every kind
-  return BFIN_KINDS * (nch + (nch + BGROUP_MIN - 1) / BGROUP_MIN);
-}
-
-int64_t batch_element_partials(int32_t nelmt) {
-  return (int64_t)nelmt + ((int64_t)nelmt + BGROUP_MIN - 1) / BGROUP_MIN;
-}
-
-int64_t batch_equation_chunks(int64_t n1) { return nchunks_host(n1); }
-
-static inline unsigned chunk_blocks(int64_t n1, int B) {
-  const int64_t per = 256 / B;  // chunks per block
-  return (unsigned)((nchunks_host(n1) + per - 1) / per);
-}
-
 static inline int bmv_threads(int B) {
   int t = 81 * B;
   if (t > 256) t = 256;
@@ -1215,110 +573,15 @@ void launch_bmv_f64(hipStream_t s, int32_t nelmt, int B, int n_cu, const double*
                      Y, rlist);
 }
 
-void launch_bupdate(hipStream_t s, int64_t n1, int B, const int32_t* rowptr,
-                    const int32_t* slots, const float* Y, const float* dinv, float* r,
-                    double* part, const int32_t* cst, const BCol* bc) {
-  const int ck = batch_chunk(n1);
-  const bool gr = batch_grouped(nchunks_host(n1));
-#define SGEO_UPD(W, G)                                                                  \
-  hipLaunchKernelGGL((k_bupdate<W, G>), dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1, \
-                     B, ck, rowptr, slots, Y, dinv, r, part, cst, bc)
-  if (B == 64) {
-    if (gr) SGEO_UPD(true, true); else SGEO_UPD(true, false);
-  } else {
-    if (gr) SGEO_UPD(false, true); else SGEO_UPD(false, false);
-  }
-#undef SGEO_UPD
-}
-
-void launch_bxfold(hipStream_t s, int64_t n1, int B, double* x, const float* p,
-                   double* part, const int32_t* cst, const BCol* bc) {
-  if (batch_grouped(nchunks_host(n1)))
-    hipLaunchKernelGGL(k_bxfold<true>, dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1, B,
-                       batch_chunk(n1), x, p, part, cst, bc);
-  else
-    hipLaunchKernelGGL(k_bxfold<false>, dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1, B,
-                       batch_chunk(n1), x, p, part, cst, bc);
-}
-
-void launch_bpupdate(hipStream_t s, int64_t n1, int B, const float* r,
-                     const float* dinv, float* p, double* part, const int32_t* cst,
-                     const BCol* bc) {
-  if (batch_grouped(nchunks_host(n1)))
-    hipLaunchKernelGGL(k_bpupdate<true>, dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1, B,
-                       batch_chunk(n1), r, dinv, p, part, cst, bc);
-  else
-    hipLaunchKernelGGL(k_bpupdate<false>, dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1,
-                       B, batch_chunk(n1), r, dinv, p, part, cst, bc);
-}
-
 void launch_bpromote(hipStream_t s, int B, int32_t* cst, BCol* bc, int32_t* rlist,
                      int32_t* rslot) {
   hipLaunchKernelGGL(k_bpromote, dim3(1), dim3(64), 0, s, B, cst, bc, rlist, rslot);
-}
-
-void launch_bresid(hipStream_t s, int64_t n1, int B, const int32_t* rowptr,
-                   const int32_t* slots, const double* Y64, const double* load,
-                   const float* dinv, const double* x, float* r, float* p,
-                   double* part, const int32_t* cst, const int32_t* rslot) {
-  if (batch_grouped(nchunks_host(n1)))
-    hipLaunchKernelGGL(k_bresid<true>, dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1, B,
-                       batch_chunk(n1), rowptr, slots, Y64, load, dinv, x, r, p, part, cst,
-                       rslot);
-  else
-    hipLaunchKernelGGL(k_bresid<false>, dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1, B,
-                       batch_chunk(n1), rowptr, slots, Y64, load, dinv, x, r, p, part, cst,
-                       rslot);
-}
-
-void launch_bmaterialize(hipStream_t s, int64_t n1, int B, double* x, const float* p,
-                         const int32_t* cst, BCol* bc) {
-  hipLaunchKernelGGL(k_bmaterialize, dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1, B,
-                     batch_chunk(n1), x, p, cst, bc);
-  hipLaunchKernelGGL(k_bxlag_clear, dim3((B + 63) / 64), dim3(64), 0, s, B, cst, bc);
-}
-
-#define BFIN_DIRECT_ELEMENTS 4096
-
-// `nch` partials per column and kind in `part` (equation chunks, or elements
-// for ALPHA); the group partials follow them.  Small systems: one launch,
-// the final stage reading what the kernels wrote (groups of four chunks, or
-// for ALPHA the element shares of up to BFIN_DIRECT_ELEMENTS elements).
-// Large ones: the coalesced group stage, then the final stage.
-void launch_bfinalize(hipStream_t s, int64_t nch, int B, double* part,
-                      int32_t* cst, BCol* bc, int what, int xw) {
-  const bool direct = what == BFIN_ALPHA ? nch <= BFIN_DIRECT_ELEMENTS : batch_grouped(nch);
-  if (direct) {
-    const int64_t ng = what == BFIN_ALPHA ? nch : (nch + 3) / 4;
-    hipLaunchKernelGGL(k_bfinalize, dim3(B), dim3(256), 0, s, ng, B, part, cst, bc, what,
-                       xw);
-    return;
-  }
-  const int G = batch_group(nch);
-  const int64_t ng = (nch + G - 1) / G;
-  // group partials after the chunk partials: for the equation-chunk
-  // reductions after all three kinds (RESID runs before k_bpupdate writes
-  // kind 2), for ALPHA after the element shares
-  double* part2 = part + (what == BFIN_ALPHA ? 1 : BFIN_KINDS) * nch * B;
-  hipLaunchKernelGGL(k_bgroup, dim3((unsigned)((ng * B + 255) / 256)), dim3(256), 0,
-                     s, nch, B, G, part, part2, cst, what);
-  hipLaunchKernelGGL(k_bfinalize, dim3(B), dim3(256), 0, s, ng, B, part2, cst, bc, what,
-                     xw);
 }
 
 void launch_bload(hipStream_t s, int64_t n1, int B, const double* ext,
                   const double* body, double* load, const int32_t* active) {
   hipLaunchKernelGGL(k_bload, dim3(grid_stride(n1 * B)), dim3(256), 0, s, n1, B,
                      ext, body, load, active);
-}
-
-void launch_buerr(hipStream_t s, int64_t n1, int B, double* x, double* oldx,
-                  double* part, PlasticScalars* ps, const int32_t* active,
-                  double nl_tol) {
-  hipLaunchKernelGGL(k_buerr, dim3(chunk_blocks(n1, B)), dim3(256), 0, s, n1, B,
-                     batch_chunk(n1), x, oldx, part, active);
-  hipLaunchKernelGGL(k_buerr_finalize, dim3(B), dim3(256), 0, s, nchunks_host(n1),
-                     B, part, ps, active, nl_tol);
 }
 
 void launch_col_io(hipStream_t s, int64_t n1, int B, int j, double* a,

@@ -2157,14 +2157,13 @@ static void batch_step_launches(sgeo_batch* b, bool prof, bool resid, bool xw) {
   hipStream_t s = c->stream;
   const int B = b->B;
   const int64_t n1 = b->n1;
-  const int64_t nch = batch_equation_chunks(n1);
   if (resid) {
     launch_bpromote(s, B, b->d_cst, b->d_bc, b->d_rlist, b->d_rslot);
     launch_bmv_f64(s, m->nelmt, B, c->n_cu, m->d_KP64, m->d_gdof, b->d_x, b->d_Y64,
                    b->d_rlist);
     launch_bresid(s, n1, B, m->d_rowptr, m->d_slots, b->d_Y64, b->d_load, b->d_dinv32,
-                  b->d_x, b->d_r, b->d_p, b->d_part, b->d_cst, b->d_rslot);
-    launch_bfinalize(s, nch, B, b->d_part, b->d_cst, b->d_bc, BFIN_RESID);
+                  b->d_x, b->d_r, b->d_p, b->d_part, b->d_cst, b->d_rslot, b->d_rlist);
+    launch_bfinalize(s, n1, B, b->d_part, b->d_cst, b->d_bc, BFIN_RESID);
   }
   launch_bpupdate(s, n1, B, b->d_r, b->d_dinv32, b->d_p, b->d_part, b->d_cst, b->d_bc);
   if (prof) prof_mark(c);
@@ -2177,7 +2176,7 @@ static void batch_step_launches(sgeo_batch* b, bool prof, bool resid, bool xw) {
   launch_bupdate(s, n1, B, m->d_rowptr, m->d_slots, b->d_Y32, b->d_dinv32, b->d_r,
                  b->d_part, b->d_cst, b->d_bc);
   if (xw) launch_bxfold(s, n1, B, b->d_x, b->d_p, b->d_part, b->d_cst, b->d_bc);
-  launch_bfinalize(s, nch, B, b->d_part, b->d_cst, b->d_bc, BFIN_INNER, xw ? 1 : 0);
+  launch_bfinalize(s, n1, B, b->d_part, b->d_cst, b->d_bc, BFIN_INNER, xw ? 1 : 0);
 }
 
 // `chunk` lockstep CG steps of every running column (FP64 residuals on the

@@ -208,9 +208,8 @@ struct BmvGeom {
   int xcd_split = 1;
 };
 
-int64_t batch_partials(int64_t n1);          // per column, equation-chunk partials
-int64_t batch_element_partials(int32_t nelmt);  // per column, element p.Kp shares
-int64_t batch_equation_chunks(int64_t n1);
+int64_t batch_partials(int64_t n1);          // per column, partials of the equations' groups
+int64_t batch_element_partials(int32_t nelmt);  // per column, p.Kp shares and their groups
 // eorder: the walk over the elements (a permutation of 0 .. nelmt - 1)
 void launch_bmv_mfma_f32(hipStream_t s, int32_t nelmt, int B, int n_cu, BmvGeom geom,
                          const float* KP, const int32_t* gdof, const int32_t* eorder,
@@ -241,9 +240,10 @@ void launch_bpromote(hipStream_t s, int B, int32_t* cst, BCol* bc, int32_t* rlis
 void launch_bresid(hipStream_t s, int64_t n1, int B, const int32_t* rowptr,
                    const int32_t* slots, const double* Y64, const double* load,
                    const float* dinv, const double* x, float* r, float* p,
-                   double* part, const int32_t* cst, const int32_t* rslot);
-// xw (INNER only): this step's update wrote x (checked against each column)
-void launch_bfinalize(hipStream_t s, int64_t nch, int B, double* part,
+                   double* part, const int32_t* cst, const int32_t* rslot,
+                   const int32_t* rlist);
+// n: equations (elements for ALPHA); xw (INNER only): this step's update wrote x (checked against each column)
+void launch_bfinalize(hipStream_t s, int64_t n, int B, double* part,
                       int32_t* cst, BCol* bc, int what, int xw = 0);
 void launch_bload(hipStream_t s, int64_t n1, int B, const double* ext,
                   const double* body, double* load, const int32_t* active);

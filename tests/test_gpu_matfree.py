@@ -141,3 +141,28 @@ def test_batched_solve_from_geometry_and_from_uploaded_matrices(ctx, grid):
     a = _engine_x(ctx, mesh, spec, 4, 0)
     b = _engine_x(ctx, mesh, spec, 4, 0, upload=True)
     assert rel_l2(a, b) < 1e-10
+
+
+# equation counts around the tiles' lengths: fewer than one tile, a tile's
+# edge, several tiles per wave (1, 2, 4 columns) with a ragged end, and above
+# 131,072 equations, where the tiles grow
+@pytest.mark.parametrize("grid", [(1, 1, 1), (2, 2, 2), (5, 3, 2), (9, 7, 11), (21, 16, 18)])
+def test_engine_steps_same_bits_around_tile_edges(ctx, grid):
+    """x after 24 steps (three x writes, FP64 residuals between) has the same
+    bits in engines of 1 to 64 columns, and follows the FP64 iterate of the
+    drop-in: FP32 directions and residuals keep it within 1e-3 of it over
+    so few iterations."""
+    mesh = _mesh(*grid)
+    spec = hex2spec(mesh)
+    xs = [_engine_x(ctx, mesh, spec, ncol, 24, cols=min(ncol, 2)) for ncol in (1, 2, 4, 8, 16, 32, 64)]
+    for x in xs[1:]:
+        assert np.array_equal(x, xs[0])
+    gam, ym, nu, *_ = mesh.material_arrays()
+    dm = DeviceMesh(ctx, spec, len(gam))
+    try:
+        ext, _ = dm.build_stiffness(gam, ym, nu)
+        if spec.neq > 100:
+            u, _, _ = dm.solve(ext, cg_tol=1e-14, cg_maxiter=24)
+            assert rel_l2(xs[0], u) < 1e-3
+    finally:
+        dm.close()
