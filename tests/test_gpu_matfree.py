@@ -166,3 +166,31 @@ def test_engine_steps_same_bits_around_tile_edges(ctx, grid):
             assert rel_l2(xs[0], u) < 1e-3
     finally:
         dm.close()
+
+
+@pytest.mark.parametrize("grid", [(1, 1, 1), (3, 2, 1), (9, 4, 3)])
+def test_stiffness_of_distorted_elements_bits(ctx, grid):
+    """K, its diagonal and the gravity load of strongly distorted elements
+    are the oracle's bits; where a corner is not finite every entry of that
+    element is NaN, as the full sums give it."""
+    import oracle as O
+    mesh = slope_mesh(*grid, materials=SOILS, layer_z=[10.0], jitter=0.25, seed=11)
+    spec = hex2spec(mesh)
+    gam, ym, nu, *_ = mesh.material_arrays()
+    km, _, ext0 = O.stiffness_bodyload(spec, gam, nu, ym)
+    dm = DeviceMesh(ctx, spec, len(gam))
+    try:
+        ext, _ = dm.build_stiffness(gam, ym, nu)
+        assert np.array_equal(dm.download_stiffness(), km)
+        assert np.array_equal(ext, ext0)
+    finally:
+        dm.close()
+    spec.corners = spec.corners.copy()
+    spec.corners[-1, 3, 1] = np.nan
+    dm = DeviceMesh(ctx, spec, len(gam))
+    try:
+        dm.build_stiffness(gam, ym, nu)
+        k = dm.download_stiffness()
+        assert np.isnan(k[-1]).all() and np.array_equal(k[:-1], km[:-1])
+    finally:
+        dm.close()
