@@ -787,9 +787,9 @@ __global__ __launch_bounds__(256) void k_uerr_finalize(
 
 // --------------------------------------------------------------------------
 // inverse map (equation -> element slots) built on the device: the same
-// CSR the host counting sort of sgeo_mesh_create builds (slots of every
-// equation g >= 1 in ascending e*81+i order; the index-0 sink stays empty,
-// no assembly reads it).  Every kernel checks the equation range itself.
+// CSR a stable counting sort on the host builds (slots of every equation
+// g >= 1 in ascending e*81+i order; the index-0 sink stays empty, no assembly
+// reads it).  Every kernel checks the equation range itself.
 // --------------------------------------------------------------------------
 __global__ void k_fill_i32(int64_t n, int32_t* __restrict__ a, int32_t v) {
   for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n;
@@ -812,13 +812,33 @@ __global__ void k_csr_count(int64_t ns, int32_t neq, const int32_t* __restrict__
   }
 }
 
-// in-place inclusive scan of a[0..n) by one block of 1024 threads, 4096
-// entries per round (4 per thread), the running total carried between rounds
-__global__ __launch_bounds__(1024) void k_scan_i32(int64_t n, int32_t* __restrict__ a) {
+// *longest (zero before) = the largest count of cnt[g + 1], 1 <= g < n1
+__global__ __launch_bounds__(SGEO_VEC_THREADS) void k_csr_longest(
+    int64_t n1, const int32_t* __restrict__ cnt, int32_t* __restrict__ longest) {
+  int32_t m = 0;
+  for (int64_t g = 1 + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; g < n1;
+       g += (int64_t)gridDim.x * blockDim.x)
+    m = max(m, cnt[g + 1]);
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) m = max(m, __shfl_xor(m, off, 64));
+  if ((threadIdx.x & 63) == 0) atomicMax(longest, m);
+}
+
+// In-place inclusive scan: each block of 1024 threads scans its SCAN_SEG
+// entries (four per thread) and leaves their total; the totals are scanned by
+// one block (total NULL: rounds of SCAN_SEG, the running sum carried) and
+// k_scan_add adds them to the segments after them.  One block over 1.6 M
+// entries had taken 0.92 ms, a latency-bound round after another; the three
+// launches take 19 us.
+#define SCAN_SEG 4096
+__global__ __launch_bounds__(1024) void k_scan_i32(int64_t n, int32_t* __restrict__ a,
+                                                   int32_t* __restrict__ total) {
   __shared__ int32_t wsum[16];
   const int t = threadIdx.x, lane = t & 63, w = t >> 6;
   int32_t carry = 0;
-  for (int64_t base = 0; base < n; base += 4096) {
+  const int64_t first = (int64_t)blockIdx.x * SCAN_SEG;
+  const int64_t last = total ? min(n, first + SCAN_SEG) : n;
+  for (int64_t base = first; base < last; base += SCAN_SEG) {
     const int64_t i0 = base + (int64_t)t * 4;
     int32_t v[4], s = 0;
 #pragma unroll
@@ -851,6 +871,13 @@ __global__ __launch_bounds__(1024) void k_scan_i32(int64_t n, int32_t* __restric
     carry += wsum[15];
     __syncthreads();  // wsum is rewritten by the next round
   }
+  if (total && t == 0) total[blockIdx.x] = carry;
+}
+
+__global__ __launch_bounds__(SGEO_VEC_THREADS) void k_scan_add(
+    int64_t n, int32_t* __restrict__ a, const int32_t* __restrict__ total) {
+  const int64_t i = SCAN_SEG + blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
+  if (i < n) a[i] += total[i / SCAN_SEG - 1];
 }
 
 // cursor[g] = rowptr[g]; slots[cursor[g]++] = q for every entry of g >= 1
@@ -894,18 +921,34 @@ void launch_set_i32(hipStream_t s, int32_t* a, int32_t v) {
   hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, (int64_t)1, a, v);
 }
 
-// rowptr (n1 + 1 entries) and slots of gdof (ns entries) into caller memory;
-// cursor (n1 entries) is a temporary; *bad (zeroed here) reports entries
-// outside 0..neq
-void launch_csr_build(hipStream_t s, int64_t ns, int32_t neq, const int32_t* gdof,
-                      int32_t* rowptr, int32_t* slots, int32_t* cursor, int32_t* bad) {
+// The two halves of the map in caller memory.  count: rowptr (n1 + 1 entries)
+// of gdof (ns entries); flags[0] (zeroed here) reports entries outside 0..neq,
+// flags[1] the longest row.  fill: slots.  tmp and cursor (n1 entries each) are
+// temporaries.
+// A row is sorted by one thread inserting its entries one after another: for
+// rows as short as a mesh's.
+void launch_csr_count(hipStream_t s, int64_t ns, int32_t neq, const int32_t* gdof,
+                      int32_t* rowptr, int32_t* tmp, int32_t* flags) {
   const int64_t n1 = (int64_t)neq + 1;
   hipLaunchKernelGGL(k_fill_i32, dim3(grid_stride_blocks(n1 + 1)), dim3(SGEO_VEC_THREADS),
                      0, s, n1 + 1, rowptr, 0);
-  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, (int64_t)1, bad, 0);
+  hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, s, (int64_t)2, flags, 0);
   hipLaunchKernelGGL(k_csr_count, dim3(grid_stride_blocks(ns)), dim3(SGEO_VEC_THREADS), 0,
-                     s, ns, neq, gdof, rowptr, bad);
-  hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, n1 + 1, rowptr);
+                     s, ns, neq, gdof, rowptr, flags);
+  hipLaunchKernelGGL(k_csr_longest, dim3(std::min(256u, grid_stride_blocks(n1))),
+                     dim3(SGEO_VEC_THREADS), 0, s, n1, rowptr, flags + 1);
+  const int64_t ne = n1 + 1, nseg = (ne + SCAN_SEG - 1) / SCAN_SEG;  // nseg <= n1
+  hipLaunchKernelGGL(k_scan_i32, dim3((unsigned)nseg), dim3(1024), 0, s, ne, rowptr, tmp);
+  if (nseg > 1) {
+    hipLaunchKernelGGL(k_scan_i32, dim3(1), dim3(1024), 0, s, nseg, tmp, (int32_t*)nullptr);
+    hipLaunchKernelGGL(k_scan_add, dim3(nblk(ne - SCAN_SEG, SGEO_VEC_THREADS)),
+                       dim3(SGEO_VEC_THREADS), 0, s, ne, rowptr, tmp);
+  }
+}
+
+void launch_csr_fill(hipStream_t s, int64_t ns, int32_t neq, const int32_t* gdof,
+                     const int32_t* rowptr, int32_t* slots, int32_t* cursor) {
+  const int64_t n1 = (int64_t)neq + 1;
   hipLaunchKernelGGL(k_copy_i32, dim3(grid_stride_blocks(n1)), dim3(SGEO_VEC_THREADS), 0,
                      s, n1, rowptr, cursor);
   hipLaunchKernelGGL(k_csr_fill, dim3(grid_stride_blocks(ns)), dim3(SGEO_VEC_THREADS), 0,

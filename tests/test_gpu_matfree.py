@@ -168,6 +168,33 @@ def test_engine_steps_same_bits_around_tile_edges(ctx, grid):
         dm.close()
 
 
+def test_inverse_map_rows_beside_the_device_sort(ctx):
+    """K p where an equation gathers 63, 64, 65 or thousands of element
+    entries (rows of up to 64 are sorted on the device, longer ones on the
+    host), and a refused equation number: the sums run over the entries in
+    ascending element order, so they equal the oracle's bit for bit."""
+    import oracle as O
+    rng = np.random.default_rng(9)
+    for nelmt, neq, shared in ((7, 40, 63), (7, 40, 64), (7, 40, 65), (120, 9, 4000)):
+        flat = rng.integers(0, neq, nelmt * 81).astype(np.int32)  # neq itself: shared below
+        flat[rng.permutation(flat.size)[:shared]] = neq
+        gdof = flat.reshape(nelmt, 81)
+        spec = hex2spec(_mesh(nelmt, 1, 1))
+        spec.gdof_elmt, spec.neq = gdof, neq
+        k = rng.normal(size=(nelmt, 81, 81))
+        p = rng.normal(size=neq + 1)
+        p[0] = 0.0
+        dm = DeviceMesh(ctx, spec, 2)
+        try:
+            dm.upload_stiffness(k, np.ones(neq + 1))
+            assert np.array_equal(dm.matvec(p)[1:], O.ebe_matvec(neq, k, gdof, p)[1:])
+        finally:
+            dm.close()
+        gdof[nelmt - 1, 80] = neq + 1
+        with pytest.raises(RuntimeError, match=rf"gdof_elmt\[{nelmt * 81 - 1}\]={neq + 1}"):
+            DeviceMesh(ctx, spec, 2)
+
+
 @pytest.mark.parametrize("grid", [(1, 1, 1), (3, 2, 1), (9, 4, 3)])
 def test_stiffness_of_distorted_elements_bits(ctx, grid):
     """K, its diagonal and the gravity load of strongly distorted elements
