@@ -6,8 +6,9 @@
 // systems, at most 16,384 partial tiles on large ones).  A tile's partial of
 // a column is the sum of eight interleaved accumulators, accumulator i
 // taking the equations 8 s + i of the tile in order of s, combined pairwise
-// (0,1) (2,3) .., then the pairs, then the two halves; four tiles make a
-// group, summed in order, and one partial leaves the block per group.  None
+// (0,1) (2,3) .., then the pairs, then the two halves; four or eight tiles
+// make a group (tile_group), summed in order, and one partial leaves the
+// block per group.  None
 // of it depends on the column count B or on the launch, so a column's bits
 // are the same in any engine, while the lanes are laid out for B: with 64
 // columns a wave walks one equation at a time and keeps the eight
@@ -20,9 +21,8 @@
 // 97 -> 29 and x write 117 -> 44 on 25,344 elements, 8 columns; update 18.9
 // -> 8.0 on 6,300, one column; update 111 -> 102, x write 233 -> 189 on
 // 12,544, 64 columns, where both stream at 4.3 - 4.6 TB/s of the card's 4.8.
-// The groups' partials are few enough for one final launch per reduction;
-// it had been a grouping launch of 9 - 14 us and a final one of 4 - 6, and
-// is 4 - 10 now.
+// The groups' partials are few enough for one final stage per reduction; it
+// had been a grouping launch of 9 - 14 us and a final one of 4 - 6.
 #pragma clang fp contract(off)
 
 #include "sgeo_device.h"
@@ -30,13 +30,14 @@
 
 namespace sgeo {
 
-#define TILE_WAVES 4  // waves per block, tiles per group
-#define TILE_BLOCK (64 * TILE_WAVES)
-template <int B>
+template <int B, int G>  // G tiles per group
 struct Tile {
   static constexpr int NR = 64 / B < 8 ? 64 / B : 8;  // equations side by side per tile
   static constexpr int A = 8 / NR;                    // accumulators per lane
   static constexpr int TPW = 64 / (B * NR);           // tiles per wave
+  static constexpr int W = TPW < G / 4 ? G / TPW : 4;  // waves per block
+  static constexpr int NT = 64 * W;                    // threads per block
+  static constexpr int GPB = W * TPW / G;              // groups per block
 };
 
 // One pass over this wave's tile(s).  f.load(g) reads what equation g of the
@@ -45,19 +46,19 @@ struct Tile {
 // from g.
 // The loads of F::BATCH equations are issued together; g is clamped for them,
 // never for apply.  Every thread of the block calls it.
-template <int B, int NK, class F>
+template <int B, int G, int NK, class F>
 __device__ __forceinline__ void tile_walk(F& f, int64_t n1, int T, bool act,
                                           const int (&kind)[NK], const bool (&is_max)[NK],
                                           const bool (&put)[NK], double* __restrict__ part,
                                           int64_t ng) {
-  using S_ = Tile<B>;
-  constexpr int NR = S_::NR, A = S_::A, TPW = S_::TPW;
+  using S_ = Tile<B, G>;
+  constexpr int NR = S_::NR, A = S_::A, TPW = S_::TPW, W = S_::W;
   constexpr int AB = A < F::BATCH ? A : F::BATCH;  // accumulators and steps of a batch
   constexpr int U = F::BATCH / AB;
-  __shared__ double red[NK][TILE_WAVES * TPW][B];
+  __shared__ double red[NK][W * TPW][B];
   const int t = threadIdx.x, l = t & 63, w = t >> 6;
   const int j = l % B, row = (l / B) % NR, sub = l / (B * NR);
-  const int64_t tile = ((int64_t)blockIdx.x * TILE_WAVES + w) * TPW + sub;
+  const int64_t tile = ((int64_t)blockIdx.x * W + w) * TPW + sub;
   const int64_t g0 = tile * T;
   const bool on = act && g0 < n1;
   double acc[NK][A];
@@ -124,20 +125,215 @@ __device__ __forceinline__ void tile_walk(F& f, int64_t n1, int T, bool act,
     if (row == 0) red[k][w * TPW + sub][j] = acc[k][0];
   }
   __syncthreads();
-  if (t >= TPW * B) return;
+  if (t >= S_::GPB * B) return;
   const int q = t / B;  // group of the block; t % B is this lane's column
-  const int64_t g = (int64_t)blockIdx.x * TPW + q;
+  const int64_t g = (int64_t)blockIdx.x * S_::GPB + q;
   if (g >= ng) return;
 #pragma unroll
   for (int k = 0; k < NK; k++) {
     if (!put[k]) continue;
-    double a = red[k][TILE_WAVES * q][j];
+    double a = red[k][G * q][j];
 #pragma unroll
-    for (int i = 1; i < TILE_WAVES; i++) {
-      const double o = red[k][TILE_WAVES * q + i][j];
+    for (int i = 1; i < G; i++) {
+      const double o = red[k][G * q + i][j];
       a = is_max[k] ? fmax(a, o) : a + o;
     }
     part[(kind[k] * ng + g) * B + j] = a;
+  }
+}
+
+// --------------------------------------------------------------------------
+// The final stage of a reduction combines the groups' partials and advances
+// the columns' state machines.
+//   RESID: r.z of the FP64 residual, max|x| (START).
+//   ALPHA: the elements' p.Kp shares from the product (a "group" is one of
+//          their tiles' groups, or an element below BFIN_DIRECT_ELEMENTS).
+//   INNER: max|x|, r.z, max|p|.
+// Row i of 256 takes the values i, i + 256, ..; the rows are combined by the
+// bits of i from the highest down.  The order depends on the count of values
+// only, wherever the stage runs: in a launch of its own (k_bfinalize), or,
+// where the values are few (BFIN_FUSED), in every block of the kernel that
+// needs its result: ALPHA in the update, INNER in the next step's direction.
+// There each block reads all values, 2 - 3 us, and a step of a small system
+// is three launches instead of five.  Plastic iterations against launches of
+// their own everywhere: sweeps of 8 columns on 384 elements 72 -> 64 ms, one
+// column on 6,300 elements 25.6 -> 24.0 and on 25,344 77.4 -> 73.5, two on
+// 12,544 56.0 -> 53.9.  Above BFIN_FUSED the read costs more than the launch
+// (8 columns on 25,344 elements, 6,300 values per kind: update 29 -> 37 us); a
+// launch reads with a block per column, since few wide blocks cannot draw the
+// values in fast enough (64 columns on 12,544 elements: 22 us by blocks of
+// eight columns, 16 by one).
+// --------------------------------------------------------------------------
+#define BFIN_KINDS 4  // max|x|, r.z, max|p| of the steps on state 0 and state 1
+#define BFIN_ROWS 256
+#define BFIN_FUSED 4096  // values per kind, all columns
+
+__device__ __forceinline__ int fin_states(int what) {
+  return what == BFIN_RESID ? (BCOL_BIT(BCOL_START) | BCOL_BIT(BCOL_REPLACE))
+                            : BCOL_BIT(BCOL_INNER);
+}
+
+// kind k of `what` combines by max (else by sum)
+__device__ __forceinline__ constexpr bool fin_max(int what, int k) {
+  return (what == BFIN_INNER && k != 1) || (what == BFIN_RESID && k == 1);
+}
+
+__device__ __forceinline__ constexpr int fin_kinds(int what) {
+  return what == BFIN_INNER ? 3 : what == BFIN_RESID ? 2 : 1;
+}
+
+// Columns j0 .. j0 + CB - 1 by a block of NT threads: v[k] of column
+// j0 + t % CB in every thread.  Kind k of value b at src[k][b * B + j].
+template <int WHAT, int CB, int NT>
+__device__ __forceinline__ void fin_combine(const double* const (&src)[3], int64_t ng, int B,
+                                            int j0, double (&v)[3]) {
+  constexpr int NK = fin_kinds(WHAT);
+  constexpr int RPT = 256 * CB / NT > 0 ? 256 * CB / NT : 1;  // rows per thread
+  constexpr int H = BFIN_ROWS / RPT;                          // rows after the thread's own
+  static_assert(H % 8 == 0, "eight low rows");
+  __shared__ double top[NK][H][CB], low[NK][8][CB];
+  const int t = threadIdx.x, c = t % CB, row = t / CB;
+  auto op = [](int k, double a, double b) { return fin_max(WHAT, k) ? fmax(a, b) : a + b; };
+  if (row < H) {
+    double a[NK][RPT];
+#pragma unroll
+    for (int k = 0; k < NK; k++)
+#pragma unroll
+      for (int m = 0; m < RPT; m++) a[k][m] = 0.0;
+    constexpr int U = 8 / RPT;  // eight values of a kind in flight
+    const int n = (int)ng;
+    for (int b0 = row; b0 < n; b0 += U * BFIN_ROWS) {
+      double y[NK][U][RPT];
+#pragma unroll
+      for (int k = 0; k < NK; k++)
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int m = 0; m < RPT; m++) {  // past the end: the last value, not used
+            const int b = min(b0 + u * BFIN_ROWS + m * H, n - 1);
+            y[k][u][m] = src[k][b * B + j0 + c];
+          }
+#pragma unroll
+      for (int k = 0; k < NK; k++)
+#pragma unroll
+        for (int u = 0; u < U; u++)
+#pragma unroll
+          for (int m = 0; m < RPT; m++)
+            if (b0 + u * BFIN_ROWS + m * H < n) a[k][m] = op(k, a[k][m], y[k][u][m]);
+    }
+#pragma unroll
+    for (int k = 0; k < NK; k++) {
+#pragma unroll
+      for (int h = RPT / 2; h > 0; h /= 2)
+#pragma unroll
+        for (int m = 0; m < h; m++) a[k][m] = op(k, a[k][m], a[k][m + h]);
+      top[k][row][c] = a[k][0];
+    }
+  }
+  __syncthreads();
+  if (row < 8) {
+    constexpr int N = H / 8;
+#pragma unroll
+    for (int k = 0; k < NK; k++) {
+      double a[N];
+#pragma unroll
+      for (int m = 0; m < N; m++) a[m] = top[k][row + 8 * m][c];
+#pragma unroll
+      for (int h = N / 2; h > 0; h /= 2)
+#pragma unroll
+        for (int m = 0; m < h; m++) a[m] = op(k, a[m], a[m + h]);
+      low[k][row][c] = a[0];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < NK; k++) {
+    double a[8];
+#pragma unroll
+    for (int m = 0; m < 8; m++) a[m] = low[k][m][c];
+#pragma unroll
+    for (int h = 4; h > 0; h /= 2)
+#pragma unroll
+      for (int m = 0; m < h; m++) a[m] = op(k, a[m], a[m + h]);
+    v[k] = a[0];
+  }
+}
+
+// one column's step of its state machine; st: its state
+__device__ __forceinline__ void fin_advance(int what, const double (&v)[3], BCol& c, int32_t& st,
+                                            int xw) {
+  switch (what) {
+    case BFIN_RESID:  // v0 = r.z of the FP64 residual, v1 = max|x| (START)
+      c.nrep += 1;
+      if (st == BCOL_START) {
+        c.rz = v[0];
+        c.rz0 = v[0];
+        c.it = 0;
+        c.pending = 0;
+        c.maxx = v[1];
+        c.xsum = 0.0;
+        c.npend = 0;
+        st = (v[0] == 0.0) ? BCOL_DONE : BCOL_INNER;  // r = 0: x is exact
+      } else {  // replaces r_{k+1}: beta = r.z (true) / r_k.z_k
+        c.beta = v[0] / c.rz_prev;
+        c.rz = v[0];
+        c.rz0 = v[0];
+        c.pending = 1;
+        st = BCOL_INNER;
+      }
+      break;
+    case BFIN_ALPHA:  // v0 = p.Kp
+      c.alpha = c.rz / v[0];
+      c.alpha_hist[(c.it + 1) & 7] = c.alpha;
+      c.pending = 0;
+      break;
+    case BFIN_INNER: {  // v0 = max|x| (x written), v1 = r.z, v2 = max|p|
+      c.it += 1;
+      c.maxp = v[2];
+      const double a = fabs(c.alpha) * v[2];
+      const bool xit = (c.it & (c.xlen - 1)) == 0;
+      if (xit != (xw != 0)) {
+        // the step's update and the column disagree on whether x was
+        // written (the engine's step phase and the column's iteration
+        // count went apart): the column ends, and the host reports it
+        c.xerr = 1;
+        st = BCOL_FAIL;
+        break;
+      }
+      bool stop;
+      if (xit) {
+        // relative update test of src/solver.f90:65 (after the x update)
+        stop = a / v[0] <= c.tol;
+        c.maxx = v[0];
+        c.xsum = 0.0;
+        c.npend = 0;
+      } else {
+        // x_it = x_w + sum of alpha_k p_k over the iterations after the last
+        // write w is not written yet, but max|x_it| >= max|x_w| - xsum with
+        // xsum the sum of |alpha_k| max|p_k|: a <= tol (max|x_w| - xsum)
+        // passes the same test for certain.  Only inside the window of
+        // relative width ~tol xsum / max|x| (~xlen tol^2 near convergence)
+        // where the bound cannot decide does the solve iterate once more
+        // than the test would.
+        c.xsum += a;
+        stop = a <= c.tol * (c.maxx - c.xsum);
+        c.npend += 1;
+      }
+      if (stop) {
+        st = BCOL_DONE;
+      } else if (c.it >= c.maxiter) {
+        st = BCOL_FAIL;
+      } else {
+        c.rz_prev = c.rz;
+        // due for an FP64 residual: replaced at the next residual step, by
+        // when the column may have iterated on
+        if (v[1] <= c.inner_tol * c.rz0) c.want_rep = 1;
+        c.beta = v[1] / c.rz;
+        c.rz = v[1];
+        c.pending = 1;
+      }
+      break;
+    }
   }
 }
 
@@ -165,20 +361,55 @@ struct PUpdate {
   }
 };
 
-template <int B>
-__global__ __launch_bounds__(TILE_BLOCK) void k_bpupdate(int64_t n1, int T, int64_t ng,
-                                                  const float* __restrict__ r,
-                                                  const float* __restrict__ dinv,
-                                                  float* __restrict__ p,
-                                                  double* __restrict__ part,
-                                                  const int32_t* __restrict__ cst,
-                                                  const BCol* __restrict__ bc) {
-  const int j = threadIdx.x % B;
-  const bool act = cst[j] == BCOL_INNER && bc[j].pending;
-  const int i = bc[j].it + 1, pm = bc[j].pmask;
+// FIN: every block first runs the INNER stage of the step before on the state
+// (cst, bc); the first one writes the new state.  slot: where max|p| goes.
+template <int B, int G, bool FIN>
+__global__ __launch_bounds__((Tile<B, G>::NT)) void k_bpupdate(
+    int64_t n1, int T, int64_t ng, const float* __restrict__ r, const float* __restrict__ dinv,
+    float* __restrict__ p, double* part, int slot, const int32_t* __restrict__ cst,
+    const BCol* __restrict__ bc, int32_t* __restrict__ cstn, BCol* __restrict__ bcn, int xw) {
+  const int t = threadIdx.x, j = t % B;
+  bool act = cst[j] == BCOL_INNER;
+  int i, pm;
+  float beta;
+  if constexpr (FIN) {
+    __shared__ float s_beta[B];
+    __shared__ int32_t s_it[B], s_pm[B], s_act[B];
+    double v[3];
+    const double* const src[3] = {part + (xw ? 0 : ng * B), part + ng * B,
+                                  part + (5 - slot) * ng * B};
+    BCol c;
+    int32_t st;
+    if (t < B) {  // in flight beside the values
+      c = bc[t];
+      st = cst[t];
+    }
+    fin_combine<BFIN_INNER, B, Tile<B, G>::NT>(src, ng, B, 0, v);
+    if (t < B) {
+      if (act) fin_advance(BFIN_INNER, v, c, st, xw);
+      s_act[t] = st == BCOL_INNER && c.pending;
+      s_beta[t] = (float)c.beta;
+      s_it[t] = c.it;
+      s_pm[t] = c.pmask;
+      if (blockIdx.x == 0) {
+        bcn[t] = c;
+        cstn[t] = st;
+      }
+    }
+    __syncthreads();
+    act = s_act[j];
+    i = s_it[j] + 1;
+    pm = s_pm[j];
+    beta = s_beta[j];
+  } else {
+    act = act && bc[j].pending;
+    i = bc[j].it + 1;
+    pm = bc[j].pmask;
+    beta = (float)bc[j].beta;
+  }
   const int64_t nv = n1 * B;
-  PUpdate<B> f{r, dinv, p + ((i - 1) & pm) * nv, p + (i & pm) * nv, (float)bc[j].beta, j};
-  tile_walk<B, 1>(f, n1, T, act, {2}, {true}, {act}, part, ng);
+  PUpdate<B> f{r, dinv, p + ((i - 1) & pm) * nv, p + (i & pm) * nv, beta, j};
+  tile_walk<B, G, 1>(f, n1, T, act, {slot}, {true}, {act}, part, ng);
 }
 
 // The update of an iteration, with kp assembled on the fly:
@@ -265,18 +496,36 @@ struct Update {
   }
 };
 
-template <int B>
-__global__ __launch_bounds__(TILE_BLOCK) void k_bupdate(
+// FIN: every block first runs the ALPHA stage on the nfin values of fin; the
+// first one writes alpha to the state, where no block of this launch reads it.
+template <int B, int G, bool FIN>
+__global__ __launch_bounds__((Tile<B, G>::NT)) void k_bupdate(
     int64_t n1, int T, int64_t ng, const int32_t* __restrict__ rowptr,
     const int32_t* __restrict__ slots, const float* __restrict__ Y,
     const float* __restrict__ dinv, float* __restrict__ r, double* __restrict__ part,
-    const int32_t* __restrict__ cst, const BCol* __restrict__ bc) {
-  __shared__ int32_t idx[B >= 8 ? TILE_WAVES * (65 + UPD_SL) : 1];
-  const int j = threadIdx.x % B;
+    const int32_t* __restrict__ cst, BCol* bc, const double* __restrict__ fin, int64_t nfin) {
+  __shared__ int32_t idx[B >= 8 ? Tile<B, G>::W * (65 + UPD_SL) : 1];
+  const int t = threadIdx.x, j = t % B;
   const bool act = cst[j] == BCOL_INNER;
-  int32_t* wr = idx + (B >= 8 ? (threadIdx.x >> 6) * (65 + UPD_SL) : 0);
-  Update<B> f{rowptr, slots, Y, dinv, r, n1, (float)bc[j].alpha, j, wr, wr + 65, 0, false};
-  tile_walk<B, 1>(f, n1, T, act, {1}, {false}, {act}, part, ng);
+  double alpha;
+  if constexpr (FIN) {
+    double v[3];
+    const double* const src[3] = {fin, fin, fin};
+    const double rz = bc[j].rz;
+    const int i = bc[j].it + 1;
+    fin_combine<BFIN_ALPHA, B, Tile<B, G>::NT>(src, nfin, B, 0, v);
+    alpha = rz / v[0];
+    if (blockIdx.x == 0 && t < B && act) {
+      bc[t].alpha = alpha;
+      bc[t].alpha_hist[i & 7] = alpha;
+      bc[t].pending = 0;
+    }
+  } else {
+    alpha = bc[j].alpha;
+  }
+  int32_t* wr = idx + (B >= 8 ? (t >> 6) * (65 + UPD_SL) : 0);
+  Update<B> f{rowptr, slots, Y, dinv, r, n1, (float)alpha, j, wr, wr + 65, 0, false};
+  tile_walk<B, G, 1>(f, n1, T, act, {1}, {false}, {act}, part, ng);
 }
 
 // The x write of an iteration i with i % xlen == 0 (INNER columns), after
@@ -315,8 +564,8 @@ struct XFold {
   }
 };
 
-template <int B>
-__global__ __launch_bounds__(TILE_BLOCK) void k_bxfold(int64_t n1, int T, int64_t ng,
+template <int B, int G>
+__global__ __launch_bounds__((Tile<B, G>::NT)) void k_bxfold(int64_t n1, int T, int64_t ng,
                                                 double* __restrict__ x,
                                                 const float* __restrict__ p,
                                                 double* __restrict__ part,
@@ -339,7 +588,7 @@ __global__ __launch_bounds__(TILE_BLOCK) void k_bxfold(int64_t n1, int T, int64_
     f.al[k] = bj.alpha_hist[it & 7];
     f.pk[k] = (uint32_t)(it & bj.pmask) * (uint32_t)(n1 * B);
   }
-  tile_walk<B, 1>(f, n1, T, act, {0}, {true}, {act}, part, ng);
+  tile_walk<B, G, 1>(f, n1, T, act, {0}, {true}, {act}, part, ng);
 }
 
 // FP64 residual for START / REPLACE columns: r64 = load - sum Y64 (element
@@ -391,8 +640,8 @@ struct Resid {
   }
 };
 
-template <int B>
-__global__ __launch_bounds__(TILE_BLOCK) void k_bresid(
+template <int B, int G>
+__global__ __launch_bounds__((Tile<B, G>::NT)) void k_bresid(
     int64_t n1, int T, int64_t ng, const int32_t* __restrict__ rowptr,
     const int32_t* __restrict__ slots, const double* __restrict__ Y64,
     const double* __restrict__ load, const float* __restrict__ dinv,
@@ -404,7 +653,7 @@ __global__ __launch_bounds__(TILE_BLOCK) void k_bresid(
   const bool act = st == BCOL_START || st == BCOL_REPLACE;
   Resid<B> f{rowptr, slots, Y64, load, x, dinv, r, p + n1 * B, j, act ? rslot[j] : 0,
              st == BCOL_START};
-  tile_walk<B, 3>(f, n1, T, act, {0, 1, 2}, {false, true, true},
+  tile_walk<B, G, 3>(f, n1, T, act, {0, 1, 2}, {false, true, true},
                   {act, act, st == BCOL_START}, part, ng);
 }
 
@@ -433,8 +682,8 @@ struct UErr {
   }
 };
 
-template <int B>
-__global__ __launch_bounds__(TILE_BLOCK) void k_buerr(int64_t n1, int T, int64_t ng,
+template <int B, int G>
+__global__ __launch_bounds__((Tile<B, G>::NT)) void k_buerr(int64_t n1, int T, int64_t ng,
                                                double* __restrict__ x,
                                                double* __restrict__ oldx,
                                                double* __restrict__ part,
@@ -442,7 +691,7 @@ __global__ __launch_bounds__(TILE_BLOCK) void k_buerr(int64_t n1, int T, int64_t
   const int j = threadIdx.x % B;
   const bool act = active[j] != 0;
   UErr<B> f{x, oldx, j};
-  tile_walk<B, 2>(f, n1, T, act, {0, 1}, {true, true}, {act, act}, part, ng);
+  tile_walk<B, G, 2>(f, n1, T, act, {0, 1}, {true, true}, {act, act}, part, ng);
 }
 
 // the elements' p.Kp shares, as "equations" of the same tiles
@@ -457,15 +706,15 @@ struct Shares {
   __device__ __forceinline__ void apply(const double& d, int64_t, double (&v)[1]) { v[0] = d; }
 };
 
-template <int B>
-__global__ __launch_bounds__(TILE_BLOCK) void k_bshares(int64_t n, int T, int64_t ng,
+template <int B, int G>
+__global__ __launch_bounds__((Tile<B, G>::NT)) void k_bshares(int64_t n, int T, int64_t ng,
                                                  const double* __restrict__ edot,
                                                  double* __restrict__ part,
                                                  const int32_t* __restrict__ cst) {
   const int j = threadIdx.x % B;
   const bool act = cst[j] == BCOL_INNER;
   Shares<B> f{edot, j};
-  tile_walk<B, 1>(f, n, T, act, {0}, {false}, {act}, part, ng);
+  tile_walk<B, G, 1>(f, n, T, act, {0}, {false}, {act}, part, ng);
 }
 
 // The deferred x updates of a column whose solve ended between two x
@@ -510,150 +759,29 @@ __global__ void k_bxlag_clear(int B, const int32_t* __restrict__ cst,
   if (cst[j] == BCOL_DONE || cst[j] == BCOL_FAIL) bc[j].npend = 0;
 }
 
-// The final stage combines the groups' partials and advances the columns'
-// state machines.
-//   RESID: r.z of the FP64 residual, max|x| (START).
-//   ALPHA: the elements' p.Kp shares from the product (a "group" is one of
-//          their tiles' groups, or an element below BFIN_DIRECT_ELEMENTS).
-//   INNER: max|x|, r.z, max|p|.
-#define BFIN_KINDS 3
-
-__device__ __forceinline__ int fin_states(int what) {
-  return what == BFIN_RESID ? (BCOL_BIT(BCOL_START) | BCOL_BIT(BCOL_REPLACE))
-                            : BCOL_BIT(BCOL_INNER);
-}
-
-__device__ __forceinline__ int fin_kinds(int what) {
-  return what == BFIN_INNER ? 3 : what == BFIN_RESID ? 2 : 1;
-}
-
-// kind k of `what` combines by max (else by sum)
-__device__ __forceinline__ bool fin_max(int what, int k) {
-  return (what == BFIN_INNER && k != 1) || (what == BFIN_RESID && k == 1);
-}
-
-// `ng` values per column and kind in gp[(kind * ng + b) * B + j]: the groups'
-// partials, or the element shares themselves of ALPHA on small meshes
-// One block per column; each thread takes every 256th value in order, the
-// loads of four and of every kind together, then a wave tree, then the four
-// waves in order.
-__global__ __launch_bounds__(256) void k_bfinalize(int64_t ng, int B,
-                                                   const double* __restrict__ gp,
-                                                   int32_t* __restrict__ cst,
-                                                   BCol* __restrict__ bc,
-                                                   int what, int xw) {
-  __shared__ double red[BFIN_KINDS][4];
+// The stage in a launch of its own; state in (cst, bc), out (cstn, bcn), which
+// may be the same.
+template <int WHAT>
+__global__ __launch_bounds__(256) void k_bfinalize(int64_t ng, int B, const double* s0,
+                                                   const double* s1, const double* s2,
+                                                   const int32_t* cst, const BCol* bc,
+                                                   int32_t* cstn, BCol* bcn, int xw) {
   const int j = blockIdx.x;
-  const int st = cst[j];
-  if (!((fin_states(what) >> st) & 1)) return;  // uniform per block
-  const int nk = fin_kinds(what);
-  double a[BFIN_KINDS] = {0.0, 0.0, 0.0};
-  for (int64_t b0 = threadIdx.x; b0 < ng; b0 += 4 * 256) {
-    double y[BFIN_KINDS][4];
-#pragma unroll
-    for (int k = 0; k < BFIN_KINDS; k++)
-      if (k < nk)
-#pragma unroll
-        for (int i = 0; i < 4; i++) {  // past the end: the last value, not used
-          const int64_t b = b0 + 256 * i < ng ? b0 + 256 * i : ng - 1;
-          y[k][i] = gp[(k * ng + b) * B + j];
-        }
-#pragma unroll
-    for (int k = 0; k < BFIN_KINDS; k++)
-      if (k < nk)
-#pragma unroll
-        for (int i = 0; i < 4; i++)
-          if (b0 + 256 * i < ng) a[k] = fin_max(what, k) ? fmax(a[k], y[k][i]) : a[k] + y[k][i];
+  BCol c;
+  int32_t st = cst[j];
+  const bool act = (fin_states(WHAT) >> st) & 1;  // uniform per block
+  if (threadIdx.x == 0) c = bc[j];
+  double v[3];
+  if (act) {
+    const double* const src[3] = {s0, s1, s2};
+    fin_combine<WHAT, 1, 256>(src, ng, B, j, v);
+  } else if (cst == cstn) {
+    return;
   }
-#pragma unroll
-  for (int k = 0; k < BFIN_KINDS; k++) {
-    if (k < nk) {
-      const double v = fin_max(what, k) ? wave_max(a[k]) : wave_sum(a[k]);
-      if ((threadIdx.x & 63) == 0) red[k][threadIdx.x >> 6] = v;
-    }
-  }
-  __syncthreads();
   if (threadIdx.x != 0) return;
-  double v[BFIN_KINDS] = {0.0, 0.0, 0.0};
-  for (int k = 0; k < nk; k++) {
-    const bool mx = fin_max(what, k);
-#pragma unroll
-    for (int i = 0; i < 4; i++) v[k] = mx ? fmax(v[k], red[k][i]) : v[k] + red[k][i];
-  }
-  BCol& c = bc[j];
-  switch (what) {
-    case BFIN_RESID:  // v0 = r.z of the FP64 residual, v1 = max|x| (START)
-      c.nrep += 1;
-      if (st == BCOL_START) {
-        c.rz = v[0];
-        c.rz0 = v[0];
-        c.it = 0;
-        c.pending = 0;
-        c.maxx = v[1];
-        c.xsum = 0.0;
-        c.npend = 0;
-        cst[j] = (v[0] == 0.0) ? BCOL_DONE : BCOL_INNER;  // r = 0: x is exact
-      } else {  // replaces r_{k+1}: beta = r.z (true) / r_k.z_k
-        c.beta = v[0] / c.rz_prev;
-        c.rz = v[0];
-        c.rz0 = v[0];
-        c.pending = 1;
-        cst[j] = BCOL_INNER;
-      }
-      break;
-    case BFIN_ALPHA:  // v0 = p.Kp
-      c.alpha = c.rz / v[0];
-      c.alpha_hist[(c.it + 1) & 7] = c.alpha;
-      c.pending = 0;
-      break;
-    case BFIN_INNER: {  // v0 = max|x| (x written), v1 = r.z, v2 = max|p|
-      c.it += 1;
-      c.maxp = v[2];
-      const double a = fabs(c.alpha) * v[2];
-      const bool xit = (c.it & (c.xlen - 1)) == 0;
-      if (xit != (xw != 0)) {
-        // the step's update and the column disagree on whether x was
-        // written (the engine's step phase and the column's iteration
-        // count went apart): the column ends, and the host reports it
-        c.xerr = 1;
-        cst[j] = BCOL_FAIL;
-        break;
-      }
-      bool stop;
-      if (xit) {
-        // relative update test of src/solver.f90:65 (after the x update)
-        stop = a / v[0] <= c.tol;
-        c.maxx = v[0];
-        c.xsum = 0.0;
-        c.npend = 0;
-      } else {
-        // x_it = x_w + sum of alpha_k p_k over the iterations after the last
-        // write w is not written yet, but max|x_it| >= max|x_w| - xsum with
-        // xsum the sum of |alpha_k| max|p_k|: a <= tol (max|x_w| - xsum)
-        // passes the same test for certain.  Only inside the window of
-        // relative width ~tol xsum / max|x| (~xlen tol^2 near convergence)
-        // where the bound cannot decide does the solve iterate once more
-        // than the test would.
-        c.xsum += a;
-        stop = a <= c.tol * (c.maxx - c.xsum);
-        c.npend += 1;
-      }
-      if (stop) {
-        cst[j] = BCOL_DONE;
-      } else if (c.it >= c.maxiter) {
-        cst[j] = BCOL_FAIL;
-      } else {
-        c.rz_prev = c.rz;
-        // due for an FP64 residual: replaced at the next residual step, by
-        // when the column may have iterated on
-        if (v[1] <= c.inner_tol * c.rz0) c.want_rep = 1;
-        c.beta = v[1] / c.rz;
-        c.rz = v[1];
-        c.pending = 1;
-      }
-      break;
-    }
-  }
+  if (act) fin_advance(WHAT, v, c, st, xw);
+  bcn[j] = c;
+  cstn[j] = st;
 }
 
 __global__ __launch_bounds__(256) void k_buerr_finalize(
@@ -692,8 +820,15 @@ static int tile_len(int64_t n) {
   return t;
 }
 
+// tiles per group, by the count only too: eight (blocks of eight waves where a
+// wave walks one tile) halve what the final stages read, and cost the large
+// systems' streaming kernels the waves that wait for the last tile.  Plastic
+// iterations, four against eight: 11,800 equations (8 columns) 69.6 / 64.2 ms,
+// 85,000 (8) 31.7 / 31.2, 160,000 (8) 44.9 / 46.2, 322,000 (64) 402 / 424.
+static int tile_group(int64_t n) { return n <= (1 << 17) ? 8 : 4; }
+
 static inline int64_t tile_groups(int64_t n) {
-  const int64_t per = TILE_WAVES * (int64_t)tile_len(n);
+  const int64_t per = tile_group(n) * (int64_t)tile_len(n);
   return (n + per - 1) / per;
 }
 
@@ -712,16 +847,42 @@ int64_t batch_element_partials(int32_t nelmt) { return (int64_t)nelmt + tile_gro
       SGEO_COL(kern, 1, n, __VA_ARGS__)                                                     \
     }                                                                                       \
   } while (0)
+#define SGEO_COLS8(kern, n, ...)                                                            \
+  do {                                                                                      \
+    const int T_ = tile_len(n);                                                             \
+    const int64_t ng_ = tile_groups(n);                                                     \
+    switch (B) {                                                                            \
+      SGEO_COL(kern, 8, n, __VA_ARGS__) SGEO_COL(kern, 4, n, __VA_ARGS__)                   \
+      SGEO_COL(kern, 2, n, __VA_ARGS__) SGEO_COL(kern, 1, n, __VA_ARGS__)                   \
+    }                                                                                       \
+  } while (0)
 #define SGEO_COL(kern, BB, n, ...)                                                          \
   case BB:                                                                                  \
-    hipLaunchKernelGGL(kern<BB>, dim3((unsigned)((ng_ + Tile<BB>::TPW - 1) / Tile<BB>::TPW)), \
-                       dim3(TILE_BLOCK), 0, s, n, T_, ng_, __VA_ARGS__);                    \
+    if (tile_group(n) == 8) SGEO_COLG(kern, BB, 8, n, __VA_ARGS__);                         \
+    else SGEO_COLG(kern, BB, 4, n, __VA_ARGS__);                                            \
     break;
+#define SGEO_COLG(kern, BB, G, n, ...)                                                      \
+  hipLaunchKernelGGL((kern<BB, G>),                                                         \
+                     dim3((unsigned)((ng_ + Tile<BB, G>::GPB - 1) / Tile<BB, G>::GPB)),     \
+                     dim3(Tile<BB, G>::NT), 0, s, n, T_, ng_, __VA_ARGS__)
+
+template <int B, int G>
+static constexpr auto k_bupdate_run = k_bupdate<B, G, false>;
+template <int B, int G>
+static constexpr auto k_bupdate_fin = k_bupdate<B, G, true>;
+template <int B, int G>
+static constexpr auto k_bpupdate_run = k_bpupdate<B, G, false>;
+template <int B, int G>
+static constexpr auto k_bpupdate_fin = k_bpupdate<B, G, true>;
 
 void launch_bupdate(hipStream_t s, int64_t n1, int B, const int32_t* rowptr,
                     const int32_t* slots, const float* Y, const float* dinv, float* r,
-                    double* part, const int32_t* cst, const BCol* bc) {
-  SGEO_COLS(k_bupdate, n1, rowptr, slots, Y, dinv, r, part, cst, bc);
+                    double* part, const int32_t* cst, BCol* bc, const BFinSrc* fin) {
+  if (fin)
+    SGEO_COLS8(k_bupdate_fin, n1, rowptr, slots, Y, dinv, r, part, cst, bc, fin->v, fin->n);
+  else
+    SGEO_COLS(k_bupdate_run, n1, rowptr, slots, Y, dinv, r, part, cst, bc,
+              (const double*)nullptr, (int64_t)0);
 }
 
 void launch_bxfold(hipStream_t s, int64_t n1, int B, double* x, const float* p,
@@ -729,10 +890,20 @@ void launch_bxfold(hipStream_t s, int64_t n1, int B, double* x, const float* p,
   SGEO_COLS(k_bxfold, n1, x, p, part, cst, bc);
 }
 
+// cur: the state (of two) that the step runs on, and where its max|p| goes;
+// fin: the INNER stage of the step before, on the other state, comes first
 void launch_bpupdate(hipStream_t s, int64_t n1, int B, const float* r,
-                     const float* dinv, float* p, double* part, const int32_t* cst,
-                     const BCol* bc) {
-  SGEO_COLS(k_bpupdate, n1, r, dinv, p, part, cst, bc);
+                     const float* dinv, float* p, double* part, int32_t* cst, BCol* bc,
+                     int cur, bool fin, int xw) {
+  int32_t* cn = cst + cur * B;
+  BCol* bn = bc + cur * B;
+  if (fin)
+    SGEO_COLS8(k_bpupdate_fin, n1, r, dinv, p, part, 2 + cur,
+               (const int32_t*)(cst + (cur ^ 1) * B), (const BCol*)(bc + (cur ^ 1) * B), cn, bn,
+               xw);
+  else
+    SGEO_COLS(k_bpupdate_run, n1, r, dinv, p, part, 2 + cur, (const int32_t*)cn,
+              (const BCol*)bn, (int32_t*)nullptr, (BCol*)nullptr, 0);
 }
 
 void launch_bresid(hipStream_t s, int64_t n1, int B, const int32_t* rowptr,
@@ -760,24 +931,45 @@ void launch_buerr(hipStream_t s, int64_t n1, int B, double* x, double* oldx,
 }
 
 // up to here the final stage reads the elements' shares themselves: 16 per
-// thread, less than the launch that would group them
+// row, less than the launch that would group them.  By the element count
+// only: the grouping is part of the order of the sum.
 #define BFIN_DIRECT_ELEMENTS 4096
 
-// RESID and INNER: the groups' partials of n equations in `part`; ALPHA: n
-// element shares, their groups' partials after them
-void launch_bfinalize(hipStream_t s, int64_t n, int B, double* part,
-                      int32_t* cst, BCol* bc, int what, int xw) {
-  int64_t ng = tile_groups(n);
-  if (what == BFIN_ALPHA) {
-    if (n <= BFIN_DIRECT_ELEMENTS) {
-      ng = n;
-    } else {
-      double* groups = part + n * B;
-      SGEO_COLS(k_bshares, n, part, groups, cst);
-      part = groups;
-    }
-  }
-  hipLaunchKernelGGL(k_bfinalize, dim3(B), dim3(256), 0, s, ng, B, part, cst, bc, what, xw);
+BFinSrc launch_bshares(hipStream_t s, int32_t nelmt, int B, double* edot, const int32_t* cst) {
+  if (nelmt <= BFIN_DIRECT_ELEMENTS) return {edot, nelmt};
+  double* groups = edot + (int64_t)nelmt * B;
+  SGEO_COLS(k_bshares, (int64_t)nelmt, (const double*)edot, groups, cst);
+  return {groups, tile_groups(nelmt)};
+}
+
+bool batch_fuse_inner(int64_t n1, int B) { return B <= 8 && tile_groups(n1) * B <= BFIN_FUSED; }
+bool batch_fuse_alpha(const BFinSrc& q, int B) { return B <= 8 && q.n * B <= BFIN_FUSED; }
+
+template <int WHAT>
+static void finalize(hipStream_t s, int64_t ng, int B, const double* s0, const double* s1,
+                     const double* s2, const int32_t* cst, const BCol* bc, int32_t* cstn,
+                     BCol* bcn, int xw) {
+  hipLaunchKernelGGL(k_bfinalize<WHAT>, dim3(B), dim3(256), 0, s, ng, B, s0, s1, s2, cst, bc,
+                     cstn, bcn, xw);
+}
+
+void launch_bfin_resid(hipStream_t s, int64_t n1, int B, const double* part, int32_t* cst,
+                       BCol* bc) {
+  const int64_t ng = tile_groups(n1);
+  finalize<BFIN_RESID>(s, ng, B, part, part + ng * B, part, cst, bc, cst, bc, 0);
+}
+
+void launch_bfin_alpha(hipStream_t s, const BFinSrc& q, int B, int32_t* cst, BCol* bc) {
+  finalize<BFIN_ALPHA>(s, q.n, B, q.v, q.v, q.v, cst, bc, cst, bc, 0);
+}
+
+// from state cur (of two) to state 0; xw: the step's update wrote x (checked
+// against each column)
+void launch_bfin_inner(hipStream_t s, int64_t n1, int B, const double* part, int32_t* cst,
+                       BCol* bc, int cur, int xw) {
+  const int64_t ng = tile_groups(n1), nk = ng * B;
+  finalize<BFIN_INNER>(s, ng, B, part + (xw ? 0 : nk), part + nk, part + (2 + cur) * nk,
+                       cst + cur * B, bc + cur * B, cst, bc, xw);
 }
 
 }  // namespace sgeo

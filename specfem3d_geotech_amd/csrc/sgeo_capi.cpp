@@ -1751,8 +1751,8 @@ extern "C" int sgeo_batch_create(sgeo_mesh* m, int32_t ncol, const double* extlo
   TRY(dalloc(&b->d_flags, (size_t)m->nelmt * 27 * ncol, acc));
   TRY(dalloc(&b->d_mp, (size_t)std::max(1, m->nmat) * ncol, acc));
   TRY(dalloc(&b->d_ps, (size_t)ncol, acc));
-  TRY(dalloc(&b->d_bc, (size_t)ncol, acc));
-  TRY(dalloc(&b->d_cst, (size_t)ncol, acc));
+  TRY(dalloc(&b->d_bc, (size_t)ncol * 2, acc));  // two states (BStep)
+  TRY(dalloc(&b->d_cst, (size_t)ncol * 2, acc));
   TRY(dalloc(&b->d_mask, (size_t)ncol, acc));
   TRY(dalloc(&b->d_islast, (size_t)ncol, acc));
   TRY(dalloc(&b->d_cols, (size_t)ncol, acc));
@@ -1782,10 +1782,10 @@ extern "C" int sgeo_batch_create(sgeo_mesh* m, int32_t ncol, const double* extlo
   HIPCHK(hipMemcpyAsync(b->d_ext, extload, b->n1 * 8, hipMemcpyHostToDevice, s));
   TRY(batch_sync_operator(b));
   HIPCHK(hipMemsetAsync(b->d_mask, 0, ncol * 4, s));
-  HIPCHK(hipMemsetAsync(b->d_cst, 0, ncol * 4, s));
+  HIPCHK(hipMemsetAsync(b->d_cst, 0, 2 * ncol * 4, s));
   HIPCHK(hipMemsetAsync(b->d_rlist, 0, 65 * 4, s));
   HIPCHK(hipMemsetAsync(b->d_rslot, 0, 64 * 4, s));
-  HIPCHK(hipMemsetAsync(b->d_bc, 0, ncol * sizeof(BCol), s));
+  HIPCHK(hipMemsetAsync(b->d_bc, 0, 2 * ncol * sizeof(BCol), s));
   HIPCHK(hipMemsetAsync(b->d_ps, 0, ncol * sizeof(PlasticScalars), s));
   HIPCHK(hipMemsetAsync(b->d_x, 0, nv * 8, s));
   HIPCHK(hipGetLastError());
@@ -1870,16 +1870,15 @@ extern "C" int sgeo_batch_set_geometry(sgeo_batch* b, int32_t blocks_per_cu,
 
 // Y = K P of the iterating columns, and the elements' p.Kp shares: from the
 // geometry on built meshes, else on the stored packed FP32 matrices
-static void batch_product(sgeo_batch* b, BmvGeom g) {
+static void batch_product(sgeo_batch* b, BmvGeom g, const int32_t* cst, const BCol* bc) {
   sgeo_mesh* m = b->mesh;
   const int want = BCOL_BIT(BCOL_INNER);
   if (m->built)
     launch_bmf(m->ctx->stream, m->nelmt, b->B, g, m->d_geo, m->d_gdof,
-               b->d_eorder, b->d_p, b->n1 * b->B, b->d_Y32, b->d_edot, b->d_cst, b->d_bc, want);
+               b->d_eorder, b->d_p, b->n1 * b->B, b->d_Y32, b->d_edot, cst, bc, want);
   else
     launch_bmv_mfma_f32(m->ctx->stream, m->nelmt, b->B, m->ctx->n_cu, g, m->d_KP32, m->d_gdof,
-                        b->d_eorder, b->d_p, b->n1 * b->B, b->d_Y32, b->d_edot, b->d_cst,
-                        b->d_bc, want);
+                        b->d_eorder, b->d_p, b->n1 * b->B, b->d_Y32, b->d_edot, cst, bc, want);
 }
 
 // Launch-geometry autotuner of the product: times `reps` launches of
@@ -1911,7 +1910,7 @@ extern "C" int sgeo_batch_autotune(sgeo_batch* b, int32_t reps, int32_t* blocks_
       g.blocks_per_cu = bpc;
       g.xcd_split = xs;
       auto launch = [&]() {
-        batch_product(b, g);
+        batch_product(b, g, b->d_cst, b->d_bc);
       };
       launch();  // warm-up
       HIPCHK(hipEventRecord(e0, s));
@@ -2177,7 +2176,16 @@ static bool pcg_running(int st) {
 // With `resid` (a residual step), the step first forms the FP64 residual of
 // the columns that start a call or are due for a replacement (a no-op
 // launch when there are none).
-static void batch_step_launches(sgeo_batch* b, bool prof, bool resid, bool xw) {
+// The columns' state is in one of two places (cur); it is in the first before
+// a residual step and at the end of a chunk.  `close`: the step is the last
+// one before either.
+struct BStep {
+  int cur = 0;
+  bool open = false;  // the last step's INNER stage has not run yet
+  int xw = 0;         // whether that step wrote x
+};
+static void batch_step_launches(sgeo_batch* b, bool prof, bool resid, bool xw, bool close,
+                                BStep& st) {
   sgeo_mesh* m = b->mesh;
   sgeo_ctx* c = m->ctx;
   hipStream_t s = c->stream;
@@ -2189,20 +2197,31 @@ static void batch_step_launches(sgeo_batch* b, bool prof, bool resid, bool xw) {
                    b->d_rlist);
     launch_bresid(s, n1, B, m->d_rowptr, m->d_slots, b->d_Y64, b->d_load, b->d_dinv32,
                   b->d_x, b->d_r, b->d_p, b->d_part, b->d_cst, b->d_rslot, b->d_rlist);
-    launch_bfinalize(s, n1, B, b->d_part, b->d_cst, b->d_bc, BFIN_RESID);
+    launch_bfin_resid(s, n1, B, b->d_part, b->d_cst, b->d_bc);
   }
-  launch_bpupdate(s, n1, B, b->d_r, b->d_dinv32, b->d_p, b->d_part, b->d_cst, b->d_bc);
+  if (st.open) st.cur ^= 1;
+  launch_bpupdate(s, n1, B, b->d_r, b->d_dinv32, b->d_p, b->d_part, b->d_cst, b->d_bc, st.cur,
+                  st.open, st.xw);
+  int32_t* cst = b->d_cst + st.cur * B;
+  BCol* bc = b->d_bc + st.cur * B;
   if (prof) prof_mark(c);
   // Y = K P and the elements' p.Kp shares; alpha = r.z / p.Kp
-  batch_product(b, b->geom);
+  batch_product(b, b->geom, cst, bc);
   if (prof) prof_mark(c);
-  launch_bfinalize(s, m->nelmt, B, b->d_edot, b->d_cst, b->d_bc, BFIN_ALPHA);
+  const BFinSrc q = launch_bshares(s, m->nelmt, B, b->d_edot, cst);
+  const bool fuse = batch_fuse_alpha(q, B);
+  if (!fuse) launch_bfin_alpha(s, q, B, cst, bc);
   // kp assembled from Y; r and r.z; on the x-writing steps x and max|x|;
   // the stop test
   launch_bupdate(s, n1, B, m->d_rowptr, m->d_slots, b->d_Y32, b->d_dinv32, b->d_r,
-                 b->d_part, b->d_cst, b->d_bc);
-  if (xw) launch_bxfold(s, n1, B, b->d_x, b->d_p, b->d_part, b->d_cst, b->d_bc);
-  launch_bfinalize(s, n1, B, b->d_part, b->d_cst, b->d_bc, BFIN_INNER, xw ? 1 : 0);
+                 b->d_part, cst, bc, fuse ? &q : nullptr);
+  if (xw) launch_bxfold(s, n1, B, b->d_x, b->d_p, b->d_part, cst, bc);
+  st.open = !close && batch_fuse_inner(n1, B);
+  st.xw = xw ? 1 : 0;
+  if (!st.open) {
+    launch_bfin_inner(s, n1, B, b->d_part, b->d_cst, b->d_bc, st.cur, st.xw);
+    st.cur = 0;
+  }
 }
 
 // `chunk` lockstep CG steps of every running column (FP64 residuals on the
@@ -2222,8 +2241,10 @@ static int batch_steps(sgeo_batch* b, int chunk, bool* any_running) {
   if (b->use_graphs && !c->prof && gi >= 0 && b->gstep % per == 0) {
     if (!b->gexec[gi]) {
       HIPCHK(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+      BStep st;
       for (int it = 0; it < chunk; it++)
-        batch_step_launches(b, false, it % per == 0, (it + 1) % xlen == 0);
+        batch_step_launches(b, false, it % per == 0, (it + 1) % xlen == 0,
+                            it + 1 == chunk || (it + 1) % per == 0, st);
       hipGraph_t g = nullptr;
       const hipError_t ec = hipStreamEndCapture(s, &g);
       if (ec != hipSuccess || !g) return fail(SGEO_EHIP, "graph capture failed");
@@ -2232,9 +2253,11 @@ static int batch_steps(sgeo_batch* b, int chunk, bool* any_running) {
     }
     HIPCHK(hipGraphLaunch(b->gexec[gi], s));
   } else {
+    BStep st;
     for (int it = 0; it < chunk; it++)
       batch_step_launches(b, c->prof, (b->gstep + it) % per == 0,
-                          (b->gstep + it + 1) % xlen == 0);
+                          (b->gstep + it + 1) % xlen == 0,
+                          it + 1 == chunk || (b->gstep + it + 1) % per == 0, st);
   }
   b->gstep += chunk;
   b->stat_steps += chunk;

@@ -210,6 +210,11 @@ struct BmvGeom {
   int xcd_split = 1;
 };
 
+struct BFinSrc {  // values that the ALPHA stage sums: v[b * B + column], b < n
+  const double* v;
+  int64_t n;
+};
+
 int64_t batch_partials(int64_t n1);          // per column, partials of the equations' groups
 int64_t batch_element_partials(int32_t nelmt);  // per column, p.Kp shares and their groups
 // eorder: the walk over the elements (a permutation of 0 .. nelmt - 1)
@@ -229,12 +234,12 @@ void launch_bmv_f64(hipStream_t s, int32_t nelmt, int B, int n_cu, const double*
                     const int32_t* rlist);
 void launch_bupdate(hipStream_t s, int64_t n1, int B, const int32_t* rowptr,
                     const int32_t* slots, const float* Y, const float* dinv, float* r,
-                    double* part, const int32_t* cst, const BCol* bc);
+                    double* part, const int32_t* cst, BCol* bc, const BFinSrc* fin);
 void launch_bxfold(hipStream_t s, int64_t n1, int B, double* x, const float* p,
                    double* part, const int32_t* cst, const BCol* bc);
 void launch_bpupdate(hipStream_t s, int64_t n1, int B, const float* r,
-                     const float* dinv, float* p, double* part, const int32_t* cst,
-                     const BCol* bc);
+                     const float* dinv, float* p, double* part, int32_t* cst, BCol* bc,
+                     int cur, bool fin, int xw);
 void launch_bmaterialize(hipStream_t s, int64_t n1, int B, double* x, const float* p,
                          const int32_t* cst, BCol* bc);
 void launch_bpromote(hipStream_t s, int B, int32_t* cst, BCol* bc, int32_t* rlist,
@@ -244,9 +249,17 @@ void launch_bresid(hipStream_t s, int64_t n1, int B, const int32_t* rowptr,
                    const float* dinv, const double* x, float* r, float* p,
                    double* part, const int32_t* cst, const int32_t* rslot,
                    const int32_t* rlist);
-// n: equations (elements for ALPHA); xw (INNER only): this step's update wrote x (checked against each column)
-void launch_bfinalize(hipStream_t s, int64_t n, int B, double* part,
-                      int32_t* cst, BCol* bc, int what, int xw = 0);
+// the final stages (sgeo_bvec.hip); cst and bc hold two states of B columns
+// each, a step's INNER stage goes from one to the other where it is fused into
+// the next step's direction, and to state 0 where it is not
+BFinSrc launch_bshares(hipStream_t s, int32_t nelmt, int B, double* edot, const int32_t* cst);
+bool batch_fuse_inner(int64_t n1, int B);
+bool batch_fuse_alpha(const BFinSrc& q, int B);
+void launch_bfin_resid(hipStream_t s, int64_t n1, int B, const double* part, int32_t* cst,
+                       BCol* bc);
+void launch_bfin_alpha(hipStream_t s, const BFinSrc& q, int B, int32_t* cst, BCol* bc);
+void launch_bfin_inner(hipStream_t s, int64_t n1, int B, const double* part, int32_t* cst,
+                       BCol* bc, int cur, int xw);
 void launch_bload(hipStream_t s, int64_t n1, int B, const double* ext,
                   const double* body, double* load, const int32_t* active);
 void launch_buerr(hipStream_t s, int64_t n1, int B, double* x, double* oldx,
