@@ -449,75 +449,112 @@ __global__ __launch_bounds__(256) void k_pcg_finalize(
 // blocks of 256, four times as many compute units at work.
 // Measured, us per iteration without the product: 28,969 equations 29
 // before (five kernels, four rows per thread one after another), 12.7 with
-// blocks of 1,024, 10.6 with 256; 3,489,480 equations 141 before, 116 now.
+// blocks of 1,024, 10.6 with 256, 9.5 with the partials of all kinds in
+// flight together; 3,489,480 equations 141 before, 112 now.
 // --------------------------------------------------------------------------
 #define PCG_DIRECT 1024
 #define PCG_BLOCK 1024
 static_assert(PCG_BLOCK == SGEO_VEC_THREADS * SGEO_VEC_ITEMS, "partials of 1,024 equations");
 
-// sum (or max) of v[0..n) over the block in k_pcg_finalize's order; every
-// thread gets it
-template <bool MAX>
-__device__ __forceinline__ double combine(const double* __restrict__ v, int n, double* lds) {
-  if (n == 1) return v[0];
+// v[k] = sum (bit k of MAXES: max) of in[k][0..n) over the block in
+// k_pcg_finalize's order, in every thread.  The kinds' values are in flight
+// together: one after another each cost the latency of values that other XCDs
+// wrote, and two barriers.
+template <int NK, int MAXES>
+__device__ __forceinline__ void combine(const double* const (&in)[NK], int n, double (&v)[NK]) {
+  if (n == 1) {
+#pragma unroll
+    for (int k = 0; k < NK; k++) v[k] = in[k][0];
+    return;
+  }
+  __shared__ double red[NK][4];
   const int t = threadIdx.x;
+  auto op = [](int k, double a, double b) { return (MAXES >> k) & 1 ? fmax(a, b) : a + b; };
   if (t < 256) {
-    double a = 0.0;
-#pragma unroll 4
-    for (int b = t; b < n; b += 256) a = MAX ? fmax(a, v[b]) : a + v[b];
-    a = MAX ? wave_max(a) : wave_sum(a);
-    if ((t & 63) == 0) lds[t >> 6] = a;
+    double a[NK];
+#pragma unroll
+    for (int k = 0; k < NK; k++) a[k] = 0.0;
+    for (int b0 = t; b0 < n; b0 += 4 * 256) {
+      double y[NK][4];
+#pragma unroll
+      for (int k = 0; k < NK; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)  // past the end: the last value, not used
+          y[k][i] = in[k][min(b0 + 256 * i, n - 1)];
+#pragma unroll
+      for (int k = 0; k < NK; k++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+          if (b0 + 256 * i < n) a[k] = op(k, a[k], y[k][i]);
+    }
+#pragma unroll
+    for (int k = 0; k < NK; k++) {
+      a[k] = (MAXES >> k) & 1 ? wave_max(a[k]) : wave_sum(a[k]);
+      if ((t & 63) == 0) red[k][t >> 6] = a[k];
+    }
   }
   __syncthreads();
-  double s = 0.0;
 #pragma unroll
-  for (int i = 0; i < 4; i++) s = MAX ? fmax(s, lds[i]) : s + lds[i];
-  __syncthreads();
-  return s;
+  for (int k = 0; k < NK; k++) {
+    v[k] = 0.0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[k] = op(k, v[k], red[k][i]);
+  }
 }
 
-// partials in[k][0..n) -> out[k], kinds k < 3 (a NULL kind is left out); bit
-// k of `maxes`: a maximum.  One block.
+// partials in[k][0..n) -> out[k]: max|u|, r.z and max|p|, or p.Kp alone (the
+// others NULL).  One block.
 struct Kinds {
   const double* in[3];
-  int maxes;
 };
 __global__ __launch_bounds__(256) void k_pcg_collapse(int n, Kinds kinds,
                                                       double* __restrict__ out,
                                                       const PcgScalars* __restrict__ sc) {
   if (sc->done) return;
-  __shared__ double lds[4];
-#pragma unroll
-  for (int k = 0; k < 3; k++) {
-    if (!kinds.in[k]) continue;
-    const double a = (kinds.maxes >> k) & 1 ? combine<true>(kinds.in[k], n, lds)
-                                            : combine<false>(kinds.in[k], n, lds);
-    if (threadIdx.x == 0) out[k] = a;
+  if (!kinds.in[1]) {  // p.Kp alone
+    double v[1];
+    combine<1, 0>({kinds.in[0]}, n, v);
+    if (threadIdx.x == 0) out[0] = v[0];
+    return;
   }
+  double v[3];
+  combine<3, 5>({kinds.in[0], kinds.in[1], kinds.in[2]}, n, v);
+  if (threadIdx.x < 3) out[threadIdx.x] = v[threadIdx.x];
 }
 
-// a block's partial of one kind from its BS values; lds holds them
-template <int BS, bool MAX>
-__device__ __forceinline__ void block_partial(double v, double* lds, double* red,
-                                              double* __restrict__ part) {
+// the block's partials of NK kinds (bit k of MAXES: a max) from its threads'
+// values
+template <int BS, int NK, int MAXES>
+__device__ __forceinline__ void block_partials(const double (&v)[NK],
+                                               double* const (&part)[NK]) {
+  __shared__ double lds[NK][BS > 256 ? BS : 1], red[NK][4];
   const int t = threadIdx.x;
+  auto op = [](int k, double a, double b) { return (MAXES >> k) & 1 ? fmax(a, b) : a + b; };
   if (BS > 256) {
-    lds[t] = v;
+#pragma unroll
+    for (int k = 0; k < NK; k++) lds[k][t] = v[k];
     __syncthreads();
   }
   if (t < 256) {
-    double a = BS > 256 ? 0.0 : v;
 #pragma unroll
-    for (int k = 0; k < BS / 256 && BS > 256; k++) a = MAX ? fmax(a, lds[t + 256 * k]) : a + lds[t + 256 * k];
-    a = MAX ? wave_max(a) : wave_sum(a);
-    if ((t & 63) == 0) red[t >> 6] = a;
+    for (int k = 0; k < NK; k++) {
+      double a = BS > 256 ? 0.0 : v[k];
+#pragma unroll
+      for (int i = 0; i < BS / 256 && BS > 256; i++) a = op(k, a, lds[k][t + 256 * i]);
+      a = (MAXES >> k) & 1 ? wave_max(a) : wave_sum(a);
+      if ((t & 63) == 0) red[k][t >> 6] = a;
+    }
   }
   __syncthreads();
-  if (t == 0) {
-    double s = 0.0;
+  if (t < NK) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) s = MAX ? fmax(s, red[i]) : s + red[i];
-    part[blockIdx.x] = s;
+    for (int k = 0; k < NK; k++) {
+      if (t != k) continue;
+      double s = 0.0;
+#pragma unroll
+      for (int i = 0; i < 4; i++) s = op(k, s, red[k][i]);
+      part[k][blockIdx.x] = s;
+    }
   }
 }
 
@@ -528,7 +565,6 @@ __global__ __launch_bounds__(BS) void k_pcg_start(
     const double* __restrict__ dinv, double* __restrict__ r, double* __restrict__ p,
     double* __restrict__ part_rz, double* __restrict__ part_p,
     const PcgScalars* __restrict__ sc) {
-  __shared__ double lds[BS > 256 ? BS : 1], red[4];
   const int64_t g = (int64_t)blockIdx.x * BS + threadIdx.x;
   double s = 0.0, m = 0.0;
   if (g < n1) {
@@ -539,8 +575,7 @@ __global__ __launch_bounds__(BS) void k_pcg_start(
     s = rg * zg;
     m = fabs(zg);
   }
-  block_partial<BS, false>(s, lds, red, part_rz);
-  block_partial<BS, true>(m, lds, red, part_p);
+  block_partials<BS, 2, 2>({s, m}, {part_rz, part_p});
 }
 
 // the row's element contributions (at most 8 on hexahedral meshes) loaded
@@ -567,7 +602,6 @@ __global__ __launch_bounds__(BS) void k_pcg_asm(
     const double* __restrict__ Y, const double* __restrict__ p, double* __restrict__ kp,
     double* __restrict__ part, const PcgScalars* __restrict__ sc) {
   if (sc->done) return;
-  __shared__ double lds[BS > 256 ? BS : 1], red[4];
   const int64_t g = (int64_t)blockIdx.x * BS + threadIdx.x;
   double s = 0.0;
   if (g < n1) {
@@ -575,7 +609,7 @@ __global__ __launch_bounds__(BS) void k_pcg_asm(
     kp[g] = v;
     s = p[g] * v;
   }
-  block_partial<BS, false>(s, lds, red, part);
+  block_partials<BS, 1, 0>({s}, {part});
 }
 
 // n_dot partials of p.Kp in `dot`; FUSED: kp is summed from Y here
@@ -587,9 +621,9 @@ __global__ __launch_bounds__(BS) void k_pcg_step(
     double* __restrict__ r, const double* __restrict__ dot, int n_dot,
     double* __restrict__ part_u, double* __restrict__ part_rz, PcgScalars* __restrict__ sc) {
   if (sc->done) return;
-  __shared__ double lds[BS > 256 ? BS : 1], red[4];
   const int64_t g = (int64_t)blockIdx.x * BS + threadIdx.x;
   const bool in = g < n1;
+  const double rz = sc->rz;
   double v = 0.0, ug = 0.0, pg = 0.0, rg = 0.0, dg = 0.0;
   if (in) {  // in flight while the partials are combined
     ug = u[g];
@@ -599,8 +633,10 @@ __global__ __launch_bounds__(BS) void k_pcg_step(
     if (!FUSED) v = kp[g];
     else if (g > 0) v = gather_row8(rowptr, slots, Y, g);
   }
-  const double pkp = combine<false>(dot, n_dot, red);
-  const double alpha = sc->rz / pkp;
+  double c[1];
+  combine<1, 0>({dot}, n_dot, c);
+  const double pkp = c[0];
+  const double alpha = rz / pkp;
   double m = 0.0, s = 0.0;
   if (in) {
     ug = ug + alpha * pg;
@@ -610,8 +646,7 @@ __global__ __launch_bounds__(BS) void k_pcg_step(
     r[g] = rg;
     s = rg * (dg * rg);
   }
-  block_partial<BS, true>(m, lds, red, part_u);
-  block_partial<BS, false>(s, lds, red, part_rz);
+  block_partials<BS, 2, 1>({m, s}, {part_u, part_rz});
   if (blockIdx.x == 0 && threadIdx.x == 0) {  // read by later kernels only
     sc->pkp = pkp;
     sc->alpha = alpha;
@@ -631,7 +666,6 @@ __global__ __launch_bounds__(BS) void k_pcg_dir(
     if (writer) *scn = *sc;
     return;
   }
-  __shared__ double lds[BS > 256 ? BS : 1], red[4];
   const int64_t g = (int64_t)blockIdx.x * BS + threadIdx.x;
   const bool in = g < n1;
   double rg = 0.0, dg = 0.0, pg = 0.0;
@@ -640,16 +674,16 @@ __global__ __launch_bounds__(BS) void k_pcg_dir(
     dg = dinv[g];
     pg = p[g];
   }
-  const double maxu = combine<true>(part_u, n_part, red);
-  const double rz = combine<false>(part_rz, n_part, red);
-  const double maxp = combine<true>(part_p, n_part, red);
-  const int it = sc->iter + 1;
+  PcgScalars n = *sc;
+  double c[3];
+  combine<3, 5>({part_u, part_rz, part_p}, n_part, c);
+  const double maxu = c[0], rz = c[1], maxp = c[2];
+  const int it = n.iter + 1;
   // src/solver.f90:65: the relative update of u
-  const bool conv = fabs(sc->alpha) * maxp / maxu <= sc->tol;
-  const bool fail = !conv && it >= sc->maxiter;
-  const double beta = rz / sc->rz;
+  const bool conv = fabs(n.alpha) * maxp / maxu <= n.tol;
+  const bool fail = !conv && it >= n.maxiter;
+  const double beta = rz / n.rz;
   if (writer) {
-    PcgScalars n = *sc;
     n.iter = it;
     n.maxu = maxu;
     n.maxp = maxp;
@@ -658,7 +692,7 @@ __global__ __launch_bounds__(BS) void k_pcg_dir(
       n.conv_iter = it;
     } else if (fail) {
       n.done = 2;
-      n.conv_iter = sc->maxiter + 1;  // DO-loop variable after exhaustion
+      n.conv_iter = n.maxiter + 1;  // DO-loop variable after exhaustion
     } else {
       n.beta = beta;
       n.rz = rz;
@@ -672,7 +706,7 @@ __global__ __launch_bounds__(BS) void k_pcg_dir(
     p[g] = pg;
     m = fabs(pg);
   }
-  block_partial<BS, true>(m, lds, red, part_pn);
+  block_partials<BS, 1, 1>({m}, {part_pn});
 }
 
 // --------------------------------------------------------------------------
@@ -1133,7 +1167,7 @@ void launch_pcg_iteration(hipStream_t s, int64_t n1, int it, const int32_t* rowp
                        (const double*)p, kp, q.dot, cc);
   if (nd > PCG_DIRECT) {
     hipLaunchKernelGGL(k_pcg_collapse, dim3(1), dim3(256), 0, s, nd,
-                       Kinds{{dot, nullptr, nullptr}, 0}, q.c_dot, cc);
+                       Kinds{{dot, nullptr, nullptr}}, q.c_dot, cc);
     dot = q.c_dot;
     nd = 1;
   }
@@ -1143,7 +1177,7 @@ void launch_pcg_iteration(hipStream_t s, int64_t n1, int it, const int32_t* rowp
   hipLaunchKernelGGL(step, grid, block, 0, s, n1, rowptr, slots, Y, (const double*)kp,
                      (const double*)p, dinv, u, r, dot, nd, q.u, q.rz, cur);
   if (np > PCG_DIRECT) {
-    hipLaunchKernelGGL(k_pcg_collapse, dim3(1), dim3(256), 0, s, np, Kinds{{pu, prz, pp}, 5},
+    hipLaunchKernelGGL(k_pcg_collapse, dim3(1), dim3(256), 0, s, np, Kinds{{pu, prz, pp}},
                        q.c_vec, cc);
     pu = q.c_vec;
     prz = pu + 1;
