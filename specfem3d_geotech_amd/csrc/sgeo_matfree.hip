@@ -111,10 +111,13 @@ __device__ __forceinline__ void point_flux(const T adj[3][3], T lam, T mu, const
 // Blocks are mapped so that each XCD walks a contiguous eighth of the
 // elements: neighbours' gathers meet in that XCD's L2.
 //
-// Measured: 111 us on 144,000 elements against 801 us for the packed
-// matrices (k_ebe_packed_pipe, 4.8 TB/s, at the copy rate), 7.9 against
-// 33 us on 4,921.  The 262 MB it must move take 55 us at that rate; the rest
-// is the LDS traffic (63 values per point) and the latency of the gathers.
+// Measured on 144,000 elements: 109 us (124 with the gathers awaited before
+// the Jacobians were formed) against 801 us for the packed matrices
+// (k_ebe_packed_pipe, 4.8 TB/s, at the copy rate); 33 against 8 us on 4,921.
+// The 262 MB it must move take 55 us at that rate; the rest is the LDS traffic
+// (63 values per point) and, at four waves per SIMD (124 registers), the
+// latency of the gathers.  Five waves per SIMD gain 2.6 % on 144,000 elements
+// and lose 2 % on 4,921; six spill into the time of both (129 us).
 // --------------------------------------------------------------------------
 #define MF_EPB 9
 #define MF_XCD 8
@@ -130,16 +133,18 @@ __global__ __launch_bounds__(256) void k_mf64(
   const int32_t blk = (blockIdx.x % MF_XCD) * per + blockIdx.x / MF_XCD;
   if (blk >= nblk) return;  // uniform per block
   __shared__ double s_u[MF_EPB * 81];
-  __shared__ double s_xc[MF_EPB * 24];
+  __shared__ __align__(16) double s_xc[MF_EPB * 24];
   __shared__ double s_R[MF_EPB][9][27];
   const int t = threadIdx.x;
   const int64_t e0 = (int64_t)blk * MF_EPB;
   const int ne = nelmt - e0 < MF_EPB ? (int)(nelmt - e0) : MF_EPB;
   const int32_t* gd = gdof + e0 * 81;
+  int32_t g[3];
+  double ug[3];
 #pragma unroll
   for (int k = 0; k < 3; k++) {  // 9 * 81 = 729 <= 3 * 256
     const int q = t + 256 * k;
-    if (q < ne * 81) s_u[q] = p[gd[q]];
+    g[k] = q < ne * 81 ? gd[q] : 0;
   }
   if (t < ne * 24) s_xc[t] = corners[e0 * 24 + t];
   const int el = t / 27, i = t - 27 * el;
@@ -148,11 +153,19 @@ __global__ __launch_bounds__(256) void k_mf64(
   double2 lm = {0.0, 0.0};
   if (on) lm = lame[mat_id[e0 + el] - 1];
   __syncthreads();
+  // the gathers are in flight while the Jacobians are formed
+#pragma unroll
+  for (int k = 0; k < 3; k++) ug[k] = p[g[k]];
   auto fma = [](double a, double b, double c) { return __builtin_fma(a, b, c); };
+  double adj[3][3], w = 0.0;
+  if (on) w = gll_weight(i) / adjugate_point(ix, iy, iz, s_xc + el * 24, adj);
+#pragma unroll
+  for (int k = 0; k < 3; k++) {
+    const int q = t + 256 * k;
+    if (q < ne * 81) s_u[q] = ug[k];
+  }
+  __syncthreads();
   if (on) {
-    double adj[3][3];
-    const double det = adjugate_point(ix, iy, iz, s_xc + el * 24, adj);
-    const double w = gll_weight(i) / det;
     const double* u = s_u + el * 81;
     double H[3][3], R[3][3];
     const DRow<double> dx = d_row<double>(ix), dy = d_row<double>(iy), dz = d_row<double>(iz);
