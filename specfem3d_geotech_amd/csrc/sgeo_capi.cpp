@@ -677,7 +677,7 @@ extern "C" int sgeo_mesh_download_stiffness(sgeo_mesh* m, double* k) {
 // the stored matrices
 static void ebe_elem(sgeo_mesh* m, const double* p, double* Y, int skip_mode,
                      bool stored = false, double* part = nullptr,
-                     const PcgScalars* sc = nullptr) {
+                     const PcgScalars* sc = nullptr, int back = 0) {
   hipStream_t s = m->ctx->stream;
   if (!sc) sc = m->ctx->d_sc;
   if (!stored && matrix_free(m)) {
@@ -688,11 +688,11 @@ static void ebe_elem(sgeo_mesh* m, const double* p, double* Y, int skip_mode,
       launch_ebe_packed_f32(s, m->nelmt, m->d_KP32, m->d_gdof, p, Y, part, sc, skip_mode);
     else
       launch_ebe_packed_f64(s, m->nelmt, m->ctx->n_cu, m->d_KP64, m->d_gdof, p, Y, part, sc,
-                            skip_mode);
+                            skip_mode, back);
   } else if (m->kprec == SGEO_K_F32) {
-    launch_ebe_elem_f32k(s, m->nelmt, m->d_K32, m->d_gdof, p, Y, part, sc, skip_mode);
+    launch_ebe_elem_f32k(s, m->nelmt, m->d_K32, m->d_gdof, p, Y, part, sc, skip_mode, back);
   } else {
-    launch_ebe_elem_f64(s, m->nelmt, m->d_K64, m->d_gdof, p, Y, part, sc, skip_mode);
+    launch_ebe_elem_f64(s, m->nelmt, m->d_K64, m->d_gdof, p, Y, part, sc, skip_mode, back);
   }
 }
 
@@ -908,7 +908,8 @@ static int pcg_tree(sgeo_mesh* m, double* d_u, const double* d_f, double tol,
     const int n = std::min<int32_t>(chunk, maxiter - enq);
     for (int it = 0; it < n; it++, enq++) {
       TRY(prof_mark(c));
-      ebe_elem(m, m->d_p, m->d_Y, 1, trial, shares ? q.dot : nullptr, c->d_sc + (enq & 1));
+      ebe_elem(m, m->d_p, m->d_Y, 1, trial, shares ? q.dot : nullptr, c->d_sc + (enq & 1),
+               enq & 1);
       TRY(prof_mark(c));
       launch_pcg_iteration(s, n1, enq, m->d_rowptr, m->d_slots, m->d_Y,
                            shares ? nullptr : m->d_kp, m->d_dinv, d_u, m->d_r, m->d_p, q,

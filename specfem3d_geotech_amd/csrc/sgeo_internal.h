@@ -51,13 +51,13 @@ void launch_stiffness(hipStream_t s, int32_t nelmt, const double* corners,
 void launch_round_f32(hipStream_t s, int64_t n, const double* a, float* b);
 void launch_ebe_elem_f64(hipStream_t s, int32_t nelmt, const double* K,
                          const int32_t* gdof, const double* p, double* Y, double* part,
-                         const PcgScalars* sc, int skip_mode);
+                         const PcgScalars* sc, int skip_mode, int back);
 void launch_ebe_elem_f32k(hipStream_t s, int32_t nelmt, const float* K,
                           const int32_t* gdof, const double* p, double* Y, double* part,
-                          const PcgScalars* sc, int skip_mode);
+                          const PcgScalars* sc, int skip_mode, int back);
 void launch_ebe_packed_f64(hipStream_t s, int32_t nelmt, int n_cu, const double* KP,
                            const int32_t* gdof, const double* p, double* Y, double* part,
-                           const PcgScalars* sc, int skip_mode);
+                           const PcgScalars* sc, int skip_mode, int back);
 void launch_ebe_packed_f32(hipStream_t s, int32_t nelmt, const float* KP,
                            const int32_t* gdof, const double* p, double* Y, double* part,
                            const PcgScalars* sc, int skip_mode);

@@ -33,10 +33,10 @@ static inline unsigned grid_stride_blocks(int64_t n) {
 
 // the block's sum of v (NW waves) into its partial
 template <int NW>
-__device__ __forceinline__ void put_share(double v, double* __restrict__ part) {
+__device__ __forceinline__ void put_share(double v, double* __restrict__ part, int blk) {
   __shared__ double red[NW];
   v = block_sum<NW>(v, red);
-  if (threadIdx.x == 0) part[blockIdx.x] = v;
+  if (threadIdx.x == 0) part[blk] = v;
 }
 
 // --------------------------------------------------------------------------
@@ -49,18 +49,22 @@ __device__ __forceinline__ void put_share(double v, double* __restrict__ part) {
 // into LDS once; row r sums c = 0..80 in order, as matmul(km, p(egdof))
 // (src/solver.f90:57).
 // skip_mode: 0 none, 1 return when sc->done, 2 return when !sc->u_nonzero.
+// back: the elements from the last to the first.  A solve alternates, so that
+// an iteration starts with the matrices that the last one left in the 256 MB
+// MALL (30,030 elements, 1.6 GB: solves of 200 iterations 65.8 -> 64.2 ms).
 // part (may be NULL): the block's share of p.Kp = sum_e p_e . Y_e.
 template <typename KT>
 __global__ __launch_bounds__(256) void k_ebe_elem(
     int32_t nelmt, const KT* __restrict__ K, const int32_t* __restrict__ gdof,
     const double* __restrict__ p, double* __restrict__ Y, double* __restrict__ part,
-    const PcgScalars* __restrict__ sc, int skip_mode) {
+    const PcgScalars* __restrict__ sc, int skip_mode, int back) {
   if (skip_mode == 1 && sc->done) return;
   if (skip_mode == 2 && !sc->u_nonzero) return;
   __shared__ double pe[3][81];
   const int t = threadIdx.x;
   const int el = t / 81, r = t - 81 * el;
-  const int64_t e = (int64_t)blockIdx.x * 3 + el;
+  const int blk = back ? gridDim.x - 1 - blockIdx.x : blockIdx.x;
+  const int64_t e = (int64_t)blk * 3 + el;
   const bool valid = (t < 243) && (e < nelmt);
   if (valid) pe[el][r] = p[gdof[e * 81 + r]];
   __syncthreads();
@@ -74,7 +78,7 @@ __global__ __launch_bounds__(256) void k_ebe_elem(
     Y[e * 81 + r] = a;
     d = a * pl[r];
   }
-  if (part) put_share<4>(d, part);
+  if (part) put_share<4>(d, part, blk);
 }
 
 // --------------------------------------------------------------------------
@@ -123,20 +127,20 @@ __global__ __launch_bounds__(128) void k_ebe_packed(
     Y[e * 81 + r] = a;
     d = a * pe[r];
   }
-  if (part) put_share<2>(d, part);
+  if (part) put_share<2>(d, part, blockIdx.x);
 }
 
 // Persistent, pipelined form of k_ebe_packed<double>: a few 128-thread
 // blocks per CU walk the elements.  While element e is multiplied from LDS,
-// the next element's packed K is in flight into registers (16-byte
-// non-temporal loads) and its gathered p into a register, with gdof read
+// the next element's packed K is in flight into registers (16-byte loads) and
+// its gathered p into a register, with gdof read
 // one element further ahead; both reach LDS after the product, behind the
 // block's barrier.  Row r sums c ascending as k_ebe_packed does: the same
 // bits.
 __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
     int32_t nelmt, const double* __restrict__ KP, const int32_t* __restrict__ gdof,
     const double* __restrict__ p, double* __restrict__ Y, double* __restrict__ part,
-    const PcgScalars* __restrict__ sc, int skip_mode) {
+    const PcgScalars* __restrict__ sc, int skip_mode, int back) {
   if (skip_mode == 1 && sc->done) return;
   if (skip_mode == 2 && !sc->u_nonzero) return;
   typedef double v2d __attribute__((ext_vector_type(2)));
@@ -145,25 +149,31 @@ __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
   __shared__ __align__(16) double u[SGEO_KPACK];
   __shared__ double pe[2][81];
   const int t = threadIdx.x;
-  const int64_t stride = gridDim.x;
-  int64_t e = blockIdx.x;
+  // this block's elements, blockIdx.x and every gridDim.x-th after it, from
+  // the last to the first when `back`
+  int64_t stride = gridDim.x, e = blockIdx.x;
+  if (back) {
+    e = e < nelmt ? e + (nelmt - 1 - e) / stride * stride : -1;
+    stride = -stride;
+  }
+  auto in = [&](int64_t q) { return q >= 0 && q < nelmt; };
   v2d kr[PT];
   int32_t gn = 0;  // gdof of the next element
-  if (e < nelmt) {
+  if (in(e)) {
     const v2d* src = reinterpret_cast<const v2d*>(KP + e * SGEO_KPACK);
 #pragma unroll
     for (int i = 0; i < PT; i++) {
       const int q = t + 128 * i;
-      if (q < NV) kr[i] = __builtin_nontemporal_load(src + q);
+      if (q < NV) kr[i] = src[q];
     }
     if (t < 81) pe[0][t] = p[gdof[e * 81 + t]];
-    if (t < 81 && e + stride < nelmt) gn = gdof[(e + stride) * 81 + t];
+    if (t < 81 && in(e + stride)) gn = gdof[(e + stride) * 81 + t];
   }
   const int r = t;
   const int rbase = r * (r + 1) / 2;
   int cur = 0;
   double share = 0.0;
-  for (; e < nelmt; e += stride) {
+  for (; in(e); e += stride) {
     v2d* dst = reinterpret_cast<v2d*>(u);
 #pragma unroll
     for (int i = 0; i < PT; i++) {
@@ -173,17 +183,17 @@ __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
     __syncthreads();  // K of e and pe[cur] visible
     const int64_t en = e + stride;
     double pn = 0.0;
-    if (en < nelmt) {  // in flight during the product
+    if (in(en)) {  // in flight during the product
       const v2d* src = reinterpret_cast<const v2d*>(KP + en * SGEO_KPACK);
 #pragma unroll
       for (int i = 0; i < PT; i++) {
         const int q = t + 128 * i;
-        if (q < NV) kr[i] = __builtin_nontemporal_load(src + q);
+        if (q < NV) kr[i] = src[q];
       }
       if (t < 81) pn = p[gn];
     }
     int32_t gnn = 0;
-    if (t < 81 && en + stride < nelmt) gnn = gdof[(en + stride) * 81 + t];
+    if (t < 81 && in(en + stride)) gnn = gdof[(en + stride) * 81 + t];
     if (t < 81) {
       const double* pl = pe[cur];
       double a = 0.0;
@@ -200,7 +210,7 @@ __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
     __syncthreads();  // u and pe[cur] free, pe[cur ^ 1] visible
     cur ^= 1;
   }
-  if (part) put_share<2>(share, part);
+  if (part) put_share<2>(share, part, blockIdx.x);
 }
 
 // blocks per CU of the persistent FP64 product (LDS 28 KB per block)
@@ -996,26 +1006,26 @@ void launch_csr_fill(hipStream_t s, int64_t ns, int32_t neq, const int32_t* gdof
 // --------------------------------------------------------------------------
 void launch_ebe_elem_f64(hipStream_t s, int32_t nelmt, const double* K,
                          const int32_t* gdof, const double* p, double* Y, double* part,
-                         const PcgScalars* sc, int skip_mode) {
+                         const PcgScalars* sc, int skip_mode, int back) {
   if (nelmt <= 0) return;
   hipLaunchKernelGGL(k_ebe_elem<double>, dim3(nblk(nelmt, 3)), dim3(256), 0, s,
-                     nelmt, K, gdof, p, Y, part, sc, skip_mode);
+                     nelmt, K, gdof, p, Y, part, sc, skip_mode, back);
 }
 
 void launch_ebe_elem_f32k(hipStream_t s, int32_t nelmt, const float* K,
                           const int32_t* gdof, const double* p, double* Y, double* part,
-                          const PcgScalars* sc, int skip_mode) {
+                          const PcgScalars* sc, int skip_mode, int back) {
   if (nelmt <= 0) return;
   hipLaunchKernelGGL(k_ebe_elem<float>, dim3(nblk(nelmt, 3)), dim3(256), 0, s,
-                     nelmt, K, gdof, p, Y, part, sc, skip_mode);
+                     nelmt, K, gdof, p, Y, part, sc, skip_mode, back);
 }
 
 void launch_ebe_packed_f64(hipStream_t s, int32_t nelmt, int n_cu, const double* KP,
                            const int32_t* gdof, const double* p, double* Y, double* part,
-                           const PcgScalars* sc, int skip_mode) {
+                           const PcgScalars* sc, int skip_mode, int back) {
   if (nelmt <= 0) return;
-  hipLaunchKernelGGL(k_ebe_packed_pipe, dim3((unsigned)ebe_packed_blocks(nelmt, n_cu)), dim3(128), 0, s, nelmt, KP,
-                     gdof, p, Y, part, sc, skip_mode);
+  hipLaunchKernelGGL(k_ebe_packed_pipe, dim3((unsigned)ebe_packed_blocks(nelmt, n_cu)),
+                     dim3(128), 0, s, nelmt, KP, gdof, p, Y, part, sc, skip_mode, back);
 }
 
 void launch_ebe_packed_f32(hipStream_t s, int32_t nelmt, const float* KP,
