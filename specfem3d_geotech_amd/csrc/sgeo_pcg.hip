@@ -92,6 +92,42 @@ __global__ __launch_bounds__(256) void k_ebe_elem(
 // y_r = sum_c K(r,c) p_c, c ascending, with K(r,c) = U(min(r,c), max(r,c)).
 // The reference's K_e is symmetric only to the last bit, so this path
 // agrees with the full-storage product to rounding, not bit for bit.
+
+// Row r of the packed matrix u times pe, c ascending.  The place of K(r,c) is
+// a choice of two bases plus a constant of c; written with the index formula
+// in a loop, its 21 integer operations per entry, not the loads, set the time
+// of the product.  Nine entries are read ahead of the nine being added.
+// Measured: 9,315 elements 57.8 -> 43.9 us per product, 5.7 TB/s, which is
+// what the full-storage product reads at; plastic iterations 145 -> 121 ms.
+template <typename KT>
+__device__ __forceinline__ double packed_row(const KT* u, const double* pe, int r) {
+  int rbase = r * (r + 1) / 2;
+  double a = 0.0;
+  // ties the places read next to the sum so far: formed ahead, and the entries
+  // read ahead, they would take every register
+  auto pin = [&]() { asm volatile("" : "+v"(rbase), "+v"(r), "+v"(a)); };
+  KT k[2][9];
+  double q[2][9];
+  auto fetch = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < 9; i++) {
+      const int c = 9 * b + i, col = c * (c + 1) / 2;
+      const KT* at = u + (c < r ? rbase + (c - col) : r);
+      k[b & 1][i] = at[col];
+      q[b & 1][i] = pe[c];
+    }
+  };
+  fetch(0);
+#pragma unroll
+  for (int b = 0; b < 9; b++) {
+    pin();
+    if (b < 8) fetch(b + 1);
+#pragma unroll
+    for (int i = 0; i < 9; i++) a = a + (double)k[b & 1][i] * q[b & 1][i];
+  }
+  return a;
+}
+
 template <typename KT>
 __global__ __launch_bounds__(128) void k_ebe_packed(
     int32_t nelmt, const KT* __restrict__ KP, const int32_t* __restrict__ gdof,
@@ -117,13 +153,7 @@ __global__ __launch_bounds__(128) void k_ebe_packed(
   double d = 0.0;
   if (t < 81) {
     const int r = t;
-    const int rbase = r * (r + 1) / 2;
-    double a = 0.0;
-#pragma unroll 9
-    for (int c = 0; c < 81; c++) {
-      const int idx = (r <= c) ? (c * (c + 1) / 2 + r) : (rbase + c);
-      a = a + (double)u[idx] * pe[c];
-    }
+    const double a = packed_row(u, pe, r);
     Y[e * 81 + r] = a;
     d = a * pe[r];
   }
@@ -170,7 +200,6 @@ __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
     if (t < 81 && in(e + stride)) gn = gdof[(e + stride) * 81 + t];
   }
   const int r = t;
-  const int rbase = r * (r + 1) / 2;
   int cur = 0;
   double share = 0.0;
   for (; in(e); e += stride) {
@@ -196,12 +225,7 @@ __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
     if (t < 81 && in(en + stride)) gnn = gdof[(en + stride) * 81 + t];
     if (t < 81) {
       const double* pl = pe[cur];
-      double a = 0.0;
-#pragma unroll 9
-      for (int c = 0; c < 81; c++) {
-        const int idx = (r <= c) ? (c * (c + 1) / 2 + r) : (rbase + c);
-        a = a + u[idx] * pl[c];
-      }
+      const double a = packed_row(u, pl, r);
       Y[e * 81 + r] = a;
       share = share + a * pl[r];
       pe[cur ^ 1][t] = pn;
