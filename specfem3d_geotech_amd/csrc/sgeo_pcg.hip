@@ -612,19 +612,24 @@ __global__ __launch_bounds__(BS) void k_pcg_start(
   block_partials<BS, 2, 2>({s, m}, {part_rz, part_p});
 }
 
-// the row's element contributions (at most 8 on hexahedral meshes) loaded
-// together, then summed in slot order
+// The row's element contributions (at most 8 on hexahedral meshes), then
+// summed in slot order.  All eight are loaded, past the row's end its last one
+// again: conditional loads compile to a branch each, and every slot's latency
+// stood before the next one's (solves of 1,152 elements 10.5 -> 9.7 ms, 4,921
+// packed 15.0 -> 14.0, 144,000 packed 30.3 -> 29.0).
 __device__ __forceinline__ double gather_row8(const int32_t* __restrict__ rowptr,
                                               const int32_t* __restrict__ slots,
                                               const double* __restrict__ Y, int64_t g) {
   const int32_t q0 = rowptr[g], q1 = rowptr[g + 1];
+  int32_t at[8];
   double v[8];
 #pragma unroll
-  for (int i = 0; i < 8; i++) v[i] = q0 + i < q1 ? Y[slots[q0 + i]] : 0.0;
+  for (int i = 0; i < 8; i++) at[i] = slots[max(min(q0 + i, q1 - 1), 0)];
+#pragma unroll
+  for (int i = 0; i < 8; i++) v[i] = Y[q1 > q0 ? at[i] : 0];
   double kp = 0.0;
 #pragma unroll
-  for (int i = 0; i < 8; i++)
-    if (q0 + i < q1) kp = kp + v[i];
+  for (int i = 0; i < 8; i++) kp = q0 + i < q1 ? kp + v[i] : kp;
   for (int32_t q = q0 + 8; q < q1; q++) kp = kp + Y[slots[q]];
   return kp;
 }
