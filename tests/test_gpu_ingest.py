@@ -94,3 +94,34 @@ def test_device_numbering_large_mesh(ctx):
     assert dev.neq == 3489480
     assert np.array_equal(dev.g_num, host.g_num)
     assert np.array_equal(dev.gdof_elmt, host.gdof_elmt)
+
+
+def test_large_results_through_pinned_pieces(ctx):
+    """Arrays at and around the size from which a result is filled piece by
+    piece (4 MiB, pieces of 1 MiB): K of 79, 80 and 81 elements (4.1 to 4.3
+    MB) and of 400 is what was uploaded, from one thread and from two at once
+    on the same context."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    from specfem3d_geotech_amd.mesh import slope_mesh
+    from specfem3d_geotech_amd.solver import DeviceMesh
+    from specfem3d_geotech_amd.spec import hex2spec
+    rng = np.random.default_rng(3)
+
+    def loaded(nelmt):
+        spec = hex2spec(slope_mesh(nelmt, 1, 1))
+        dm = DeviceMesh(ctx, spec, 1)
+        k = rng.normal(size=(nelmt, 81, 81))
+        dm.upload_stiffness(k, np.ones(spec.neq + 1))
+        return dm, k
+
+    made = [loaded(n) for n in (79, 80, 81, 400)]
+    try:
+        for dm, k in made:
+            assert np.array_equal(dm.download_stiffness(), k)
+        with ThreadPoolExecutor(2) as pool:
+            for (dm, k), got in zip(made, pool.map(lambda q: q[0].download_stiffness(), made)):
+                assert np.array_equal(got, k)
+    finally:
+        for dm, _ in made:
+            dm.close()
