@@ -221,3 +221,25 @@ def test_stiffness_of_distorted_elements_bits(ctx, grid):
         assert np.isnan(k[-1]).all() and np.array_equal(k[:-1], km[:-1])
     finally:
         dm.close()
+
+
+def test_matrices_buffer_of_a_closed_mesh_serves_the_next(ctx):
+    """Meshes made one after another on one context, each closed before the
+    next: equal, a little smaller (the kept buffer serves it), much smaller
+    and larger (it does not).  Each has the oracle's matrices, and two alive
+    at once do not share a buffer."""
+    import oracle as O
+    alive = []
+    for nelmt in (60, 60, 50, 20, 80, 60):
+        spec = hex2spec(_mesh(nelmt, 1, 1))
+        gam, ym, nu, *_ = _mesh(nelmt, 1, 1).material_arrays()
+        km, _, _ = O.stiffness_bodyload(spec, gam, nu, ym)
+        dm = DeviceMesh(ctx, spec, len(gam))
+        dm.build_stiffness(gam, ym, nu)
+        assert np.array_equal(dm.download_stiffness(), km)
+        alive.append((dm, km))
+        if len(alive) == 2:  # the one before is still what it was
+            old, old_km = alive.pop(0)
+            assert np.array_equal(old.download_stiffness(), old_km)
+            old.close()
+    alive[0][0].close()
