@@ -104,7 +104,7 @@ def parse():
                     help="batched engine: launch every step's kernels one by one "
                          "(kernel-trace profilers record graph replays poorly)")
     ap.add_argument("--geometry", default=None,
-                    help="sweep mode: MFMA product launch geometry 'blocks_per_cu,xcd_split' "
+                    help="sweep mode: launch geometry of the element product 'blocks_per_cu,xcd_split' "
                          "instead of the autotuner's pick (e.g. 3,1)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--residual-period", type=int, default=8,
@@ -150,23 +150,12 @@ def single_trial_pcg(ctx, dm, ext, ym, nu, phi, coh, psi, steps, warm):
     return dt_s, n, ms
 
 
-def measured_traffic(kernel_key):
-    """HBM bytes per launch of a kernel from the committed PMC summary
-    (profiles/traffic.json: FETCH_SIZE and WRITE_SIZE runs scaled by what
-    the counters read for a copy of known size), or None."""
-    try:
-        with open(os.path.join(ROOT, "profiles", "traffic.json")) as fh:
-            return json.load(fh)[kernel_key]["bytes_per_launch"]
-    except (OSError, KeyError, ValueError):
-        return None
-
-
-def roofline(kernel, bytes_per_launch, n, ms, extra=None, traffic=None):
+def roofline(kernel, bytes_per_launch, n, ms, extra=None):
     avg = ms / max(n, 1)
     ach = bytes_per_launch / (avg * 1e-3) / 1e9 if n else 0.0
     out = dict(kernel=kernel, bound="hbm", achieved=round(ach, 1), peak=HBM_PEAK_GBS,
                unit="GB/s", frac=round(ach / HBM_PEAK_GBS, 4), avg_launch_ms=round(avg, 4),
-               launches=n, bytes_per_launch=int(bytes_per_launch), traffic=traffic)
+               launches=n, bytes_per_launch=int(bytes_per_launch), traffic=None)
     if extra:
         out.update(extra)
     return out
@@ -242,7 +231,7 @@ def mode_sweep(a, ctx, wl, mesh, spec, prep_s, copy_gbs):
             bpc, xs = (int(v) for v in a.geometry.split(","))
             eng.set_geometry(bpc, bool(xs))
             tune.update(blocks_per_cu=bpc, xcd_split=xs, fixed=True)
-        log("autotune (MFMA product launch geometry): " + ", ".join(
+        log("autotune (element product launch geometry): " + ", ".join(
             f"{c['blocks_per_cu']}/CU {'xcd' if c['xcd_split'] else 'flat'} {c['ms']:.3f} ms"
             for c in tune["candidates"]))
         def window(nsteps):
@@ -264,7 +253,7 @@ def mode_sweep(a, ctx, wl, mesh, spec, prep_s, copy_gbs):
         ended_in_window = len(done_rows) - ended0
         log(f"  timed: {steps} steps in {dt_s:.3f} s")
         # the roofline window right after: the same steps launched one by one
-        # with HIP events around every MFMA product on the library's stream
+        # with HIP events around every product on the library's stream
         ctx.profile(1)
         dtp_s, sp0, sp1 = window(prof_steps)
         nl, kms = ctx.profile(0)
@@ -277,16 +266,17 @@ def mode_sweep(a, ctx, wl, mesh, spec, prep_s, copy_gbs):
     b_eff = ncg / max(nsteps, 1)  # trials iterating per step
     per_trial_ms = dt_s / max(ncg, 1) * 1e3
     # algorithmic bytes of one element-product launch at the roofline
-    # window's columns: packed FP32 K, gdof, the gathered P, the written Y
-    # and the written FP64 p.Kp share of the iterating columns
+    # window's columns: the points' FP32 geometry (27 of 48 bytes), gdof and
+    # the element's place in the walk, the gathered P, the written Y and the
+    # written FP64 p.Kp share of the iterating columns
     b_prof = (sp1["cg_iterations"] - sp0["cg_iterations"]) / max(
         sp1["batched_steps"] - sp0["batched_steps"], 1)
-    kbytes = E * (3328 * 4 + 81 * 4 + (2 * 81 * 4 + 8) * b_prof)
+    kbytes = E * (27 * 48 + 82 * 4 + (2 * 81 * 4 + 8) * b_prof)
     res = dict(
         metric=METRIC, value=N * ncg / dt_s, unit="DOF-iterations/s", n_gpus=1,
         steps=nsteps, warmup=warm, ms_per_step=dt_s / nsteps * 1e3,
         higher_is_better=True, scaling="weak", vs_baseline=None,
-        dtype="f32 inner CG (MFMA) + f64 dots/x/residual/yield", data=DATA,
+        dtype="f32 inner CG + f64 dots/x/residual/yield", data=DATA,
         config=dict(workload=wl.description + f"; {B} form-A strength realisations "
                     "resident, each column walking its own SRF sweep 1.00:0.05:2.00 in "
                     f"steady state; the window is {nsteps} batched CG steps (each advances "
@@ -294,8 +284,8 @@ def mode_sweep(a, ctx, wl, mesh, spec, prep_s, copy_gbs):
                     "PCG starts and FP64 residuals that fall inside it; "
                     f"{ended_in_window} SRF trials ended in the window",
                     nelmt=E, neq=N, trials=B,
-                    form="batched mixed precision", k_storage="packed f32 (S=3328) + "
-                    "packed f64 for the residual", cg_tol=ctl["cg_tol"], inner_tol=itol,
+                    form="batched mixed precision", k_storage="none in f32 (point geometry, "
+                    "1,296 B per element) + packed f64 for the residual", cg_tol=ctl["cg_tol"], inner_tol=itol,
                     residual_period=a.residual_period,
                     nl_tol=ctl["nl_tol"], nl_maxiter=ctl["nl_maxiter"],
                     batch_hbm_gb=round(nbytes / 1e9, 2), copy_kernel_gbs=round(copy_gbs, 1),
@@ -316,16 +306,12 @@ def mode_sweep(a, ctx, wl, mesh, spec, prep_s, copy_gbs):
         timing=dict(headline="HIP-graph replays of the batched steps (production path), "
                     "wall clock around exactly `steps` steps",
                     roofline=f"{prof_steps} further steps launched one by one with HIP "
-                             "events around every k_bmv_mfma launch on the library's stream",
+                             "events around every element-product launch on the library's stream",
                     roofline_window_ms_per_step=round(dtp_s / max(prof_steps, 1) * 1e3, 4)),
-        roofline=roofline("k_bmv_mfma<4> (v_mfma_f32_16x16x4f32)", kbytes, nl, kms,
-                          dict(bytes_model="E*(3328*4 + 81*4 + (2*81*4 + 8)*b), "
+        roofline=roofline(f"element product from the geometry, {B} columns", kbytes, nl, kms,
+                          dict(bytes_model="E*(27*48 + 82*4 + (2*81*4 + 8)*b), "
                                "b = mean trials iterating per step of the roofline window",
-                               b=round(b_prof, 2),
-                               traffic_source="profiles/batched_step_c1_b64_traffic.md "
-                               "(c1, 64 trials iterating)"),
-                          traffic=measured_traffic("k_bmv_mfma<4>")
-                          if (a.workload == "c1" and B == 64) else None))
+                               b=round(b_prof, 2))))
     return res
 
 
@@ -426,7 +412,7 @@ def mode_analysis(a, ctx, wl, mesh, spec, prep_s, copy_gbs):
                          nl_tot=sum(r["nl_tot"] for r in x.rows.values()))
                     for x in an]
         extra = dict(engine=stats)
-        kname = "k_bmv_mfma"
+        kname = "element product from the geometry"
     else:
         from specfem3d_geotech_amd.slope import slope3d
         kp, kf, red, bk, S = FORMS[form]
@@ -457,7 +443,7 @@ def mode_analysis(a, ctx, wl, mesh, spec, prep_s, copy_gbs):
         metric=METRIC, value=nan * 3600.0 / dt_s, unit="FOS analyses/hour", n_gpus=1,
         steps=nan, warmup=0, ms_per_step=dt_s / nan * 1e3, higher_is_better=True,
         scaling="weak", vs_baseline=None,
-        dtype="f64" if form != "batched" else "f32 inner CG (MFMA) + f64", data=DATA,
+        dtype="f64" if form != "batched" else "f32 inner CG + f64", data=DATA,
         config=dict(workload=wl.description, nelmt=E, neq=N, form=form, mode="analysis",
                     analyses=nan, trials=a.trials if form == "batched" else 1,
                     arrival_rate=a.rate, srf_parallel=a.srf_parallel, defer_nl=a.defer_nl,
@@ -555,7 +541,7 @@ def mode_serve(a):
         metric=METRIC, value=st["analyses_per_hour"], unit="FOS analyses/hour",
         n_gpus=1, steps=len(reqs), warmup=0, ms_per_step=st["wall_s"] / len(reqs) * 1e3,
         higher_is_better=True, scaling="weak", vs_baseline=None,
-        dtype="f32 inner CG (MFMA) + f64 (slopes); f64 (excavations)", data=DATA,
+        dtype="f32 inner CG + f64 (slopes); f64 (excavations)", data=DATA,
         config=dict(workload=f"serving: Poisson {a.rate or 4.0}/s, {len(reqs)} requests, "
                     f"meshes {a.min_elements}-{a.max_elements} elements log-uniform, "
                     f"{kinds.count('slope')} slope sweeps + {kinds.count('excavation')} "

@@ -176,7 +176,10 @@ int sgeo_mesh_upload_stiffness(sgeo_mesh *mesh, const double *storekm,
  * SGEO_K_F32) and format.  Derived storages are built on the device from
  * the canonical FP64 matrices (FP32 by rounding; packed keeps the upper
  * triangle k(r,c), r <= c, which the reference's matrices match to the last
- * bit only).  The full FP64 operator reproduces the reference bit for bit;
+ * bit only).  Linear solves and products with the packed FP64 operator of a
+ * mesh whose stiffness was built here are evaluated from the element corners,
+ * which agrees with the matrices to rounding; plastic iterations and uploaded
+ * matrices use the storage.  The full FP64 operator reproduces the reference bit for bit;
  * the others trade that for fewer bytes per iteration. */
 int sgeo_mesh_set_operator(sgeo_mesh *mesh, int kprec, int kfmt);
 /* Achieved HBM bandwidth of a plain device copy of `bytes` (read + write,
@@ -300,7 +303,8 @@ int sgeo_slope_accumulate_nodal(sgeo_slope *slope, int32_t first);
 /* ---- multi-trial mixed-precision engine ---------------------------------
  * Up to 64 (a power of two) strength-reduction trials on one resident mesh,
  * sharing its elastic stiffness.  Each PCG call of a trial is a Jacobi-PCG
- * whose iteration runs in FP32 (packed FP32 operator on MFMA, FP32 r, p,
+ * whose iteration runs in FP32 (the operator from the points' FP32 geometry,
+ * or the packed FP32 matrices on MFMA where they were uploaded; FP32 r, p,
  * K p) with FP64 dot products and an FP64 solution x.  The FP64 residual
  * f - K x (packed FP64 operator) starts the solve and replaces the FP32
  * recursive residual whenever r.z has dropped by inner_tol since the last
@@ -384,7 +388,7 @@ int sgeo_batch_nl_iters(sgeo_batch *batch, int32_t *nl_iter);
  * HIP-event timing with sgeo_profile always uses separate launches).  The
  * results are the same bits either way. */
 int sgeo_batch_set_graphs(sgeo_batch *batch, int enable);
-/* Launch-geometry autotuner of the MFMA element product (no counterpart in
+/* Launch-geometry autotuner of the element product (no counterpart in
  * the reference, which has no GPU product).  Times `reps` launches of each
  * candidate on this engine's mesh and iterating columns -- blocks per CU
  * 4, 3, 2, 1 with the XCD-aware element split, then 4, 3, 2, 1 with a plain
@@ -417,7 +421,7 @@ int sgeo_batch_set_deferred_x(sgeo_batch *batch, int32_t enable);
  * iterations of all trials (seeded elastic solutions not counted), FP64
  * residuals of all trials, and batched steps (one step = one CG iteration
  * of every running column).  sgeo_profile times the batched element-product
- * launches (k_bmv_mfma) like the single-trial one. */
+ * launches like the single-trial one. */
 int sgeo_batch_stats(sgeo_batch *batch, int64_t *inner_iters,
                      int64_t *outer_iters, int64_t *steps);
 

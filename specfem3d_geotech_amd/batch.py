@@ -95,7 +95,7 @@ class BatchEngine:
         check(L.lib().sgeo_batch_set_graphs(self.h, int(enable)), "sgeo_batch_set_graphs")
 
     def autotune(self, reps: int = 5) -> Dict:
-        """Launch geometry of the MFMA product, timed on this mesh with the
+        """Launch geometry of the element product, timed on this mesh with the
         columns iterating now (at least one must be); keeps the fastest."""
         bpc, xs = C.c_int32(), C.c_int32()
         best = C.c_double()
