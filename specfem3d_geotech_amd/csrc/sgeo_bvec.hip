@@ -183,10 +183,12 @@ __device__ __forceinline__ constexpr int fin_kinds(int what) {
 }
 
 // Columns j0 .. j0 + CB - 1 by a block of NT threads: v[k] of column
-// j0 + t % CB in every thread.  Kind k of value b at src[k][b * B + j].
+// j0 + t % CB in every thread.  Kind k of value b at src[k][b * B + j]; kinds
+// below k0 are left out (INNER of a step that did not write x has no max|x|:
+// a third less to read).
 template <int WHAT, int CB, int NT>
 __device__ __forceinline__ void fin_combine(const double* const (&src)[3], int64_t ng, int B,
-                                            int j0, double (&v)[3]) {
+                                            int j0, int k0, double (&v)[3]) {
   constexpr int NK = fin_kinds(WHAT);
   constexpr int RPT = 256 * CB / NT > 0 ? 256 * CB / NT : 1;  // rows per thread
   constexpr int H = BFIN_ROWS / RPT;                          // rows after the thread's own
@@ -206,20 +208,22 @@ __device__ __forceinline__ void fin_combine(const double* const (&src)[3], int64
       double y[NK][U][RPT];
 #pragma unroll
       for (int k = 0; k < NK; k++)
+        if (k >= k0)
 #pragma unroll
-        for (int u = 0; u < U; u++)
+          for (int u = 0; u < U; u++)
 #pragma unroll
-          for (int m = 0; m < RPT; m++) {  // past the end: the last value, not used
-            const int b = min(b0 + u * BFIN_ROWS + m * H, n - 1);
-            y[k][u][m] = src[k][b * B + j0 + c];
-          }
+            for (int m = 0; m < RPT; m++) {  // past the end: the last value, not used
+              const int b = min(b0 + u * BFIN_ROWS + m * H, n - 1);
+              y[k][u][m] = src[k][b * B + j0 + c];
+            }
 #pragma unroll
       for (int k = 0; k < NK; k++)
+        if (k >= k0)
 #pragma unroll
-        for (int u = 0; u < U; u++)
+          for (int u = 0; u < U; u++)
 #pragma unroll
-          for (int m = 0; m < RPT; m++)
-            if (b0 + u * BFIN_ROWS + m * H < n) a[k][m] = op(k, a[k][m], y[k][u][m]);
+            for (int m = 0; m < RPT; m++)
+              if (b0 + u * BFIN_ROWS + m * H < n) a[k][m] = op(k, a[k][m], y[k][u][m]);
     }
 #pragma unroll
     for (int k = 0; k < NK; k++) {
@@ -376,15 +380,14 @@ __global__ __launch_bounds__((Tile<B, G>::NT)) void k_bpupdate(
     __shared__ float s_beta[B];
     __shared__ int32_t s_it[B], s_pm[B], s_act[B];
     double v[3];
-    const double* const src[3] = {part + (xw ? 0 : ng * B), part + ng * B,
-                                  part + (5 - slot) * ng * B};
+    const double* const src[3] = {part, part + ng * B, part + (5 - slot) * ng * B};
     BCol c;
     int32_t st;
     if (t < B) {  // in flight beside the values
       c = bc[t];
       st = cst[t];
     }
-    fin_combine<BFIN_INNER, B, Tile<B, G>::NT>(src, ng, B, 0, v);
+    fin_combine<BFIN_INNER, B, Tile<B, G>::NT>(src, ng, B, 0, xw ? 0 : 1, v);
     if (t < B) {
       if (act) fin_advance(BFIN_INNER, v, c, st, xw);
       s_act[t] = st == BCOL_INNER && c.pending;
@@ -535,7 +538,7 @@ __global__ __launch_bounds__((Tile<B, G>::NT)) void k_bupdate(
     const double* const src[3] = {fin, fin, fin};
     const double rz = bc[j].rz;
     const int i = bc[j].it + 1;
-    fin_combine<BFIN_ALPHA, B, Tile<B, G>::NT>(src, nfin, B, 0, v);
+    fin_combine<BFIN_ALPHA, B, Tile<B, G>::NT>(src, nfin, B, 0, 0, v);
     alpha = rz / v[0];
     if (blockIdx.x == 0 && t < B && act) {
       bc[t].alpha = alpha;
@@ -794,7 +797,7 @@ __global__ __launch_bounds__(256) void k_bfinalize(int64_t ng, int B, const doub
   double v[3];
   if (act) {
     const double* const src[3] = {s0, s1, s2};
-    fin_combine<WHAT, 1, 256>(src, ng, B, j, v);
+    fin_combine<WHAT, 1, 256>(src, ng, B, j, WHAT == BFIN_INNER && !xw ? 1 : 0, v);
   } else if (cst == cstn) {
     return;
   }
@@ -988,7 +991,7 @@ void launch_bfin_alpha(hipStream_t s, const BFinSrc& q, int B, int32_t* cst, BCo
 void launch_bfin_inner(hipStream_t s, int64_t n1, int B, const double* part, int32_t* cst,
                        BCol* bc, int cur, int xw) {
   const int64_t ng = tile_groups(n1), nk = ng * B;
-  finalize<BFIN_INNER>(s, ng, B, part + (xw ? 0 : nk), part + nk, part + (2 + cur) * nk,
+  finalize<BFIN_INNER>(s, ng, B, part, part + nk, part + (2 + cur) * nk,
                        cst + cur * B, bc + cur * B, cst, bc, xw);
 }
 
