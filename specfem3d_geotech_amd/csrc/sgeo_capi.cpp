@@ -2041,11 +2041,12 @@ extern "C" int sgeo_batch_set_geometry(sgeo_batch* b, int32_t blocks_per_cu,
 }
 
 // Y = K P of the iterating columns, and the elements' p.Kp shares: from the
-// geometry on built meshes, else on the stored packed FP32 matrices
+// geometry on built meshes, else on the stored packed FP32 matrices.  Only
+// after batch_sync_operator, which sees to the operand of one of the two.
 static void batch_product(sgeo_batch* b, BmvGeom g, const int32_t* cst, const BCol* bc) {
   sgeo_mesh* m = b->mesh;
   const int want = BCOL_BIT(BCOL_INNER);
-  if (m->built)
+  if (b->built)
     launch_bmf(m->ctx->stream, m->nelmt, b->B, g, m->d_geo, m->d_gdof,
                b->d_eorder, b->d_p, b->n1 * b->B, b->d_Y32, b->d_edot, cst, bc, want);
   else
@@ -2070,6 +2071,7 @@ extern "C" int sgeo_batch_autotune(sgeo_batch* b, int32_t reps, int32_t* blocks_
   int inner = 0;
   for (int j = 0; j < b->B; j++) inner += b->phase[j] == BPH_RUN && b->cst[j] == BCOL_INNER;
   if (!inner) return fail(SGEO_ESTATE, "sgeo_batch_autotune: no column is iterating");
+  TRY(batch_sync_operator(b));  // the stiffness may have changed since the last step
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));

@@ -243,3 +243,41 @@ def test_matrices_buffer_of_a_closed_mesh_serves_the_next(ctx):
             assert np.array_equal(old.download_stiffness(), old_km)
             old.close()
     alive[0][0].close()
+
+
+@pytest.mark.parametrize("built", [True, False])
+@pytest.mark.parametrize("ncol", [1, 64])
+def test_autotune_after_the_stiffness_changed_hands(ctx, built, ncol):
+    """Mid-solve the mesh gets the same matrices uploaded (or built again
+    from the geometry) and the engine tunes the product that it now has; the
+    solve goes on to the solution of an engine that was left alone (both end
+    at relative updates of 1e-12 from FP64 residuals: 1e-10)."""
+    from specfem3d_geotech_amd.batch import DEFAULT_INNER_TOL, BatchEngine, device_mesh
+    from specfem3d_geotech_amd.plastic import dt_viscoplas
+    mesh = _mesh(8, 4, 6)
+    spec = hex2spec(mesh)
+    gam, ym, nu, phi, coh, psi = mesh.material_arrays()
+    ref = _engine_x(ctx, mesh, spec, ncol, 0)
+    dm, ext = device_mesh(ctx, mesh, spec)
+    try:
+        _, dinv = dm.build_stiffness(gam, ym, nu)
+        k = dm.download_stiffness()
+        if not built:
+            dm.upload_stiffness(k, dinv)
+        eng = BatchEngine(dm, ext, ncol)
+        try:
+            eng.begin(0, ym, nu, phi, coh, psi, dt_viscoplas(nu, phi, ym))
+            eng.advance(1e-12, 20000, DEFAULT_INNER_TOL, 5e-4, 1, max_steps=40)
+            if built:
+                dm.upload_stiffness(k, dinv)
+            else:
+                dm.build_stiffness(gam, ym, nu)
+            t = eng.autotune(2)
+            assert t["ms"] > 0
+            while not eng.advance(1e-12, 20000, DEFAULT_INNER_TOL, 5e-4, 1)["ended"][0]:
+                pass
+            assert rel_l2(eng.download(0)[0], ref) < 1e-10
+        finally:
+            eng.close()
+    finally:
+        dm.close()

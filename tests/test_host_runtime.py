@@ -1,0 +1,95 @@
+"""The library's host side on a stand-in HIP runtime (host_runtime.cpp):
+which kernels it launches on which buffers, and what it does when an
+allocation fails.  No GPU; each test runs in a process of its own, since the
+stand-in takes the place of the HIP runtime there."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+from conftest import ROOT
+
+PRELUDE = """
+import ctypes as C
+import sys
+sys.path.insert(0, {root!r})
+rt = C.CDLL({rt!r}, mode=C.RTLD_GLOBAL)
+rt.rt_used.restype = C.c_size_t
+rt.rt_limit.argtypes = [C.c_size_t]
+rt.rt_log.restype = C.c_char_p
+rt.rt_watch.argtypes = [C.c_char_p, C.c_int]
+import numpy as np
+from specfem3d_geotech_amd import _lib as L
+from specfem3d_geotech_amd.batch import BatchEngine
+from specfem3d_geotech_amd.mesh import slope_mesh
+from specfem3d_geotech_amd.slope import DeviceSlope
+from specfem3d_geotech_amd.solver import (K_F32, K_F64, KFMT_FULL, KFMT_PACKED, Context,
+                                          DeviceMesh)
+from specfem3d_geotech_amd.spec import hex2spec
+
+def log():
+    s = rt.rt_log().decode().splitlines()
+    rt.rt_clear()
+    return s
+
+ctx = Context(0)
+mesh = slope_mesh(3, 2, 2)
+spec = hex2spec(mesh)
+gam, ym, nu, phi, coh, psi = mesh.material_arrays()
+"""
+# leaves without the exit handlers of the HIP runtime that was loaded, but
+# not used
+EPILOGUE = """
+import os
+print("done", flush=True)
+os._exit(0)
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    lib = str(tmp_path_factory.mktemp("runtime") / "libhostruntime.so")
+    src = os.path.join(ROOT, "tests", "host_runtime.cpp")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I/opt/rocm/include", src, "-o", lib], check=True)
+
+    def run(body):
+        code = PRELUDE.format(root=ROOT, rt=lib) + body + EPILOGUE
+        r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True,
+                           timeout=120)
+        assert r.returncode == 0 and r.stdout.endswith("done\n"), r.stdout + r.stderr
+    return run
+
+
+# k_bmv_mfma's KP is its argument 3, k_bmf_lane's and k_bmf_point's geo their 2
+@pytest.mark.parametrize("build_first", [True, False])
+@pytest.mark.parametrize("ncol", [1, 64])
+def test_autotune_after_the_stiffness_changed_hands(runtime, build_first, ncol):
+    """An engine whose mesh got uploaded matrices after it was made on built
+    ones, or the other way round, tunes the product that its mesh has now, on
+    operands that exist."""
+    runtime(f"""
+dm = DeviceMesh(ctx, spec, len(gam))
+n = spec.nelmt
+def build():
+    return dm.build_stiffness(gam, ym, nu)
+def upload():
+    dm.upload_stiffness(np.zeros((81, 81, n), order='F'), np.ones(spec.neq + 1))
+ext, _ = build()
+if not {build_first}:
+    upload()
+eng = BatchEngine(dm, ext, {ncol})
+eng.set_graphs(False)
+eng.begin(0, ym, nu, phi, coh, psi, 0.1)
+eng.advance(1e-8, 100, 1e-4, 5e-4, 10, max_steps=8)
+(upload if {build_first} else build)()
+name, arg = ("k_bmv_mfma", 3) if {build_first} else ("k_bmf_", 2)
+rt.rt_watch(name.encode(), arg)
+log()
+eng.autotune(2)
+products = [s for s in log() if s.startswith("launch") and ("k_bmv_mfma" in s or "k_bmf_" in s)]
+assert products
+for s in products:
+    assert name in s and s.split()[-1] != "0", s
+""")
