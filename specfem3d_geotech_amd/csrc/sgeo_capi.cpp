@@ -236,18 +236,26 @@ static void spare_context(int device, int d) {
   if (drop) hipFree(drop);
 }
 
+// hipMalloc that fails only where no buffer lies idle.  A failed call's code
+// stays with hipGetLastError until it is read: it is taken here, so that
+// neither the call that got its memory after all nor a later one reports it.
+static hipError_t device_malloc(void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e == hipSuccess) return e;
+  (void)hipGetLastError();
+  int device = 0;
+  void* spare = hipGetDevice(&device) == hipSuccess ? spare_any(device) : nullptr;
+  if (!spare) return e;
+  hipFree(spare);
+  e = hipMalloc(p, bytes);
+  if (e != hipSuccess) (void)hipGetLastError();
+  return e;
+}
+
 template <typename T>
 static int dalloc(T** p, size_t n, size_t* acc = nullptr) {
   if (n == 0) n = 1;
-  hipError_t e = hipMalloc((void**)p, n * sizeof(T));
-  if (e != hipSuccess) {  // not while a buffer lies idle
-    int device = 0;
-    void* spare = hipGetDevice(&device) == hipSuccess ? spare_any(device) : nullptr;
-    if (spare) {
-      hipFree(spare);
-      e = hipMalloc((void**)p, n * sizeof(T));
-    }
-  }
+  const hipError_t e = device_malloc((void**)p, n * sizeof(T));
   if (e != hipSuccess)
     return fail(SGEO_ENOMEM, "hipMalloc of %zu bytes failed: %s", n * sizeof(T),
                 hipGetErrorString(e));

@@ -93,3 +93,31 @@ assert products
 for s in products:
     assert name in s and s.split()[-1] != "0", s
 """)
+
+
+def test_failed_allocation_takes_the_kept_matrices_buffer(runtime):
+    """Where device memory runs out while the matrices buffer of a closed
+    mesh lies idle, the buffer goes and the call succeeds; where there is
+    none, the call fails as out of memory and leaves nothing behind for the
+    calls after it."""
+    runtime("""
+big = 8 * 6561 * spec.nelmt
+dm = DeviceMesh(ctx, spec, len(gam))
+dm.build_stiffness(gam, ym, nu)
+dm.close()
+rt.rt_limit(rt.rt_used() + 1000)
+log()
+dm = DeviceMesh(ctx, spec, len(gam))  # larger than what is left beside the buffer
+s = log()
+assert any(x.startswith("fail") for x in s) and "free %d" % big in s, s
+rt.rt_limit(rt.rt_used() + 1000)
+for call in (lambda: dm.build_stiffness(gam, ym, nu), lambda: DeviceMesh(ctx, spec, len(gam))):
+    try:
+        call()
+        assert False, "no room for it"
+    except RuntimeError as e:
+        assert "failed: out of memory" in str(e), e
+rt.rt_limit(1 << 40)
+dm.build_stiffness(gam, ym, nu)
+DeviceMesh(ctx, spec, len(gam)).close()
+""")
