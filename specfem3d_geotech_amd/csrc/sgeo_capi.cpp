@@ -173,7 +173,8 @@ struct sgeo_slope {
 // sgeo_mesh_destroy took 65 ms and the frees of the next numbering 20, in a
 // set-up of 20.  With the buffer kept, 60 meshes in a row took 2.1 ms each to
 // destroy.  Given back when the device's last context ends, or when an
-// allocation fails.
+// allocation of this library fails (device_malloc); other users of the GPU in
+// the process do not get at it before.
 #define SPARE_MAX ((size_t)16 << 30)
 #define SPARE_DEVICES 64
 struct Spare {
@@ -236,10 +237,10 @@ static void spare_context(int device, int d) {
   if (drop) hipFree(drop);
 }
 
-// hipMalloc that fails only where no buffer lies idle.  A failed call's code
-// stays with hipGetLastError until it is read: it is taken here, so that
-// neither the call that got its memory after all nor a later one reports it.
-static hipError_t device_malloc(void** p, size_t bytes) {
+// A failed call's code stays with hipGetLastError until it is read: it is
+// taken here, so that neither the call that got its memory after all nor a
+// later one reports it.
+hipError_t sgeo::device_malloc(void** p, size_t bytes) {
   hipError_t e = hipMalloc(p, bytes);
   if (e == hipSuccess) return e;
   (void)hipGetLastError();

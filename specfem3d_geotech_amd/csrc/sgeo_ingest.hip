@@ -227,7 +227,7 @@ struct Buf {
 
 template <typename T>
 hipError_t alloc(Buf& b, int64_t n) {
-  return hipMalloc(&b.p, (size_t)(n > 0 ? n : 1) * sizeof(T));
+  return device_malloc(&b.p, (size_t)(n > 0 ? n : 1) * sizeof(T));
 }
 
 }  // namespace
@@ -258,7 +258,7 @@ hipError_t hex2spec_run(hipStream_t s, int32_t nelmt, const double* d_coord8,
   ICHK(alloc<int32_t>(brk, n));
   ICHK(alloc<int32_t>(incl, n));
   ICHK(alloc<double>(keys, n));
-  ICHK(hipMalloc((void**)&r.corners, (size_t)nelmt * 24 * sizeof(double)));
+  ICHK(device_malloc((void**)&r.corners, (size_t)nelmt * 24 * sizeof(double)));
   auto* X = (double*)px.p;
   auto* Y = (double*)py.p;
   auto* Z = (double*)pz.p;
@@ -285,7 +285,7 @@ hipError_t hex2spec_run(hipStream_t s, int32_t nelmt, const double* d_coord8,
   ICHK(rocprim::exclusive_scan(nullptr, t1, BRK, INC, 0, (size_t)n * 3,
                                rocprim::plus<int32_t>(), s));
   tb = std::max(tb, t1);
-  ICHK(hipMalloc(&tmp.p, tb));
+  ICHK(device_malloc(&tmp.p, tb));
   hipLaunchKernelGGL(k_fill, dim3(gs(n)), dim3(256), 0, s, n, SEG, 0);
   int32_t nseg = 1;
   const double* P[3] = {X, Y, Z};
@@ -323,8 +323,8 @@ hipError_t hex2spec_run(hipStream_t s, int32_t nelmt, const double* d_coord8,
   }
   int32_t* RANK = BRK;
   hipLaunchKernelGGL(k_rank, dim3(gs(ng)), dim3(256), 0, s, ng, INC, RANK);
-  ICHK(hipMalloc((void**)&r.g_num, (size_t)n * 4));
-  ICHK(hipMalloc((void**)&r.g_coord, (size_t)ng * 3 * 8));
+  ICHK(device_malloc((void**)&r.g_num, (size_t)n * 4));
+  ICHK(device_malloc((void**)&r.g_coord, (size_t)ng * 3 * 8));
   hipLaunchKernelGGL(k_node_of_point, dim3(gs(n)), dim3(256), 0, s, n, SEG, RANK, r.g_num);
   hipLaunchKernelGGL(k_node_coord, dim3(gs(ng)), dim3(256), 0, s, ng, LAST, RANK, X, Y, Z,
                      r.g_coord);
@@ -343,12 +343,12 @@ hipError_t hex2spec_run(hipStream_t s, int32_t nelmt, const double* d_coord8,
     ICHK(rocprim::exclusive_scan(tmp.p, t, FLAG, EXCL, 0, (size_t)(3 * ng),
                                  rocprim::plus<int32_t>(), s));
   }
-  ICHK(hipMalloc((void**)&r.gdof, (size_t)ng * 3 * 4));
+  ICHK(device_malloc((void**)&r.gdof, (size_t)ng * 3 * 4));
   hipLaunchKernelGGL(k_number, dim3(gs(3 * ng)), dim3(256), 0, s, 3 * ng, FLAG, EXCL, r.gdof);
   int32_t lastx = 0, lastf = 0;
   ICHK(hipMemcpyAsync(&lastx, EXCL + (3 * ng - 1), 4, hipMemcpyDeviceToHost, s));
   ICHK(hipMemcpyAsync(&lastf, FLAG + (3 * ng - 1), 4, hipMemcpyDeviceToHost, s));
-  ICHK(hipMalloc((void**)&r.gdof_elmt, (size_t)nelmt * 81 * 4));
+  ICHK(device_malloc((void**)&r.gdof_elmt, (size_t)nelmt * 81 * 4));
   hipLaunchKernelGGL(k_gdof_elmt, dim3(gs((int64_t)nelmt * 81)), dim3(256), 0, s,
                      (int64_t)nelmt, r.g_num, r.gdof, r.gdof_elmt);
   ICHK(hipGetLastError());

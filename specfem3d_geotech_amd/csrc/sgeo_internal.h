@@ -43,6 +43,11 @@ struct BodyArgs {
   double* sf_pt = nullptr;         // [col][nel][27] (excavation)
 };
 
+// hipMalloc of everything the library keeps on a device (sgeo_capi.cpp): where
+// it fails, an idle matrices buffer is given back first.  No error is left for
+// hipGetLastError.
+hipError_t device_malloc(void** p, size_t bytes);
+
 unsigned vec_reduce_blocks(int64_t n1);
 
 void launch_stiffness(hipStream_t s, int32_t nelmt, const double* corners,

@@ -121,3 +121,38 @@ rt.rt_limit(1 << 40)
 dm.build_stiffness(gam, ym, nu)
 DeviceMesh(ctx, spec, len(gam)).close()
 """)
+
+
+def test_numbering_takes_the_kept_matrices_buffer(runtime):
+    """The device numbering of the next mesh, too, gets memory that only the
+    buffer of a closed mesh holds, whichever of its allocations fails first;
+    where there is no buffer it fails and keeps nothing."""
+    runtime("""
+from specfem3d_geotech_amd.spec import hex2spec_device
+mesh = slope_mesh(3, 2, 2)
+big = 8 * 6561 * spec.nelmt
+log()
+hex2spec_device(ctx, mesh)
+sizes = [int(x.split()[1]) for x in log() if x.startswith("malloc")]
+assert len(sizes) > 15
+for left in np.cumsum([0] + sizes[:-1]):
+    dm = DeviceMesh(ctx, spec, len(gam))
+    dm.build_stiffness(gam, ym, nu)
+    dm.close()
+    rt.rt_limit(rt.rt_used() + int(left))
+    log()
+    hex2spec_device(ctx, mesh)
+    s = log()
+    assert sum(x.startswith("fail") for x in s) == 1 and "free %d" % big in s, (left, s)
+    rt.rt_limit(1 << 40)
+    used = rt.rt_used()
+    rt.rt_limit(used + int(left))
+    try:
+        hex2spec_device(ctx, mesh)
+        assert False, "no room for it"
+    except RuntimeError as e:
+        assert "out of memory" in str(e), e
+    assert rt.rt_used() == used
+    rt.rt_limit(1 << 40)
+    hex2spec_device(ctx, mesh)
+""")
