@@ -369,10 +369,10 @@ static hipError_t to_host(sgeo_ctx* c, void* host, const void* dev, size_t n) {
 
 static int ensure_part(sgeo_ctx* c, size_t n) {
   if (n <= c->part_cap) return 0;
+  double* part = nullptr;
+  TRY(dalloc(&part, n));  // where it fails, the other meshes keep theirs
   if (c->d_part) hipFree(c->d_part);
-  c->d_part = nullptr;
-  c->part_cap = 0;
-  TRY(dalloc(&c->d_part, n));
+  c->d_part = part;
   c->part_cap = n;
   return 0;
 }

@@ -156,3 +156,37 @@ for left in np.cumsum([0] + sizes[:-1]):
     rt.rt_limit(1 << 40)
     hex2spec_device(ctx, mesh)
 """)
+
+
+def test_failed_larger_mesh_leaves_the_others_their_partials(runtime):
+    """A mesh that could not be made for want of memory leaves the context's
+    reduction partials, which its other meshes use, as they were."""
+    runtime("""
+large = hex2spec(slope_mesh(40, 20, 30))
+def make(sp):
+    log()
+    dm = DeviceMesh(ctx, sp, len(gam))
+    return dm, [int(x.split()[1]) for x in log() if x.startswith("malloc")]
+dm, sizes = make(large)
+dm.close()
+ctx.close()
+ctx = Context(0)
+dm, small = make(spec)
+ext, _ = dm.build_stiffness(gam, ym, nu)
+# the partials come last: everything before them fits
+rt.rt_limit(rt.rt_used() + sum(sizes) - small[-1] - 1)
+try:
+    DeviceMesh(ctx, large, len(gam))
+    assert False, "no room for it"
+except RuntimeError as e:
+    assert "out of memory" in str(e), e
+rt.rt_limit(1 << 40)
+rt.rt_watch(b"k_pcg_begin", 2)
+log()
+try:
+    dm.solve(ext, cg_maxiter=1)  # no kernel runs, so no verdict
+except RuntimeError:
+    pass
+begin = [x for x in log() if "k_pcg_begin" in x]
+assert len(begin) == 1 and begin[0].split()[-1] != "0", begin
+""")
