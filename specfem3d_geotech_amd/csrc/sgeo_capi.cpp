@@ -725,7 +725,9 @@ static bool matrix_free(const sgeo_mesh* m) {
 }
 
 // Derived storage of the selected operator, rebuilt from the canonical FP64
-// full K whenever K changed (k_ver).
+// full K whenever K changed (k_ver).  Every entry that multiplies by it calls
+// this first: the call that changed the operator may have found no memory for
+// it.  stored: the matrices too where the product needs none.
 static int refresh_operator(sgeo_mesh* m, bool stored = false) {
   hipStream_t s = m->ctx->stream;
   const size_t nk = (size_t)m->nelmt * 6561;
@@ -1038,6 +1040,7 @@ extern "C" int sgeo_mesh_matvec(sgeo_mesh* m, const double* p, double* kp) {
   HIPCHK(hipSetDevice(c->device));
   hipStream_t s = c->stream;
   const int64_t n1 = (int64_t)m->neq + 1;
+  TRY(refresh_operator(m));
   HIPCHK(hipMemcpyAsync(m->d_p, p, n1 * 8, hipMemcpyHostToDevice, s));
   ebe_elem(m, m->d_p, m->d_Y, 0);
   launch_assemble(s, n1, m->d_rowptr, m->d_slots, m->d_Y, m->d_kp, c->d_sc, 0);
@@ -1496,6 +1499,7 @@ extern "C" int sgeo_mesh_solve(sgeo_mesh* m, double* u, const double* f,
   HIPCHK(hipSetDevice(c->device));
   hipStream_t s = c->stream;
   const size_t n1 = (size_t)m->neq + 1;
+  TRY(refresh_operator(m));
   double *d_u = nullptr, *d_f = nullptr;
   DevScratch tmp;
   TRY(tmp.alloc(&d_u, n1));
@@ -1581,7 +1585,7 @@ extern "C" int sgeo_slope_plastic_iter(sgeo_slope* t, double cg_tol,
   hipStream_t s = c->stream;
   const int64_t n1 = (int64_t)m->neq + 1;
   int32_t it = 0, ec = -1;
-  if (matrix_free(m)) TRY(ensure_packed(m, SGEO_K_F64));  // a trial multiplies the matrices
+  TRY(refresh_operator(m, true));  // a trial multiplies the matrices
   launch_load(s, n1, t->d_ext, t->d_body, t->d_load);
   TRY(pcg_device(m, t->d_x, t->d_load, cg_tol, cg_maxiter, &it, &ec, true));
   if (cg_iter) *cg_iter = it;

@@ -190,3 +190,35 @@ except RuntimeError:
 begin = [x for x in log() if "k_pcg_begin" in x]
 assert len(begin) == 1 and begin[0].split()[-1] != "0", begin
 """)
+
+
+@pytest.mark.parametrize("kprec", ["K_F64", "K_F32"])
+def test_operator_whose_storage_failed_is_not_used(runtime, kprec):
+    """Where the packed matrices of an operator could not be allocated (an
+    upload onto a mesh that had none, a choice of operator), products and
+    solves report that instead of reading matrices that are not there, and
+    work once there is room."""
+    runtime(f"""
+dm = DeviceMesh(ctx, spec, len(gam))
+ext, dinv = dm.build_stiffness(gam, ym, nu)
+if {kprec} == K_F64:
+    dm.set_operator(K_F64, KFMT_PACKED)  # from the geometry: nothing stored
+    change = lambda: dm.upload_stiffness(np.zeros((81, 81, spec.nelmt), order='F'), dinv)
+else:
+    change = lambda: dm.set_operator({kprec}, KFMT_PACKED)
+room = 20 * spec.neq
+for call in (change, lambda: dm.matvec(ext), lambda: dm.solve(ext, cg_maxiter=1)):
+    rt.rt_limit(rt.rt_used() + room)
+    log()
+    try:
+        call()
+        assert False, "no room for it"
+    except RuntimeError as e:
+        assert "out of memory" in str(e), e
+    assert not [x for x in log() if "k_ebe" in x or "k_mf64" in x]
+rt.rt_limit(1 << 40)
+rt.rt_watch(b"k_ebe_packed", 1)
+dm.matvec(ext)
+s = [x for x in log() if "k_ebe_packed" in x]
+assert len(s) == 1 and s[0].split()[-1] != "0", s
+""")
