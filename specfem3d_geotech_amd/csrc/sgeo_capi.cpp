@@ -134,6 +134,7 @@ struct sgeo_mesh {
   // K was built from the corners and materials, so products can be formed
   // from them; false for uploaded matrices
   bool built = false;
+  bool trials = false;  // a trial was made on this mesh: packed operators are stored
   double2* d_lame = nullptr;  // (lambda, mu) per material of the built K
   float4* d_geo = nullptr;    // the batched product's geometry, of version geo_ver
   int geo_ver = -1;
@@ -719,7 +720,8 @@ static int set_k_storage(sgeo_mesh* m, int kprec) {
 }
 
 // The packed FP64 operator of a built mesh is applied from the geometry
-// (k_mf64): its packed matrices are made only where a kernel reads them.
+// (k_mf64): its packed matrices are made only where a kernel reads them, for a
+// trial when it is made (or K changes after that), not amid its iterations.
 static bool matrix_free(const sgeo_mesh* m) {
   return m->built && m->kfmt == SGEO_KFMT_PACKED && m->kprec == SGEO_K_F64;
 }
@@ -739,7 +741,7 @@ static int refresh_operator(sgeo_mesh* m, bool stored = false) {
       m->k32_ver = m->k_ver;
     }
   } else if (m->kfmt == SGEO_KFMT_PACKED && m->kprec == SGEO_K_F64) {
-    if (!stored && matrix_free(m)) return 0;
+    if (!stored && !m->trials && matrix_free(m)) return 0;
     if (!m->d_KP64) TRY(dalloc(&m->d_KP64, np, &m->bytes));
     if (m->kp64_ver != m->k_ver) {
       launch_pack_upper_f64(s, m->nelmt, m->d_K64, m->d_KP64);
@@ -1392,6 +1394,8 @@ extern "C" int sgeo_slope_create(sgeo_mesh* m, const double* extload,
   TRY(dalloc(&t->d_BL, (size_t)m->nelmt * 81));
   TRY(dalloc(&t->d_flags, (size_t)m->nelmt * 27));
   TRY(dalloc(&t->d_mp, (size_t)std::max(1, m->nmat)));
+  TRY(refresh_operator(m, true));
+  m->trials = true;
   HIPCHK(hipMemcpyAsync(t->d_ext, extload, n1 * 8, hipMemcpyHostToDevice, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
   *out = guard.release();
@@ -1585,7 +1589,7 @@ extern "C" int sgeo_slope_plastic_iter(sgeo_slope* t, double cg_tol,
   hipStream_t s = c->stream;
   const int64_t n1 = (int64_t)m->neq + 1;
   int32_t it = 0, ec = -1;
-  TRY(refresh_operator(m, true));  // a trial multiplies the matrices
+  TRY(refresh_operator(m));
   launch_load(s, n1, t->d_ext, t->d_body, t->d_load);
   TRY(pcg_device(m, t->d_x, t->d_load, cg_tol, cg_maxiter, &it, &ec, true));
   if (cg_iter) *cg_iter = it;

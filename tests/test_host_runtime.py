@@ -222,3 +222,34 @@ dm.matvec(ext)
 s = [x for x in log() if "k_ebe_packed" in x]
 assert len(s) == 1 and s[0].split()[-1] != "0", s
 """)
+
+
+def test_trials_find_their_matrices_packed(runtime):
+    """A trial on the packed operator of a built mesh packs the matrices it
+    multiplies when it is made, and a change of the stiffness packs them
+    again: a plastic iteration neither allocates nor packs."""
+    runtime("""
+dm = DeviceMesh(ctx, spec, len(gam))
+ext, dinv = dm.build_stiffness(gam, ym, nu)
+dm.set_operator(K_F64, KFMT_PACKED)
+assert not [x for x in log() if "k_pack_upper" in x]
+t = DeviceSlope(dm, ext)
+t.begin_srf(ym, nu, phi, coh, psi, 0.1)
+assert len([x for x in log() if "k_pack_upper" in x]) == 1
+def iterate():
+    log()
+    try:
+        t.plastic_iter(1e-8, 1, 5e-4, False)  # no kernel runs, so no verdict
+    except RuntimeError as e:
+        assert "verdict" in str(e), e
+    s = log()
+    assert any("k_ebe_packed" in x for x in s), s
+    assert not [x for x in s if "k_pack_upper" in x or x.startswith("malloc")], s
+iterate()
+for change in (lambda: dm.build_stiffness(gam, 2 * ym, nu),
+               lambda: dm.upload_stiffness(np.zeros((81, 81, spec.nelmt), order='F'), dinv),
+               lambda: dm.build_stiffness(gam, ym, nu)):
+    change()
+    assert len([x for x in log() if "k_pack_upper" in x]) == 1
+    iterate()
+""")
