@@ -393,7 +393,10 @@ int sgeo_batch_set_graphs(sgeo_batch *batch, int enable);
  * candidate on this engine's mesh and iterating columns -- blocks per CU
  * 4, 3, 2, 1 with the XCD-aware element split, then 4, 3, 2, 1 with a plain
  * grid-stride walk (ms_table[8], in that order, may be NULL) -- and keeps the
- * fastest for later steps.  Needs at least one column iterating
+ * fastest for later steps.  From the geometry the product reads the split
+ * only, or neither on small systems: candidates that launch the same then
+ * share one timing, and what is not read keeps its value.  Needs at least one
+ * column iterating
  * (SGEO_ESTATE otherwise).  The geometry never changes a result bit, and
  * tuning between steps does not change the trials' results. */
 int sgeo_batch_autotune(sgeo_batch *batch, int32_t reps, int32_t *blocks_per_cu,

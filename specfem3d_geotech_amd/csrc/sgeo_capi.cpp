@@ -2072,8 +2072,11 @@ static void batch_product(sgeo_batch* b, BmvGeom g, const int32_t* cst, const BC
 }
 
 // Launch-geometry autotuner of the product: times `reps` launches of
-// every candidate (blocks per CU 1..3, XCD-aware split on/off) on the
+// every candidate (blocks per CU 4..1, XCD-aware split on/off) on the
 // engine's own mesh and the columns iterating now, and keeps the fastest.
+// Of the products from the geometry the lane kernel reads the split only and
+// the point kernel neither: candidates that do not differ share one timing,
+// and what is not read stays as it is.
 // The product only rewrites the element products of iterating columns from
 // their current search directions, which the next step recomputes before
 // any use, so tuning between steps changes no result.
@@ -2089,17 +2092,23 @@ extern "C" int sgeo_batch_autotune(sgeo_batch* b, int32_t reps, int32_t* blocks_
   for (int j = 0; j < b->B; j++) inner += b->phase[j] == BPH_RUN && b->cst[j] == BCOL_INNER;
   if (!inner) return fail(SGEO_ESTATE, "sgeo_batch_autotune: no column is iterating");
   TRY(batch_sync_operator(b));  // the stiffness may have changed since the last step
+  const bool reads_bpc = !b->built, reads_xcd = !b->built || !bmf_by_points(m->nelmt, b->B);
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
-  double best = 1e30;
-  BmvGeom pick = b->geom;
+  double best = 1e30, avg = 0.0;
+  BmvGeom pick = b->geom, timed;
   int k = 0;
   for (int xs = 1; xs >= 0; xs--) {
     for (int bpc = 4; bpc >= 1; bpc--, k++) {
-      BmvGeom g;
-      g.blocks_per_cu = bpc;
-      g.xcd_split = xs;
+      BmvGeom g = b->geom;
+      if (reads_bpc) g.blocks_per_cu = bpc;
+      if (reads_xcd) g.xcd_split = xs;
+      if (k > 0 && g.blocks_per_cu == timed.blocks_per_cu && g.xcd_split == timed.xcd_split) {
+        if (ms_table) ms_table[k] = avg;
+        continue;
+      }
+      timed = g;
       auto launch = [&]() {
         batch_product(b, g, b->d_cst, b->d_bc);
       };
@@ -2110,7 +2119,7 @@ extern "C" int sgeo_batch_autotune(sgeo_batch* b, int32_t reps, int32_t* blocks_
       HIPCHK(hipEventSynchronize(e1));
       float ms = 0.f;
       HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-      const double avg = (double)ms / reps;
+      avg = (double)ms / reps;
       if (ms_table) ms_table[k] = avg;
       if (avg < best) {
         best = avg;

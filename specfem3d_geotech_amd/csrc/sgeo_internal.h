@@ -231,6 +231,7 @@ void launch_bmv_mfma_f32(hipStream_t s, int32_t nelmt, int B, int n_cu, BmvGeom 
 // the same from the geometry (built meshes); geo: three float4 per point
 void launch_point_geometry(hipStream_t s, int32_t nelmt, const double* corners,
                            const int32_t* mat_id, const double2* lame, float4* geo);
+bool bmf_by_points(int32_t nelmt, int B);
 void launch_bmf(hipStream_t s, int32_t nelmt, int B, BmvGeom geom, const float4* geo,
                 const int32_t* gdof, const int32_t* eorder, const float* P, int64_t nv,
                 float* Y, double* edot, const int32_t* cst, const BCol* bc, int want_mask);

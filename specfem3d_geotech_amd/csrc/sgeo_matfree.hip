@@ -604,6 +604,10 @@ void launch_point_geometry(hipStream_t s, int32_t nelmt, const double* corners,
                      dim3(256), 0, s, nelmt, corners, mat_id, lame, geo);
 }
 
+bool bmf_by_points(int32_t nelmt, int B) {
+  return B < 4 || (int64_t)nelmt * B <= BMF_POINT_SLOTS;
+}
+
 // Product of the engine's columns from the geometry.  Of the launch geometry
 // the lane kernel takes the XCD split of its walk; it is not persistent (a
 // fixed number of blocks per CU left the last of them running alone).
@@ -611,8 +615,8 @@ void launch_bmf(hipStream_t s, int32_t nelmt, int B, BmvGeom geom, const float4*
                 const int32_t* gdof, const int32_t* eorder, const float* P, int64_t nv,
                 float* Y, double* edot, const int32_t* cst, const BCol* bc, int want_mask) {
   if (nelmt <= 0) return;
-  const int64_t nslot = (int64_t)nelmt * B;
-  if (B < 4 || nslot <= BMF_POINT_SLOTS) {
+  if (bmf_by_points(nelmt, B)) {
+    const int64_t nslot = (int64_t)nelmt * B;
     int lb = 0;
     while ((1 << lb) < B) lb++;
     hipLaunchKernelGGL(k_bmf_point, dim3((unsigned)((nslot + 7) / 8)), dim3(256), 0, s,

@@ -253,3 +253,34 @@ for change in (lambda: dm.build_stiffness(gam, 2 * ym, nu),
     assert len([x for x in log() if "k_pack_upper" in x]) == 1
     iterate()
 """)
+
+
+# ncol, elements: by points (reads no geometry), by lanes (the XCD split only)
+# and uploaded matrices (both)
+@pytest.mark.parametrize("grid,upload,distinct,pick", [((3, 2, 2), False, 1, (3, 1)),
+                                                       ((12, 5, 5), False, 2, (3, 0)),
+                                                       ((3, 2, 2), True, 8, (1, 0))])
+def test_autotune_times_what_differs(runtime, grid, upload, distinct, pick):
+    """Candidates that launch the same kernel the same way are timed once,
+    and what the product does not read stays as it was (defaults: 3 blocks
+    per CU, the XCD split).  Every timing here is shorter than the one
+    before it."""
+    runtime(f"""
+mesh = slope_mesh(*{grid})
+spec = hex2spec(mesh)
+dm = DeviceMesh(ctx, spec, len(gam))
+ext, dinv = dm.build_stiffness(gam, ym, nu)
+if {upload}:
+    dm.upload_stiffness(np.zeros((81, 81, spec.nelmt), order='F'), dinv)
+eng = BatchEngine(dm, ext, 64)
+eng.set_graphs(False)
+eng.begin(0, ym, nu, phi, coh, psi, 0.1)
+eng.advance(1e-8, 100, 1e-4, 5e-4, 10, max_steps=8)
+log()
+t = eng.autotune(3)
+n = sum("k_bm" in x for x in log())
+assert n == {distinct} * 4, n
+assert (t["blocks_per_cu"], t["xcd_split"]) == {pick}, t
+ms = [c["ms"] for c in t["candidates"]]
+assert len(ms) == 8 and len(set(ms)) == {distinct} and t["ms"] == min(ms), t
+""")
