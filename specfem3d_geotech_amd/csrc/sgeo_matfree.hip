@@ -242,7 +242,11 @@ void launch_mf64(hipStream_t s, int32_t nelmt, const double* corners, const int3
 // a line's derivatives be formed without its factors 1/2: with the line's
 // node values a, b, c, m = c - a and q = (a + c) - 2 b, twice the
 // derivatives at the three points are m - 2 q, m and m + 2 q, and the
-// transposed sums take the coefficients of 2 D.
+// transposed sums take the coefficients of 2 D.  A power of two per point
+// moves from the Lame terms to adj, whose largest entry becomes 1 .. 2: with
+// elements of length h they are E / h^3 and h^2, and FP32 would end for h below about
+// 1e-11 or above 1e14 where their product, E h as in the matrices, does not.
+// It enters a flux twice and leaves it exactly, so it changes no bit elsewhere.
 //
 // Both kernels below form every value by the same operations in the same
 // order, so a column's bits do not depend on which one ran, on B or on the
@@ -268,9 +272,13 @@ __global__ __launch_bounds__(256) void k_point_geometry(
   const double det = adjugate_point(i % 3, (i / 3) % 3, i / 9, xc, adj);
   const double w = gll_weight(i) / det;
   const double2 lm = lame[mat_id[e] - 1];
-  const double f[12] = {0.5 * adj[0][0], 0.5 * adj[0][1], 0.5 * adj[0][2], 0.5 * adj[1][0],
-                        0.5 * adj[1][1], 0.5 * adj[1][2], 0.5 * adj[2][0], 0.5 * adj[2][1],
-                        0.5 * adj[2][2], lm.x * w,        lm.y * w,        2.0 * lm.y * w};
+  double f[12] = {0.5 * adj[0][0], 0.5 * adj[0][1], 0.5 * adj[0][2], 0.5 * adj[1][0],
+                  0.5 * adj[1][1], 0.5 * adj[1][2], 0.5 * adj[2][0], 0.5 * adj[2][1],
+                  0.5 * adj[2][2], lm.x * w,        lm.y * w,        2.0 * lm.y * w};
+  double big = 0.0;
+  for (int k = 0; k < 9; k++) big = fmax(big, fabs(f[k]));
+  const int sh = big > 0.0 && big < INFINITY ? ilogb(big) : 0;
+  for (int k = 0; k < 12; k++) f[k] = ldexp(f[k], k < 9 ? -sh : 2 * sh);
   float4* o = geo + q * 3;
   for (int k = 0; k < 3; k++)
     o[k] = float4{(float)f[4 * k], (float)f[4 * k + 1], (float)f[4 * k + 2], (float)f[4 * k + 3]};

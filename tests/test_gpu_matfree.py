@@ -281,3 +281,20 @@ def test_autotune_after_the_stiffness_changed_hands(ctx, built, ncol):
             eng.close()
     finally:
         dm.close()
+
+
+@pytest.mark.parametrize("ncol,grid", [(1, (4, 3, 2)), (64, (12, 5, 5))])
+@pytest.mark.parametrize("exp", [-40, 48])
+def test_engine_in_other_units_of_length(ctx, ncol, grid, exp):
+    """The same slope in a unit of length 2^exp times as large (unit weights
+    smaller by it, moduli kept): every number of the solve is a power of two
+    times that of the plain one, so x is, bit for bit.  E / h^3 and h^2 leave
+    the range of FP32 here, E h does not."""
+    mesh = _mesh(*grid)
+    x = _engine_x(ctx, mesh, hex2spec(mesh), ncol, 24)
+    assert np.abs(x).max() > 0 and np.isfinite(x).all()
+    s = 2.0 ** exp
+    mesh.coord = mesh.coord * s
+    mesh.materials = [Material(gam=m.gam / s, ym=m.ym, nu=m.nu, phi=m.phi, coh=m.coh)
+                      for m in SOILS]
+    assert np.array_equal(_engine_x(ctx, mesh, hex2spec(mesh), ncol, 24), x * s)
