@@ -1,17 +1,19 @@
 // sgeo_batch.hip -- multi-trial (multi-RHS) kernels of the mixed-precision
 // EBE-PCG: B strength-reduction trials share one mesh and one elastic
 // stiffness (the viscoplastic method never changes K, src/slope.F90:288), so
-// every CG iteration streams K once for all B columns.
+// every CG iteration applies K once to all B columns.  Here: the FP32 product
+// of uploaded matrices, the FP64 residual product, and the columns' body
+// passes and state.  Built meshes' FP32 products come from the geometry
+// (sgeo_matfree.hip); the vector kernels and reductions are in sgeo_bvec.hip.
 //
 // Vectors are interleaved [n1][B] (column fastest): an element gathers 81
 // contiguous B-vectors and every update is unit-stride.  The inner CG
-// vectors (r, p) and the element product are FP32 (the product on MFMA; K p
-// is summed from the element products inside the update, never stored);
-// dot products, the solution x, the FP64 true residual f - K x and all
-// plastic state are FP64.  Every reduction combines per-chunk (or
-// per-element) partials in groups, then per column, in a fixed order, so a
-// column's arithmetic does not depend on B or on the other columns: a trial
-// gives the same bits alone and in any batch.
+// vectors (r, p) and the element product are FP32 (K p is summed from the
+// element products inside the update, never stored); dot products, the
+// solution x, the FP64 true residual f - K x and all plastic state are FP64.
+// Every reduction combines the partials of groups of tiles in a fixed order,
+// so a column's arithmetic does not depend on B or on the other columns: a
+// trial gives the same bits alone and in any batch.
 #pragma clang fp contract(off)
 
 #include "sgeo_device.h"
@@ -26,7 +28,7 @@ __device__ __forceinline__ bool wanted(const int32_t* cst, int j, int mask) {
 }
 
 // --------------------------------------------------------------------------
-// FP32 batched element product on MFMA:
+// FP32 batched element product of uploaded matrices, on MFMA:
 //   Y[e][r][j] = sum_c K_e(r,c) P[g(e,c)][j]
 // with v_mfma_f32_16x16x4f32 (A 16x4, B 4x16, D 16x16): rows 0..79 in 5
 // tiles of 16, columns in tiles of 16 (B < 16: one partial tile), k in 21

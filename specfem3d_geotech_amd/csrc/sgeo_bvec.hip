@@ -2,8 +2,9 @@
 // on the interleaved [equation][column] arrays.
 //
 // The equations are split into tiles of T (8 .. 256, a power of two chosen
-// by the equation count only: enough tiles to fill the chip on small
-// systems, at most 16,384 partial tiles on large ones).  A tile's partial of
+// by the equation count only: enough tiles to fill the chip on small systems,
+// at most 16,384 of them up to 4.19 million equations, where T has reached
+// 256, and n / 256 above).  A tile's partial of
 // a column is the sum of eight interleaved accumulators, accumulator i
 // taking the equations 8 s + i of the tile in order of s, combined pairwise
 // (0,1) (2,3) .., then the pairs, then the two halves; four or eight tiles
@@ -831,7 +832,6 @@ __global__ __launch_bounds__(256) void k_buerr_finalize(
     ps[j].n_plastic = 0;
   }
 }
-
 
 // --------------------------------------------------------------------------
 // launch wrappers

@@ -1775,7 +1775,7 @@ struct sgeo_batch {
   // residual list of a residual step: columns [0..64), count at [64]; and
   // each listed column's place in it
   int32_t *d_rlist = nullptr, *d_rslot = nullptr;
-  int32_t* d_eorder = nullptr;  // the MFMA product's walk over the elements
+  int32_t* d_eorder = nullptr;  // the product's walk over the elements
   double* d_part = nullptr;  // equation-chunk partials and their groups
   double* d_edot = nullptr;  // the elements' p.Kp shares and their groups
   // per column
@@ -1797,7 +1797,7 @@ struct sgeo_batch {
   bool use_graphs = true;
   hipGraph_t graph[3] = {nullptr, nullptr, nullptr};
   hipGraphExec_t gexec[3] = {nullptr, nullptr, nullptr};
-  BmvGeom geom;  // launch geometry of the MFMA product
+  BmvGeom geom;  // launch geometry of the product
   // FP64 residuals (starting and replacing columns) are formed on the steps
   // gstep with gstep % resid_period == 0; gstep counts every step the
   // engine has run, so a column's residual steps fall at fixed counts of its
@@ -1852,7 +1852,7 @@ static int batch_sync_operator(sgeo_batch* b) {
   return 0;
 }
 
-// The order in which the MFMA product walks the elements: by the Morton
+// The order in which the product walks the elements: by the Morton
 // code of the element centroid on a grid of the same spacing on every axis,
 // so the elements a product has in flight together (and each XCD's
 // contiguous share of the walk) form compact regions whose gathered P rows

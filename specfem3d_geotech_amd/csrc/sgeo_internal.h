@@ -208,7 +208,7 @@ hipError_t hex2spec_device(hipStream_t s, int32_t nelmt, const double* d_coord8,
                            double tol, SpecDev* out);
 void spec_device_free(SpecDev* d);
 
-// launch geometry of the persistent MFMA product (result bits do not
+// launch geometry of the batched element product (result bits do not
 // depend on it; chosen by sgeo_batch_autotune)
 struct BmvGeom {
   int blocks_per_cu = 3;

@@ -113,7 +113,7 @@ __device__ __forceinline__ void point_flux(const T adj[3][3], T lam, T mu, const
 //
 // Measured on 144,000 elements: 109 us (124 with the gathers awaited before
 // the Jacobians were formed) against 801 us for the packed matrices
-// (k_ebe_packed_pipe, 4.8 TB/s, at the copy rate); 33 against 8 us on 4,921.
+// (k_ebe_packed_pipe, 4.8 TB/s, at the copy rate); on 4,921, 8 against 33 us.
 // The 262 MB it must move take 55 us at that rate; the rest is the LDS traffic
 // (63 values per point) and, at four waves per SIMD (124 registers), the
 // latency of the gathers.  Five waves per SIMD gain 2.6 % on 144,000 elements

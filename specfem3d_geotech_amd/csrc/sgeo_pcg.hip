@@ -2,20 +2,21 @@
 // vector kernels (src/solver.f90:14-79) for gfx950.
 //
 // Reductions are two-phase: every block of a vector kernel writes its
-// partial sums/maxima to a scratch array, then a one-block finalize kernel
-// combines them in index order and updates the device-resident scalars.
-// The kernel boundary provides the visibility; no device-scope fences or
-// atomics are issued per block (on a multi-XCD MI355X a device-scope
-// release writes back the L2, which made a last-block-done pattern cost an
-// order of magnitude more than the streaming itself).  Partials are
-// combined in a fixed order, so results are deterministic run to run.
+// partial sums/maxima to a scratch array, and they are combined in a fixed
+// order after a kernel boundary: in the tree-ordered iteration by every block
+// of the kernel that needs the result (above PCG_DIRECT partials by
+// k_pcg_collapse before it), at a solve's start and in the reference-order mode
+// by a one-block finalize kernel.  The kernel boundary provides the
+// visibility; no device-scope fences or atomics are issued per block (on a
+// multi-XCD MI355X a device-scope release writes back the L2, which made a
+// last-block-done pattern cost an order of magnitude more than the streaming
+// itself).  The order is fixed, so results are deterministic run to run.
 //
 // Contraction is off: element products and vector updates round each
 // operation as the reference does.
 #pragma clang fp contract(off)
 
 #include <algorithm>
-#include <type_traits>
 
 #include "sgeo_device.h"
 #include "sgeo_internal.h"
@@ -86,10 +87,11 @@ __global__ __launch_bounds__(256) void k_ebe_elem(
 // --------------------------------------------------------------------------
 // K_e keeps its upper triangle U(r,c), r <= c, column by column:
 // U(r,c) at c(c+1)/2 + r, 3321 entries padded to SGEO_KPACK = 3328 so each
-// element starts 16-byte aligned.  One 128-thread block per element: the
-// block stages the packed matrix in LDS with 16-byte loads (each stored
-// entry crosses HBM once), then thread r < 81 forms
-// y_r = sum_c K(r,c) p_c, c ascending, with K(r,c) = U(min(r,c), max(r,c)).
+// element starts 16-byte aligned.  A 128-thread block stages an element's
+// packed matrix in LDS with 16-byte loads (each stored entry crosses HBM
+// once), then thread r < 81 forms y_r = sum_c K(r,c) p_c, c ascending, with
+// K(r,c) = U(min(r,c), max(r,c)).  FP32 matrices: k_ebe_packed, a block per
+// element; FP64: k_ebe_packed_pipe.
 // The reference's K_e is symmetric only to the last bit, so this path
 // agrees with the full-storage product to rounding, not bit for bit.
 
@@ -128,24 +130,20 @@ __device__ __forceinline__ double packed_row(const KT* u, const double* pe, int 
   return a;
 }
 
-template <typename KT>
 __global__ __launch_bounds__(128) void k_ebe_packed(
-    int32_t nelmt, const KT* __restrict__ KP, const int32_t* __restrict__ gdof,
+    int32_t nelmt, const float* __restrict__ KP, const int32_t* __restrict__ gdof,
     const double* __restrict__ p, double* __restrict__ Y, double* __restrict__ part,
     const PcgScalars* __restrict__ sc, int skip_mode) {
   if (skip_mode == 1 && sc->done) return;
   if (skip_mode == 2 && !sc->u_nonzero) return;
-  constexpr int PER = 16 / sizeof(KT);
-  constexpr int NV = SGEO_KPACK / PER;
-  __shared__ __align__(16) KT u[SGEO_KPACK];
+  typedef float v4f __attribute__((ext_vector_type(4)));
+  constexpr int NV = SGEO_KPACK / 4;
+  __shared__ __align__(16) float u[SGEO_KPACK];
   __shared__ double pe[81];
   const int64_t e = blockIdx.x;
   const int t = threadIdx.x;
-  typedef double v2d __attribute__((ext_vector_type(2)));
-  typedef float v4f __attribute__((ext_vector_type(4)));
-  using V = typename std::conditional<sizeof(KT) == 8, v2d, v4f>::type;
-  const V* src = reinterpret_cast<const V*>(KP + e * SGEO_KPACK);
-  V* dst = reinterpret_cast<V*>(u);
+  const v4f* src = reinterpret_cast<const v4f*>(KP + e * SGEO_KPACK);
+  v4f* dst = reinterpret_cast<v4f*>(u);
 #pragma unroll 4
   for (int q = t; q < NV; q += 128) dst[q] = __builtin_nontemporal_load(src + q);
   if (t < 81) pe[t] = p[gdof[e * 81 + t]];
@@ -160,13 +158,12 @@ __global__ __launch_bounds__(128) void k_ebe_packed(
   if (part) put_share<2>(d, part, blockIdx.x);
 }
 
-// Persistent, pipelined form of k_ebe_packed<double>: a few 128-thread
+// FP64, persistent and pipelined: a few 128-thread
 // blocks per CU walk the elements.  While element e is multiplied from LDS,
 // the next element's packed K is in flight into registers (16-byte loads) and
 // its gathered p into a register, with gdof read
 // one element further ahead; both reach LDS after the product, behind the
-// block's barrier.  Row r sums c ascending as k_ebe_packed does: the same
-// bits.
+// block's barrier.  Row r sums c ascending.
 __global__ __launch_bounds__(128) void k_ebe_packed_pipe(
     int32_t nelmt, const double* __restrict__ KP, const int32_t* __restrict__ gdof,
     const double* __restrict__ p, double* __restrict__ Y, double* __restrict__ part,
@@ -465,11 +462,12 @@ __global__ __launch_bounds__(256) void k_pcg_finalize(
 //   k_pcg_step<true>: kp summed on the fly, u += alpha p, r -= alpha kp,
 //     partials of max|u| and r.z (z = dinv r is formed, not stored),
 //   k_pcg_dir: the stop test, p = z + beta p, partials of max|p|.
-// A trial's solves form p.Kp from the assembled vector (k_pcg_asm, then
-// k_pcg_step<false>): their x enters the yield function, which at the
-// corners of the Mohr-Coulomb pyramid turns the last bits of x into
-// relative changes of 1e-7 (asin near 1), so they keep the summation order
-// they have always had.
+// A trial's solves multiply the stored matrices and form p.Kp from the
+// assembled vector (k_pcg_asm, then k_pcg_step<false>): their x enters the
+// yield function, which at the corners of the Mohr-Coulomb pyramid turns the
+// last bits of x into relative changes of 1e-7 (asin near 1), so they keep the
+// summation order they have always had.  That keeps a trial's bits; whether
+// the other order is any less accurate has not been measured.
 // Every block combines the partials that the kernel before it left, all in
 // the same order, so that no one-block kernel stands between them; above
 // PCG_DIRECT partials k_pcg_collapse does it once, in that order, since each
@@ -1061,7 +1059,7 @@ void launch_ebe_packed_f32(hipStream_t s, int32_t nelmt, const float* KP,
                            const int32_t* gdof, const double* p, double* Y, double* part,
                            const PcgScalars* sc, int skip_mode) {
   if (nelmt <= 0) return;
-  hipLaunchKernelGGL(k_ebe_packed<float>, dim3(nelmt), dim3(128), 0, s, nelmt,
+  hipLaunchKernelGGL(k_ebe_packed, dim3(nelmt), dim3(128), 0, s, nelmt,
                      KP, gdof, p, Y, part, sc, skip_mode);
 }
 
