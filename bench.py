@@ -150,12 +150,27 @@ def single_trial_pcg(ctx, dm, ext, ym, nu, phi, coh, psi, steps, warm):
     return dt_s, n, ms
 
 
-def roofline(kernel, bytes_per_launch, n, ms, extra=None):
+def measured_counters(kernel_key):
+    """What the committed counter runs read for a kernel (profiles/traffic.json:
+    HBM bytes per launch from FETCH_SIZE and WRITE_SIZE, scaled by what they
+    read for a copy of known size; share of the launch in which the SIMDs
+    issue vector instructions), or {}."""
+    try:
+        with open(os.path.join(ROOT, "profiles", "traffic.json")) as fh:
+            return json.load(fh)[kernel_key]
+    except (OSError, KeyError, ValueError):
+        return {}
+
+
+def roofline(kernel, bytes_per_launch, n, ms, extra=None, counters=None):
+    counters = counters or {}
     avg = ms / max(n, 1)
     ach = bytes_per_launch / (avg * 1e-3) / 1e9 if n else 0.0
     out = dict(kernel=kernel, bound="hbm", achieved=round(ach, 1), peak=HBM_PEAK_GBS,
                unit="GB/s", frac=round(ach / HBM_PEAK_GBS, 4), avg_launch_ms=round(avg, 4),
-               launches=n, bytes_per_launch=int(bytes_per_launch), traffic=None)
+               launches=n, bytes_per_launch=int(bytes_per_launch),
+               traffic=counters.get("bytes_per_launch"),
+               valu_issue_share=counters.get("valu_share"))
     if extra:
         out.update(extra)
     return out
@@ -311,7 +326,12 @@ def mode_sweep(a, ctx, wl, mesh, spec, prep_s, copy_gbs):
         roofline=roofline(f"element product from the geometry, {B} columns", kbytes, nl, kms,
                           dict(bytes_model="E*(27*48 + 82*4 + (2*81*4 + 8)*b), "
                                "b = mean trials iterating per step of the roofline window",
-                               b=round(b_prof, 2))))
+                               b=round(b_prof, 2),
+                               counters_source="profiles/perf_cases_counters.md (c1, 64 "
+                               "trials iterating); beside the bytes the product is held by "
+                               "vector issue"),
+                          measured_counters("k_bmf_lane<64>")
+                          if (a.workload == "c1" and B == 64) else None))
     return res
 
 

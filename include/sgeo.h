@@ -156,6 +156,9 @@ int sgeo_spec_destroy(sgeo_spec *spec);
 int sgeo_mesh_create(sgeo_ctx *ctx, int32_t nelmt, int32_t neq,
                      const double *corners, const int32_t *gdof_elmt,
                      const int32_t *mat_id, int32_t nmat, sgeo_mesh **mesh);
+/* The FP64 matrices of a destroyed mesh (up to 16 GB) stay allocated for the
+ * context's next mesh, until this library finds no memory or the device's
+ * last context ends. */
 int sgeo_mesh_destroy(sgeo_mesh *mesh);
 /* Builds storekm, the assembled diagonal and (if extload != NULL) the
  * gravity load on the device: src/preprocess.f90:74-148 with
@@ -179,7 +182,7 @@ int sgeo_mesh_upload_stiffness(sgeo_mesh *mesh, const double *storekm,
  * bit only).  Linear solves and products with the packed FP64 operator of a
  * mesh whose stiffness was built here are evaluated from the element corners,
  * which agrees with the matrices to rounding; plastic iterations and uploaded
- * matrices use the storage.  The full FP64 operator reproduces the reference bit for bit;
+ * matrices use the storage (sgeo_slope_create makes it for a mesh's trials).  The full FP64 operator reproduces the reference bit for bit;
  * the others trade that for fewer bytes per iteration. */
 int sgeo_mesh_set_operator(sgeo_mesh *mesh, int kprec, int kfmt);
 /* Achieved HBM bandwidth of a plain device copy of `bytes` (read + write,

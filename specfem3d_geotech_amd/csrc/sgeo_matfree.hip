@@ -114,9 +114,10 @@ __device__ __forceinline__ void point_flux(const T adj[3][3], T lam, T mu, const
 // Measured on 144,000 elements: 109 us (124 with the gathers awaited before
 // the Jacobians were formed) against 801 us for the packed matrices
 // (k_ebe_packed_pipe, 4.8 TB/s, at the copy rate); on 4,921, 8 against 33 us.
-// The 262 MB it must move take 55 us at that rate; the rest is the LDS traffic
-// (63 values per point) and, at four waves per SIMD (124 registers), the
-// latency of the gathers.  Five waves per SIMD gain 2.6 % on 144,000 elements
+// The 262 MB it must move take 55 us at that rate (200 MB of them cross HBM).
+// Counters: vector issue active 46 % of the time, LDS 44 % (63 values per
+// point; 8 % are bank conflicts), the waves waiting 61 % of their cycles at
+// four per SIMD (124 registers).  Five waves per SIMD gain 2.6 % on 144,000 elements
 // and lose 2 % on 4,921; six spill into the time of both (129 us).
 // --------------------------------------------------------------------------
 #define MF_EPB 9
@@ -411,9 +412,9 @@ __device__ __forceinline__ void lane_points(float (&u)[81], float (&y)[81], cons
 // block, two per SIMD.  The elements' geometry is loaded into LDS beside the
 // gathers: read point by point from memory (through the scalar cache at
 // B = 64) every line's latency stood in the wave's way, 1.72 ms on 144,000
-// elements.  Of the 1.15 ms that remain about 0.75 are the 3,400 vector
-// operations per element and column at one per 4 cycles and SIMD; the rest
-// is the start of each wave (a chain of four dependent loads).
+// elements.  Of the 1.15 ms that remain 0.78 are the 3,340 vector instructions
+// of a wave at one per 4 cycles and SIMD (counted); the rest is the start of
+// each wave (a chain of four dependent loads).  It moves 4.5 GB meanwhile.
 // Measured against k_bmv_mfma: 144,000 elements, 64 columns 1.15 against
 // 1.80 ms, 8 columns 0.185 against 0.80; 12,544 elements, 64 columns 109
 // against 165 us; 25,344, 8 columns 35 against 146.
