@@ -323,7 +323,11 @@ static hipError_t to_host(sgeo_ctx* c, void* host, const void* dev, size_t n) {
     for (hipEvent_t& ev : st.ev)
       if (!ev && e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
     if (e == hipSuccess) e = hipHostMalloc((void**)&st.buf, 2 * COPY_THREADS * COPY_PIECE);
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {  // no pinned memory to be had
+      (void)hipGetLastError();
+      st.buf = nullptr;
+      return hipMemcpyAsync(host, dev, n, hipMemcpyDeviceToHost, s);
+    }
   }
   const size_t pieces = (n + COPY_PIECE - 1) / COPY_PIECE;
   hipError_t err[COPY_THREADS] = {};

@@ -22,7 +22,7 @@ auto& kernels = *new std::map<const void*, std::string>;  // host stub -> name
 auto& blocks = *new std::map<void*, size_t>;              // device allocations
 auto& log_ = *new std::string;  // one line per launch, allocation and free
 auto& watch = *new std::string;
-size_t used = 0, limit = SIZE_MAX;
+size_t used = 0, limit = SIZE_MAX, host_limit = SIZE_MAX;
 int watch_arg = 0;
 thread_local hipError_t last = hipSuccess;
 thread_local struct {
@@ -46,6 +46,7 @@ extern "C" {
 
 // ---- test interface ----
 void rt_limit(size_t bytes) { limit = bytes; }
+void rt_host_limit(size_t bytes) { host_limit = bytes; }  // of one pinned allocation
 size_t rt_used() { return used; }
 void rt_clear() {
   std::lock_guard<std::mutex> l(mu);
@@ -86,7 +87,7 @@ hipError_t hipFree(void* p) {
   return hipSuccess;
 }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
-  *p = calloc(1, n);
+  *p = n <= host_limit ? calloc(1, n) : nullptr;
   return *p ? hipSuccess : error(hipErrorOutOfMemory);
 }
 hipError_t hipHostFree(void* p) {

@@ -17,6 +17,7 @@ sys.path.insert(0, {root!r})
 rt = C.CDLL({rt!r}, mode=C.RTLD_GLOBAL)
 rt.rt_used.restype = C.c_size_t
 rt.rt_limit.argtypes = [C.c_size_t]
+rt.rt_host_limit.argtypes = [C.c_size_t]
 rt.rt_log.restype = C.c_char_p
 rt.rt_watch.argtypes = [C.c_char_p, C.c_int]
 import numpy as np
@@ -283,4 +284,21 @@ assert n == {distinct} * 4, n
 assert (t["blocks_per_cu"], t["xcd_split"]) == {pick}, t
 ms = [c["ms"] for c in t["candidates"]]
 assert len(ms) == 8 and len(set(ms)) == {distinct} and t["ms"] == min(ms), t
+""")
+
+
+@pytest.mark.parametrize("pinned", [True, False])
+def test_large_results_without_pinned_memory(runtime, pinned):
+    """Results of several pieces arrive whole, through the pinned pieces or,
+    where those cannot be had, by a plain copy that leaves no error behind."""
+    runtime(f"""
+dm = DeviceMesh(ctx, hex2spec(slope_mesh(10, 5, 3)), len(gam))  # K of 7.9 MB
+n = dm.spec.nelmt
+k = np.random.default_rng(1).normal(size=(n, 81 * 81))
+if not {pinned}:
+    rt.rt_host_limit(1 << 16)
+dm.upload_stiffness(k, np.ones(dm.spec.neq + 1))
+for _ in range(2):
+    assert np.array_equal(np.ravel(dm.download_stiffness()), np.ravel(k))
+dm.set_operator(K_F64, KFMT_PACKED)
 """)
